@@ -1041,7 +1041,10 @@ void hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_
     // with in-kernel projector values; one fused pass otherwise (QG_SPLIT_NL=0/1 forces)
     const int split_env = env_int("QG_SPLIT_NL", -1);
     const bool split = nl && (split_env >= 0 ? split_env != 0 : segments_form(nl, dtype, MODE_NL));
-    const int cb = nl ? chunk_bands(g, dtype, nbands, split) : nbands;
+    // the sphere apply pass over the whole block behind the table projection
+    const bool sphere = nl && split_env < 0 && !t_trial && h->plan.kernels == QG_KERNELS_AUTO &&
+                        sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nullptr, true, false, s);
+    const int cb = nl && !sphere ? chunk_bands(g, dtype, nbands, split) : nbands;
     if (nl) nl->d_coef.alloc((size_t)std::min(cb, nbands) * nl->geo.ncoef);
     const int nchunks = (nbands + cb - 1) / cb;
     if (h->timing) {
@@ -1064,7 +1067,9 @@ void hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_
             else launch_project<float>(nl, nb, (const float*)pin, ld, nl->d_coef.p, s);
         }
         if (h->timing) QG_HIP(hipEventRecord(h->tev[3 * ci + 1], s));
-        if (nl && split) {
+        if (sphere) {
+            (void)sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nl->d_coef.p, true, true, s);
+        } else if (nl && split) {
             // stencil + V pass, then the projector term as a read-modify-write pass over the
             // chunk (still resident in the Infinity Cache) with many bands per item
             if (dtype == QG_F64) {
@@ -1468,6 +1473,7 @@ static void nl_build(qg_nonlocal* nl, int natoms, const double* xyz, const int* 
     nl->d_atom_coef_off.upload(gm.atom_coef_off.data(), gm.atom_coef_off.size());
     for (auto& t : nl->tiles) t.ty = t.tz = -1;
     nl->rows.clear();
+    sphere_prepare(nl);
     rows_prepare(nl);
     // Gaussian projectors can be evaluated inside the projector pass instead of read from
     // per-point tables (QG_NL_ANALYTIC=0 keeps the tables everywhere)

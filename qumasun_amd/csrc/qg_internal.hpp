@@ -196,6 +196,35 @@ struct RowsGeo {
 constexpr int kRowsProjThreads = 256;
 bool build_rows_geometry(const qg_grid& g, const NlGeometry& geo, int ty, int tzp, bool by_group, RowsGeo& o);
 
+// The sphere of one atom under one periodic shift (all its cutoffs together), as the sphere
+// apply kernels see it: centre = n + f in grid points (n integer, shift included).
+struct SphereImage {
+    int n[3];
+    int atom;
+    int b[3], e[3];      // in-grid range [b, e)
+    int nparts;
+    int part[4];         // its per-cutoff images (DevImage)
+    double f[3];
+};
+
+// channels per image the sphere kernels are instantiated for: ns s and np p channels ((1, 1) or
+// (2, 2)); ns = 0: the projector set does not fit them
+struct SphereForm {
+    int ns = 0, np = 0;
+};
+
+// Entry lists of the sphere apply kernel (qg_sphere.hip) for tiles of ty rows and one block type:
+// per (tile, plane, wavefront) a run of trips, each one entry for each of the 64 lanes.
+struct SphereGeo {
+    int ty = 0, dtype = 0, nq = 0, tpb = 0, ntile = 0;
+    int max_col = 0;     // most sphere images of one tile column
+    int ntrips = 1;
+    bool ok = false;
+    DevBuf<int> d_col_off, d_col_img, d_trip_off;
+    DevBuf<uint32_t> d_words;
+    DevBuf<unsigned char> d_vals;
+};
+
 // Caller-provided FP64 scratch of one application (projector partials, then coefficients).
 struct RowsScratch {
     double* base;
@@ -245,7 +274,13 @@ struct qg_nonlocal {
     qg::DevBuf<int64_t> d_img_tbl_off;
     // row-kernel geometry, one per (tile rows, projection slab) shape in use
     std::vector<std::unique_ptr<qg::RowsGeo>> rows;
-    std::mutex rows_mu;             // guards the creation of entries of `rows`
+    std::mutex rows_mu;             // guards the creation of entries of `rows` and `sphere`
+    // sphere apply kernels: images, channel slots and entry lists per (tile rows, type) in use
+    qg::SphereForm sphere_form;
+    std::vector<qg::SphereImage> sphere_img;
+    qg::DevBuf<qg::SphereImage> d_sphere_img;
+    qg::DevBuf<int> d_atom_chan;
+    std::vector<std::unique_ptr<qg::SphereGeo>> sphere;
     qg::DevBuf<double> rows_part;   // projector partials of qg_nonlocal_project
     // geometry generation: bumped by every (re)build of the projector geometry, so state derived
     // from it elsewhere (the k-point phase tables) knows when to rebuild
@@ -268,6 +303,11 @@ bool rows_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* p
 bool rows_laplacian_apply(const qg_grid& g, int dtype, int nbands, const void* psi, int64_t ld, void* out,
                           int64_t ld_out, double coef, int accumulate, hipStream_t s);
 void rows_prepare(qg_nonlocal* nl);
+void sphere_prepare(qg_nonlocal* nl);
+bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
+                              int64_t ld_out, const double* coef, bool may_build, bool run, hipStream_t s);
+bool sphere_prepared(qg_nonlocal* nl, int dtype);
+size_t lds_limit();
 double* scratch_address();
 void rows_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi, int64_t ld_out,
                         hipStream_t s);

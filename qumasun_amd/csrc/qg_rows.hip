@@ -1043,7 +1043,7 @@ static RowsGeo* rows_geometry(qg_nonlocal* nl, int ty, int tzp, bool by_group, b
 
 // Most LDS one workgroup may allocate on the current device (160 KB on MI355X), looked up once
 // per device.
-static size_t lds_limit() {
+size_t lds_limit() {
     static std::mutex mu;
     static size_t cached[64] = {};
     int dev = 0;
@@ -1200,7 +1200,18 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     const RowsShape sh = rows_shape(g, dtype, nbands, &h->plan);
     const RowsGeo* rg = nullptr;    // apply kernel's geometry (tile rows ty)
     const RowsGeo* rgp = nullptr;   // projection kernel's geometry (tile rows typ)
-    if (nl) {
+    const bool sphere = nl && sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nullptr, ws == nullptr,
+                                                       false, s);
+    if (nl && sphere) {
+        if (sh.typ == 0) return false;
+        QG_REQUIRE(!ws || sh.ty == rows_shape(g, dtype, 0).ty, "the projector geometry of this launch shape is not "
+                   "prepared (qg_nonlocal_create and qg_nonlocal_update prepare the default shapes)");
+        rgp = rows_geometry(nl, sh.typ, sh.tzp, false, ws == nullptr);
+        QG_REQUIRE(rgp, "the projector geometry of this launch shape is not prepared (qg_nonlocal_create and "
+                        "qg_nonlocal_update prepare the default shapes)");
+        if (!rgp->ok || rgp->max_items > kProjThreads * kItemsPT) return false;
+        if (rows_proj_lds<T>(*rgp, g, sh.nbp, (int)nl->geo.projs.size()) > lds_limit()) return false;
+    } else if (nl) {
         if (sh.typ == 0) return false;
         // with caller scratch nothing may be allocated: the geometry must exist already
         rg = rows_geometry(nl, sh.ty, sh.tzp, true, ws == nullptr);
@@ -1248,7 +1259,9 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
         }
     }
     if (timed) QG_HIP(hipEventRecord(h->tev[1], s));
-    if (!nl || rg->njs == 4) {
+    if (sphere) {
+        (void)sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, coef, ws == nullptr, true, s);
+    } else if (!nl || rg->njs == 4) {
         if (nl && rg->pform == 2)
             rows_launch_hpsi<T, 4, 2>(g, sh, rg, nl, nbands, psi, ld, hpsi, ld_out, -0.5, 1, 0, V, coef, s);
         else if (nl && rg->pform == 1)
@@ -1346,7 +1359,8 @@ void rows_prepare(qg_nonlocal* nl) {
         if (!rows_eligible(nl->gcopy, dtype, nl)) continue;
         const RowsShape sh = rows_shape(nl->gcopy, dtype, 0);
         if (sh.typ == 0) continue;
-        rows_geometry(nl, sh.ty, sh.tzp, true);
+        // the apply pass of the rows kernels only where the sphere entry lists do not serve
+        if (!sphere_prepared(nl, dtype)) rows_geometry(nl, sh.ty, sh.tzp, true);
         rows_geometry(nl, sh.typ, sh.tzp, false);
     }
 }

@@ -1,0 +1,897 @@
+// qg_sphere.hip — H·psi apply on MI355X (gfx950): stencil + local potential + projector term in
+// one pass over psi, the projector values read from per-lane entry lists.
+//
+// Reference semantics (QUMASUN source/):
+//   H psi = V psi + V_NL psi - 1/2 Lap8 psi   qumasun_mpi.matrix.h:21-43
+//   V_NL psi = sum_aj E_j c_aj beta_j         PseudoPotOperator_mpi_v2.h:465-570
+//   beta_j = p(r) Y_lm(r), Y_1m = sqrt(3/4pi) (y, z, x)/r, Y_1m(r^2 < 1e-14) = 0
+//                                             RealSphericalHarmonics.h:149-161, SetBlockYlm.h:41
+//
+// A workgroup owns a tile of ty x-rows, a slab of planes and NB bands.  Every thread owns one
+// group of VN = 16 / sizeof(T) consecutive x-points of one row for all NB bands and streams
+// through the slab in z: the 9 z-neighbours in a register queue, the current plane (with 4
+// wrapped columns and rows each side) in LDS, double buffered, one barrier per plane.
+//
+// Projector term.  For every (tile, plane, wavefront) the sphere images that touch a lane's
+// group are listed lane by lane ("trips": entry k of all 64 lanes stored together, lanes with
+// fewer entries padded with an empty image), each entry holding the radial functions at the
+// lane's VN points (s channels: p(r) Y00; p channels: p(r) sqrt(3/4pi) / r, both zero outside
+// the cutoff) and the group's integer displacement from the image centre.  The owner of a point
+// adds
+//   sum_s f_s (E c)_s + sum_p f_p [(E c)_y dy + (E c)_z dz + (E c)_x dx]
+// to it from registers, so the term needs no exponentials, no LDS exchange, no barrier and no
+// atomics, and every radial form (Gaussian or tabulated) costs the same.
+#include <algorithm>
+#include <cmath>
+#include <map>
+#include <tuple>
+#include <type_traits>
+#include "qg_internal.hpp"
+
+namespace qg {
+
+namespace {
+
+using rsrc_t = __amdgpu_buffer_rsrc_t;
+using u4 = __attribute__((ext_vector_type(4))) uint32_t;
+
+template <class T>
+struct alignas(16) Row {
+    T v[16 / sizeof(T)];
+};
+
+__device__ __forceinline__ rsrc_t rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+template <class T>
+__device__ __forceinline__ Row<T> vload(rsrc_t r, int voff, int soff) {
+    return __builtin_bit_cast(Row<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+template <class T>
+__device__ __forceinline__ void vstore(rsrc_t r, const Row<T>& v, int voff, int soff) {
+    // cache policy nt: the results are not read back here, and keeping them out of L2 leaves it to
+    // the halo rows and entry lists (3.42 -> 3.21 ms per application at 120^3 / 512 FP32 bands)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, 2);
+}
+
+// hardware workgroup ids go round-robin over the 8 XCDs; give each XCD one contiguous range of
+// logical ids (the tiles and bands of a range share halo rows and entry lists in its L2)
+__device__ __forceinline__ int xcd_order(int i, int n) {
+    const int xcd = i & 7, slot = i >> 3;
+    const int per = n >> 3, rem = n & 7;
+    return ((xcd < rem) ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + slot;
+}
+
+template <class T>
+struct Coef8 {
+    T c0;
+    T cx[4], cy[4], cz[4];
+};
+
+template <class T>
+Coef8<T> coef8(const qg_grid& g, double coef) {
+    const double w[4] = {8064.0, -1008.0, 128.0, -9.0};
+    Coef8<T> s;
+    s.c0 = (T)(-14350.0 / 5040.0 * coef *
+               (1.0 / (g.h[0] * g.h[0]) + 1.0 / (g.h[1] * g.h[1]) + 1.0 / (g.h[2] * g.h[2])));
+    for (int m = 0; m < 4; ++m) {
+        s.cx[m] = (T)(w[m] * coef / (5040.0 * g.h[0] * g.h[0]));
+        s.cy[m] = (T)(w[m] * coef / (5040.0 * g.h[1] * g.h[1]));
+        s.cz[m] = (T)(w[m] * coef / (5040.0 * g.h[2] * g.h[2]));
+    }
+    return s;
+}
+
+int round64i(int v) { return (v + 63) / 64 * 64; }
+
+// buffer offset of lanes with nothing to load or store: beyond every band's num_records, so
+// the hardware returns zero for the load and drops the store
+constexpr int kOOB = 0x7ffffff0;
+constexpr int kMaxThreads = 512;
+
+// entry word: column image | dy offset << 10 | dx offset << 21 (the last two signed 11-bit, in
+// grid points from the image's nearest grid point)
+__host__ __device__ constexpr uint32_t entry_word(int li, int dx, int dy) {
+    return (uint32_t)li | ((uint32_t)(dy & 2047) << 10) | ((uint32_t)(dx & 2047) << 21);
+}
+
+}  // namespace
+
+struct SphereArgs {
+    int nx, ny, nz;
+    int ty, tz, ntile, nslab, nbands;
+    int tg;                     // tiles per group of the workgroup order
+    int nq, tpb;                // groups per row, threads per workgroup
+    int64_t ld_in, ld_out;
+    int nw;                     // wavefronts per workgroup
+    const int* col_off;         // per tile: first column image
+    const int* col_img;         // sphere image ids
+    const SphereImage* images;
+    const int* trip_off;        // per (tile, plane, wavefront): first trip
+    int ntrips;                 // all trips, at least 1
+    const void* vals;           // [trip][radial vector][lane] 16-byte vectors
+    const uint32_t* words;      // [trip][lane]
+    const double* coef;         // nbands x ncoef, this application's bands
+    const double* coef_energy;
+    const int* atom_coef_off;
+    const int* atom_chan;       // [atom][4]: coefficient slots of its s, s, p, p channels (-1: none)
+    int ncoef;
+    int max_col;
+    double h[3];
+};
+
+// LDS bytes of an apply workgroup
+template <class T>
+static size_t sphere_lds(int nx, int ty, int nb, int ns, int np, int max_col) {
+    constexpr int VN = 16 / sizeof(T);
+    const size_t W = (size_t)(nx + 8 + VN - 1) / VN * VN;
+    return sizeof(T) * (2 * (size_t)nb * (ty + 8) * W + (size_t)(max_col + 1) * (4 + nb * (ns + 3 * np)));
+}
+
+// One workgroup of the apply pass.  NB bands; NS s and NP p channels per image; RAG: Nx is not a
+// multiple of VN (the last group of a row then overlaps its neighbour: both owners compute and
+// write the same values, and LDS is accessed by element); HV halo vectors per thread and band.
+template <class T, int NB, int NS, int NP, bool RAG, int HV>
+__device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>& sc, const T* __restrict__ V,
+                                            const T* __restrict__ psi, T* __restrict__ out, const int wg,
+                                            unsigned char* smem) {
+    constexpr int VN = 16 / sizeof(T);
+    constexpr int S = sizeof(T);
+    constexpr int NC = NS + 3 * NP;
+    constexpr int NV = NS + NP;            // 16-byte vectors per entry
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const int W = RAG ? (nx + 8 + VN - 1) / VN * VN : nx + 8;
+    const int ty = a.ty;
+    const int lband = (ty + 8) * W;
+    const int nthr = a.tpb;
+    T* planes = reinterpret_cast<T*>(smem);                    // [2][NB][ty + 8][W]
+    T* imf = planes + (size_t)2 * NB * lband;                  // [max_col + 1][4]: f.x f.y f.z, n.z
+    T* ec = imf + (size_t)(a.max_col + 1) * 4;                 // [max_col + 1][NB][NC]
+
+    // order: tiles of a group of tg, then bands, then slabs, then groups
+    const int nbg = (a.nbands + NB - 1) / NB;
+    const int grp = wg / (a.tg * nbg * a.nslab);
+    const int in_grp = wg - grp * (a.tg * nbg * a.nslab);
+    const int tgw = min(a.tg, a.ntile - grp * a.tg);
+    const int tile = grp * a.tg + in_grp % tgw;
+    const int rest = in_grp / tgw;
+    const int slab = rest / nbg;
+    const int b0 = (rest - slab * nbg) * NB;
+    const int y0 = tile * ty;
+    const int rows = min(ty, ny - y0);
+    const int z0 = slab * a.tz, z1 = min(z0 + a.tz, nz);
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int nq = a.nq;
+    const int r = tid / nq, xq = tid - r * nq;
+    const int x = RAG ? min(xq * VN, nx - VN) : xq * VN;
+    const bool own = r < rows;
+    const int plane = nx * ny;
+    const uint32_t band_bytes = (uint32_t)((int64_t)plane * nz * S);
+    rsrc_t rin[NB], rout[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        // bands past the block read the last one and store nothing
+        const int band = min(b0 + b, a.nbands - 1);
+        rin[b] = rsrc(psi + (int64_t)band * a.ld_in, band_bytes);
+        rout[b] = rsrc(out + (int64_t)band * a.ld_out, b0 + b < a.nbands ? band_bytes : 0u);
+    }
+    const rsrc_t rv = rsrc(V, band_bytes);
+    const int vo = own ? ((y0 + r) * nx + x) * S : kOOB;
+    const int lc = (r + 4) * W + 4 + x;
+    const int lw = (x < 4) ? lc + nx : ((x >= nx - 4) ? lc - nx : -1);   // wrapped copy (whole vectors)
+    int ho[HV], hl[HV];
+#pragma unroll
+    for (int k = 0; k < HV; ++k) {
+        const int v = tid + k * nthr;
+        ho[k] = kOOB;
+        hl[k] = -1;
+        if (v < 8 * nq) {
+            const int hr = v / nq, hq = v - hr * nq;
+            const int hx = RAG ? min(hq * VN, nx - VN) : hq * VN;
+            int gy = (hr < 4) ? y0 - 4 + hr : y0 + rows + (hr - 4);
+            gy = ((gy % ny) + ny) % ny;
+            ho[k] = (gy * nx + hx) * S;
+            hl[k] = ((hr < 4) ? hr : rows + hr) * W + 4 + hx;
+        }
+    }
+    // byte offset of plane z, -nz <= z < 2 nz
+    auto zoff = [&](int z) { return (z < 0 ? z + nz : (z >= nz ? z - nz : z)) * plane * S; };
+    const T hx = (T)a.h[0], hy = (T)a.h[1], hz = (T)a.h[2];
+
+    // image centres and E c of the tile's column; image ncol is the empty one of the padding
+    const int c0 = a.col_off[tile];
+    const int ncol = a.col_off[tile + 1] - c0;
+    for (int li = tid; li <= ncol; li += nthr) {
+        const SphereImage* im = a.images + a.col_img[c0 + min(li, ncol - 1)];
+        const bool ok = li < ncol;
+        imf[4 * li] = ok ? (T)im->f[0] : T(0);
+        imf[4 * li + 1] = ok ? (T)im->f[1] : T(0);
+        imf[4 * li + 2] = ok ? (T)im->f[2] : T(0);
+        imf[4 * li + 3] = ok ? (T)im->n[2] : T(0);
+    }
+    for (int i = tid; i < (ncol + 1) * NB * NC; i += nthr) {
+        const int li = i / (NB * NC), b = (i / NC) % NB, j = i % NC;
+        T v = T(0);
+        if (li < ncol && b0 + b < a.nbands) {
+            const int at = a.images[a.col_img[c0 + li]].atom;
+            const int ch = j < NS ? j : 2 + (j - NS) / 3;
+            const int slot = a.atom_chan[4 * at + ch];
+            if (slot >= 0) {
+                const int cb = a.atom_coef_off[at] + slot + (j < NS ? 0 : (j - NS) % 3);
+                v = (T)(a.coef_energy[cb] * a.coef[(int64_t)(b0 + b) * a.ncoef + cb]);
+            }
+        }
+        ec[i] = v;
+    }
+
+    // z-queue: step k of three planes holds the planes z - 4 .. z + 4 in q[k] .. q[k + 8] and
+    // loads z + 5 into q[k + 9] (step 2: into the free q[0]); the queue moves once per three planes
+    Row<T> q[NB][11];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int d = 0; d < 8; ++d) q[b][d] = vload<T>(rin[b], vo, zoff(z0 - 4 + d));
+    Row<T> hn[NB][HV], vn;
+    auto load_halo = [&](int z) {
+        vn = vload<T>(rv, vo, zoff(z));
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int k = 0; k < HV; ++k) hn[b][k] = vload<T>(rin[b], ho[k], zoff(z));
+    };
+#pragma unroll
+    for (int b = 0; b < NB; ++b) q[b][8] = vload<T>(rin[b], vo, zoff(z0 + 4));
+    load_halo(z0);
+
+    // the first K trips of a plane in registers, loaded a plane ahead: through buffer resources
+    // of exactly the plane's trips, so that those past its last one cost no traffic and every
+    // plane issues the same number of loads
+    constexpr int K = 3;
+    struct Entry {
+        Row<T> f[NV];
+        uint32_t w;
+    };
+    Entry en[K];
+    const int* toff = a.trip_off + (size_t)tile * nz * a.nw + wave;
+    int tb, n;      // first trip and number of trips of the plane whose entries are held
+    auto load_entry = [&](rsrc_t rvals, rsrc_t rwords, int k) {
+        Entry e;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) e.f[v] = vload<T>(rvals, lane * 16, (k * NV + v) * 1024);
+        e.w = __builtin_amdgcn_raw_buffer_load_b32(rwords, lane * 4, k * 256, 0);
+        return e;
+    };
+    auto load_entries = [&](int z) {
+        tb = __builtin_amdgcn_readfirstlane(toff[(size_t)z * a.nw]);
+        n = __builtin_amdgcn_readfirstlane(toff[(size_t)z * a.nw + 1]) - tb;
+        const rsrc_t rvals = rsrc((const unsigned char*)a.vals + (int64_t)tb * NV * 1024, (uint32_t)n * NV * 1024);
+        const rsrc_t rwords = rsrc(a.words + (int64_t)tb * 64, (uint32_t)n * 256);
+#pragma unroll
+        for (int k = 0; k < K; ++k) en[k] = load_entry(rvals, rwords, k);
+    };
+    load_entries(z0);
+
+    auto step = [&](auto kc, int z) {
+        constexpr int k0 = decltype(kc)::value;
+        T* Lp = planes + (size_t)((z - z0) & 1) * NB * lband;
+        const int zn = min(z + 1, z1 - 1);
+        const Row<T> vcur = vn;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            T* Lb = Lp + b * lband;
+            const Row<T>& cur = q[b][k0 + 4];
+            if (own) {
+                if constexpr (!RAG) {
+                    *reinterpret_cast<Row<T>*>(Lb + lc) = cur;
+                    if (lw >= 0) *reinterpret_cast<Row<T>*>(Lb + lw) = cur;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < VN; ++i) {
+                        Lb[lc + i] = cur.v[i];
+                        if (x + i < 4) Lb[lc + i + nx] = cur.v[i];
+                        if (x + i >= nx - 4) Lb[lc + i - nx] = cur.v[i];
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < HV; ++k)
+                if (hl[k] >= 0) {
+                    if constexpr (!RAG) {
+                        *reinterpret_cast<Row<T>*>(Lb + hl[k]) = hn[b][k];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < VN; ++i) Lb[hl[k] + i] = hn[b][k].v[i];
+                    }
+                }
+        }
+        // the next plane: every load unconditional (the slab's last plane loads one too many)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) q[b][k0 < 2 ? k0 + 9 : 0] = vload<T>(rin[b], vo, zoff(z + 5));
+        load_halo(zn);
+        __syncthreads();
+
+        Row<T> res[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            // V psi and the stencil: centre and z from the register queue, x and y from LDS
+            const T* Lc = Lp + b * lband + (own ? (r + 4) * W + x : 0);   // Lc[4 + i] is point x + i
+            T d[VN];
+            const Row<T>* qb = q[b] + k0;
+#pragma unroll
+            for (int i = 0; i < VN; ++i) {
+                d[i] = sc.c0 * qb[4].v[i];
+                d[i] += sc.cz[3] * (qb[8].v[i] + qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] + qb[1].v[i]) +
+                        sc.cz[1] * (qb[6].v[i] + qb[2].v[i]) + sc.cz[0] * (qb[5].v[i] + qb[3].v[i]);
+            }
+            {
+                T xsv[VN + 8];
+                if constexpr (!RAG) {
+#pragma unroll
+                    for (int k = 0; k < (VN + 8) / VN; ++k) {
+                        const Row<T> w = *reinterpret_cast<const Row<T>*>(Lc + k * VN);
+#pragma unroll
+                        for (int u = 0; u < VN; ++u) xsv[k * VN + u] = w.v[u];
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < VN + 8; ++k) xsv[k] = Lc[k];
+                }
+#pragma unroll
+                for (int i = 0; i < VN; ++i)
+                    d[i] += sc.cx[3] * (xsv[i + 8] + xsv[i]) + sc.cx[2] * (xsv[i + 7] + xsv[i + 1]) +
+                            sc.cx[1] * (xsv[i + 6] + xsv[i + 2]) + sc.cx[0] * (xsv[i + 5] + xsv[i + 3]);
+            }
+#pragma unroll
+            for (int m = 3; m >= 0; --m) {
+                Row<T> ym, yp;
+                if constexpr (!RAG) {
+                    ym = *reinterpret_cast<const Row<T>*>(Lc + 4 - (m + 1) * W);
+                    yp = *reinterpret_cast<const Row<T>*>(Lc + 4 + (m + 1) * W);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < VN; ++i) {
+                        ym.v[i] = Lc[4 + i - (m + 1) * W];
+                        yp.v[i] = Lc[4 + i + (m + 1) * W];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < VN; ++i) d[i] += sc.cy[m] * (yp.v[i] + ym.v[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < VN; ++i) res[b].v[i] = vcur.v[i] * qb[4].v[i] + d[i];
+            // one band's LDS values live at a time
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+        // projector term: one trip per list entry, the same number for all lanes of the wavefront
+        // (an entry's channels are summed before they meet the larger stencil value)
+        auto trip = [&](const Entry& e) {
+            const int li = (int)(e.w & 1023u);
+            const int dyi = ((int)(e.w << 11)) >> 21, dxi = ((int)e.w) >> 21;
+            const T* im = imf + 4 * li;
+            T fx, fy, fz, nzf;
+            if constexpr (VN == 4) {
+                const Row<T> w = *reinterpret_cast<const Row<T>*>(im);
+                fx = w.v[0]; fy = w.v[1]; fz = w.v[2]; nzf = w.v[3];
+            } else {
+                const Row<T> w0 = *reinterpret_cast<const Row<T>*>(im), w1 = *reinterpret_cast<const Row<T>*>(im + 2);
+                fx = w0.v[0]; fy = w0.v[1]; fz = w1.v[0]; nzf = w1.v[1];
+            }
+            const T dx0 = hx * ((T)dxi - fx), dy = hy * ((T)dyi - fy), dz = hz * (((T)z - nzf) - fz);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                T c[NC];
+                const Row<T>* ep = reinterpret_cast<const Row<T>*>(ec + ((size_t)li * NB + b) * NC);
+#pragma unroll
+                for (int k = 0; k < NC / VN; ++k) {
+                    const Row<T> w = ep[k];
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) c[k * VN + u] = w.v[u];
+                }
+T val[VN];
+#pragma unroll
+                for (int u = 0; u < VN; ++u) val[u] = e.f[0].v[u] * c[0];
+#pragma unroll
+                for (int s = 1; s < NS; ++s)
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) val[u] += e.f[s].v[u] * c[s];
+#pragma unroll
+                for (int p = 0; p < NP; ++p) {
+                    const T cy = c[NS + 3 * p], cz = c[NS + 3 * p + 1], cx = c[NS + 3 * p + 2];
+                    const T ayz = cy * dy + cz * dz;
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) val[u] += e.f[NS + p].v[u] * (ayz + cx * (dx0 + (T)u * hx));
+                }
+#pragma unroll
+                for (int u = 0; u < VN; ++u) res[b].v[u] += val[u];
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (k < n) trip(en[k]);
+        if (n > K) {
+            const rsrc_t rvals = rsrc((const unsigned char*)a.vals + (int64_t)tb * NV * 1024, (uint32_t)n * NV * 1024);
+            const rsrc_t rwords = rsrc(a.words + (int64_t)tb * 64, (uint32_t)n * 256);
+            for (int k = K; k < n; ++k) trip(load_entry(rvals, rwords, k));
+        }
+        load_entries(zn);
+        // lanes without a point store out of range (dropped)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) vstore<T>(rout[b], res[b], vo, zoff(z));
+    };
+    for (int z = z0;;) {
+        step(std::integral_constant<int, 0>{}, z);
+        if (++z >= z1) break;
+        step(std::integral_constant<int, 1>{}, z);
+        if (++z >= z1) break;
+        step(std::integral_constant<int, 2>{}, z);
+        if (++z >= z1) break;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const Row<T> next = q[b][0];
+#pragma unroll
+            for (int d = 0; d < 8; ++d) q[b][d] = q[b][d + 3];
+            q[b][8] = next;
+        }
+    }
+}
+
+template <class T, int NB, int NS, int NP, bool RAG, int HV>
+__global__ __launch_bounds__(kMaxThreads) void sphere_hpsi_kernel(SphereArgs a, Coef8<T> sc, const T* __restrict__ V,
+                                                                  const T* __restrict__ psi, T* __restrict__ out) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    sphere_body<T, NB, NS, NP, RAG, HV>(a, sc, V, psi, out, xcd_order(blockIdx.x, gridDim.x), smem);
+}
+
+// ------------------------------------------------------------------ entry lists ----
+// radial function of a channel at squared distance rr (inside its cutoff), FP64:
+// RadialGrid2::GetValueByXi (RadialGrid2.h:81-136) for tables
+__device__ double radial_dev(const DevProj& d, const double* tables, double rr) {
+    if (d.kind == QG_RADIAL_GAUSSIAN) return d.amp * exp(-rr * d.inv_2s2);
+    const double* v = tables + d.table_off;
+    if (d.r_min2 > rr) return v[0];
+    const double rel = 0.5 * log(rr) - d.xi_min;
+    const double fl = floor(rel / d.xi_delta);
+    const int i = (int)fl, n = d.n_table;
+    if (i >= n - 1) return 0.0;
+    if (i == 0 || i == n - 2) {
+        const double t = rel / d.xi_delta - fl;
+        return v[i] * (1.0 - t) + v[i + 1] * t;
+    }
+    const double t = rel / d.xi_delta - (double)i;
+    if (1 < i && i < n - 3) {
+        const double fm2 = v[i - 2], fm1 = v[i - 1], f0 = v[i], f1 = v[i + 1], f2 = v[i + 2], f3 = v[i + 3];
+        const double g0 = 2.0 / 3.0 * (f1 - fm1) - 1.0 / 12.0 * (f2 - fm2);
+        const double g1 = 2.0 / 3.0 * (f2 - f0) - 1.0 / 12.0 * (f3 - fm1);
+        const double h0 = 4.0 / 3.0 * (f1 + fm1) - 1.0 / 12.0 * (f2 + fm2) - 5.0 / 2.0 * f0;
+        const double h1 = 4.0 / 3.0 * (f2 + f0) - 1.0 / 12.0 * (f3 + fm1) - 5.0 / 2.0 * f1;
+        const double e0 = f1 - (f0 + g0 + h0 / 2.0);
+        const double e1 = g1 - (g0 + h0);
+        const double e2 = h1 - h0;
+        const double a3 = 10.0 * e0 - 4.0 * e1 + 0.5 * e2;
+        const double a4 = -15.0 * e0 + 7.0 * e1 - e2;
+        const double a5 = f1 - f0 - g0 - h0 / 2.0 - a3 - a4;
+        return f0 + t * (g0 + t * (h0 / 2.0 + t * (a3 + t * (a4 + t * a5))));
+    }
+    const double v0 = v[i], v1 = v[i + 1];
+    const double s1 = (v[i + 2] - v0) / 2.0, s0 = (v1 - v[i - 1]) / 2.0;
+    const double a = s1 + s0 - 2.0 * (v1 - v0);
+    const double b = -s1 - 2.0 * s0 + 3.0 * (v1 - v0);
+    return a * t * t * t + b * t * t + s0 * t + v0;
+}
+
+struct BuildArgs {
+    int nx, ny, nz, ty, ntile, nq, tpb, nw;
+    double h[3];
+    const int* col_off;
+    const int* col_img;
+    const SphereImage* images;
+    const DevImage* parts;       // the per-cutoff images a sphere image is made of
+    const int2* intervals;
+    const DevProj* projs;
+    const double* tables;
+    const int* atom_chan;
+    int* trips;                  // counting pass: trips per (tile, plane, wavefront)
+    const int* trip_off;         // filling pass
+    uint32_t* words;
+    void* vals;
+};
+
+// the in-cutoff x range of part p on row (y, z), or an empty one
+__device__ __forceinline__ int2 part_row(const BuildArgs& a, const DevImage& p, int y, int z) {
+    if (z < p.b[2] || z >= p.e[2] || y < p.b[1] || y >= p.e[1]) return make_int2(0, 0);
+    return a.intervals[p.row_base + (y - p.b[1]) + (p.e[1] - p.b[1]) * (z - p.b[2])];
+}
+
+// One workgroup per (tile, plane), one thread per lane of the apply workgroup.  FILL false:
+// counts the images touching each lane's group and records the wavefront's largest count; FILL
+// true: writes the lane's entries and pads to that count with the empty image.
+template <class T, int NS, int NP, bool FILL>
+__global__ __launch_bounds__(kMaxThreads) void sphere_build_kernel(BuildArgs a) {
+    constexpr int VN = 16 / sizeof(T);
+    constexpr int NV = NS + NP;
+    const int tile = blockIdx.x, z = blockIdx.y;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int y0 = tile * a.ty;
+    const int r = tid / a.nq;
+    const int x = min((tid - r * a.nq) * VN, a.nx - VN);
+    const int y = y0 + r;
+    const bool own = r < min(a.ty, a.ny - y0);
+    const int c0 = a.col_off[tile], ncol = a.col_off[tile + 1] - c0;
+    const size_t w = ((size_t)tile * a.nz + z) * a.nw + wave;
+    int n = 0;
+    const int base = FILL ? a.trip_off[w] : 0;
+    Row<T>* vals = reinterpret_cast<Row<T>*>(a.vals);
+    for (int li = 0; own && li < ncol; ++li) {
+        const SphereImage im = a.images[a.col_img[c0 + li]];
+        bool touch = false;
+        for (int k = 0; k < im.nparts; ++k) {
+            const int2 iv = part_row(a, a.parts[im.part[k]], y, z);
+            touch = touch || (iv.x < x + VN && iv.y > x);
+        }
+        if (!touch) continue;
+        if constexpr (FILL) {
+            Row<T> f[NV];
+#pragma unroll
+            for (int c = 0; c < NV; ++c)
+#pragma unroll
+                for (int u = 0; u < VN; ++u) f[c].v[u] = T(0);
+            for (int k = 0; k < im.nparts; ++k) {
+                const DevImage& p = a.parts[im.part[k]];
+                const int2 iv = part_row(a, p, y, z);
+                const double dz = a.h[2] * (double)(z - p.shift[2]) - p.R[2];
+                const double dy = a.h[1] * (double)(y - p.shift[1]) - p.R[1];
+                for (int pj = p.proj_begin; pj < p.proj_end; ++pj) {
+                    const DevProj& d = a.projs[pj];
+#pragma unroll
+                    for (int c = 0; c < NV; ++c) {
+                        // the channel of this projector: the one whose coefficient slot it fills
+                        if (a.atom_chan[4 * im.atom + (c < NS ? c : 2 + c - NS)] != d.coef_rel) continue;
+                        if ((d.l == 0) != (c < NS)) continue;
+#pragma unroll
+                        for (int u = 0; u < VN; ++u) {
+                            if (x + u < iv.x || x + u >= iv.y) continue;
+                            const double dx = a.h[0] * (double)(x + u - p.shift[0]) - p.R[0];
+                            const double rr = dx * dx + (dy * dy + dz * dz);
+                            const double rad = radial_dev(d, a.tables, rr);
+                            if (d.l == 0) f[c].v[u] = (T)(rad * 0.28209479177387814);          // Y00
+                            else f[c].v[u] = 1.0e-14 > rr ? T(0) : (T)(rad * 0.48860251190291992 / sqrt(rr));
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < NV; ++c) vals[((size_t)(base + n) * NV + c) * 64 + lane] = f[c];
+            a.words[(size_t)(base + n) * 64 + lane] = entry_word(li, x - im.n[0], y - im.n[1]);
+        }
+        ++n;
+    }
+    if constexpr (FILL) {
+        const int cnt = a.trip_off[w + 1] - base;
+        for (; n < cnt; ++n) {
+#pragma unroll
+            for (int c = 0; c < NV; ++c) vals[((size_t)(base + n) * NV + c) * 64 + lane] = Row<T>{};
+            a.words[(size_t)(base + n) * 64 + lane] = entry_word(ncol, 0, 0);
+        }
+    } else {
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) n = max(n, __shfl_xor(n, s, 64));
+        if (lane == 0) a.trips[w] = n;
+    }
+}
+
+// ------------------------------------------------------------------------ host side ----
+// Tile rows for groups of nq per row: the largest product of lane use, the share of the staged
+// rows that are the tile's own (8 halo rows), the share of tile rows inside the grid, and the
+// wavefront slots filled (two bands per workgroup take ~175 VGPRs, so a CU holds 8 wavefronts;
+// one workgroup of 8 stalls at its barriers where two of 4 overlap: 2.59 against 2.30 ms at
+// 120^3, ty 16 and 8, while 12 rows beat 8 by 183 to 214 us at 80^3 / 128 FP32 bands and by 0.88
+// to 1.0 ms at 80 x 80 x 120 / 192 FP64 bands)
+static int sphere_pick_ty(int nq, int ny, int want) {
+    if (nq > kMaxThreads) return 0;
+    const int most = std::max(1, std::min(ny, kMaxThreads / nq));
+    if (want > 0) return std::max(1, std::min(most, std::min(32, want)));
+    int best = 1;
+    double bests = -1.0;
+    for (int ty = 1; ty <= std::min(most, 16); ++ty) {
+        const int tpb = round64i(ty * nq), w = tpb / 64, ntile = (ny + ty - 1) / ty;
+        const double slots = w <= 4 ? (8 / w) * w / 8.0 : 0.75 * w / 8.0;
+        const double score = (double)ty * nq / tpb * ty / (ty + 8.0) * ny / ((double)ntile * ty) * slots;
+        if (score > bests) { bests = score; best = ty; }
+    }
+    return best;
+}
+
+static SphereForm sphere_form(const NlGeometry& geo, std::vector<int>& chan) {
+    // coefficient slots of every atom's s, s, p, p channels; the kernels hold up to 2 + 2
+    chan.assign((size_t)std::max(1, geo.natoms) * 4, -1);
+    int ns = 0, np = 0;
+    std::vector<char> seen(geo.natoms, 0);
+    for (const DevImage& im : geo.images) {
+        int* c = &chan[4 * (size_t)im.atom];
+        for (int pj = im.proj_begin; pj < im.proj_end; ++pj) {
+            const DevProj& d = geo.projs[pj];
+            const int first = d.l == 0 ? 0 : 2;
+            int k = 0;
+            while (k < 2 && c[first + k] >= 0 && c[first + k] != d.coef_rel) ++k;
+            if (k == 2) return SphereForm{};
+            c[first + k] = d.coef_rel;
+            (d.l == 0 ? ns : np) = std::max(d.l == 0 ? ns : np, k + 1);
+        }
+    }
+    return (ns <= 1 && np <= 1) ? SphereForm{1, 1} : SphereForm{2, 2};
+}
+
+bool sphere_serves(const qg_grid& g, const qg_nonlocal* nl) {
+    if (env_int("QG_SPHERE", 1) == 0) return false;
+    if (g.n[0] < 8 || g.n[0] > 1024 || g.n[2] < 8) return false;
+    if (g.ng() * 8 > (int64_t)kOOB - 64) return false;   // band bytes below the out-of-range offset
+    return nl->geo.ncoef > 0 && !nl->geo.images.empty() && nl->sphere_form.ns > 0;
+}
+
+// Sphere images of the whole cell (one per atom and periodic shift, all cutoffs together) and
+// the channel slots, from the per-cutoff images of the geometry.
+static void sphere_images(qg_nonlocal* nl) {
+    const NlGeometry& geo = nl->geo;
+    std::vector<int> chan;
+    nl->sphere_form = sphere_form(geo, chan);
+    nl->sphere_img.clear();
+    if (nl->sphere_form.ns == 0) return;
+    std::map<std::tuple<int, int, int, int>, int> at;
+    for (int i = 0; i < (int)geo.images.size(); ++i) {
+        const DevImage& im = geo.images[i];
+        const auto key = std::make_tuple(im.atom, im.shift[0], im.shift[1], im.shift[2]);
+        auto it = at.find(key);
+        if (it == at.end()) {
+            it = at.emplace(key, (int)nl->sphere_img.size()).first;
+            SphereImage s{};
+            s.atom = im.atom;
+            for (int d = 0; d < 3; ++d) {
+                const double u = im.R[d] / nl->gcopy.h[d], nn = std::rint(u);
+                s.n[d] = im.shift[d] + (int)nn;
+                s.f[d] = u - nn;
+                s.b[d] = im.b[d];
+                s.e[d] = im.e[d];
+            }
+            nl->sphere_img.push_back(s);
+        }
+        SphereImage& s = nl->sphere_img[it->second];
+        if (s.nparts == 4) { nl->sphere_form = SphereForm{}; return; }
+        s.part[s.nparts++] = i;
+        for (int d = 0; d < 3; ++d) {
+            s.b[d] = std::min(s.b[d], im.b[d]);
+            s.e[d] = std::max(s.e[d], im.e[d]);
+            // displacements beyond the entry word's 11-bit fields
+            if (s.e[d] - s.b[d] > 900) { nl->sphere_form = SphereForm{}; return; }
+        }
+    }
+    nl->d_sphere_img.upload(nl->sphere_img.data(), nl->sphere_img.size());
+    nl->d_atom_chan.upload(chan.data(), chan.size());
+}
+
+// Entry lists of tile rows ty for the block type, built on the device on first use.
+static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build) {
+    std::lock_guard<std::mutex> lk(nl->rows_mu);
+    for (auto& c : nl->sphere)
+        if (c->ty == ty && c->dtype == dtype) return c.get();
+    if (!build) return nullptr;
+    const qg_grid& g = nl->gcopy;
+    auto c = std::make_unique<SphereGeo>();
+    const int VN = dtype == QG_F32 ? 4 : 2;
+    c->ty = ty;
+    c->dtype = dtype;
+    c->nq = (g.n[0] + VN - 1) / VN;
+    c->tpb = round64i(ty * c->nq);
+    c->ntile = (g.n[1] + ty - 1) / ty;
+    const int nw = c->tpb / 64, nz = g.n[2];
+    std::vector<std::vector<int>> col(c->ntile);
+    for (int i = 0; i < (int)nl->sphere_img.size(); ++i) {
+        const SphereImage& im = nl->sphere_img[i];
+        for (int t = im.b[1] / ty; t <= (im.e[1] - 1) / ty; ++t) col[t].push_back(i);
+    }
+    std::vector<int> off(1, 0), img;
+    for (auto& v : col) {
+        img.insert(img.end(), v.begin(), v.end());
+        off.push_back((int)img.size());
+        c->max_col = std::max(c->max_col, (int)v.size());
+    }
+    if (img.empty()) img.push_back(0);
+    if (c->max_col < 1023) {
+        c->d_col_off.upload(off.data(), off.size());
+        c->d_col_img.upload(img.data(), img.size());
+        BuildArgs a{};
+        a.nx = g.n[0]; a.ny = g.n[1]; a.nz = nz;
+        a.ty = ty; a.ntile = c->ntile; a.nq = c->nq; a.tpb = c->tpb; a.nw = nw;
+        for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
+        a.col_off = c->d_col_off.p; a.col_img = c->d_col_img.p;
+        a.images = nl->d_sphere_img.p; a.parts = nl->d_images.p; a.intervals = nl->d_intervals.p;
+        a.projs = nl->d_projs.p; a.tables = nl->d_tables.p; a.atom_chan = nl->d_atom_chan.p;
+        const size_t nwv = (size_t)c->ntile * nz * nw;
+        std::vector<int> trips(nwv + 1, 0);
+        c->d_trip_off.alloc(nwv + 1);
+        a.trips = c->d_trip_off.p;
+        const bool two = nl->sphere_form.ns == 2;
+        auto launch = [&](auto tag, bool fill) {
+            using T = decltype(tag);
+            const dim3 grid(c->ntile, nz), blk(c->tpb);
+            if (two) {
+                if (fill) hipLaunchKernelGGL((sphere_build_kernel<T, 2, 2, true>), grid, blk, 0, nullptr, a);
+                else hipLaunchKernelGGL((sphere_build_kernel<T, 2, 2, false>), grid, blk, 0, nullptr, a);
+            } else {
+                if (fill) hipLaunchKernelGGL((sphere_build_kernel<T, 1, 1, true>), grid, blk, 0, nullptr, a);
+                else hipLaunchKernelGGL((sphere_build_kernel<T, 1, 1, false>), grid, blk, 0, nullptr, a);
+            }
+            QG_HIP(hipGetLastError());
+        };
+        dtype == QG_F32 ? launch(float{}, false) : launch(double{}, false);
+        QG_HIP(hipMemcpy(trips.data(), c->d_trip_off.p, nwv * sizeof(int), hipMemcpyDeviceToHost));
+        int64_t total = 0;
+        for (size_t k = 0; k <= nwv; ++k) {
+            const int n = k < nwv ? trips[k] : 0;
+            trips[k] = (int)std::min<int64_t>(total, INT32_MAX);
+            total += n;
+        }
+        const int nv = nl->sphere_form.ns + nl->sphere_form.np;
+        if (total < (1LL << 30)) {
+            c->ntrips = (int)std::max<int64_t>(1, total);
+            c->d_trip_off.upload(trips.data(), trips.size());
+            c->d_words.alloc((size_t)c->ntrips * 64);
+            c->d_vals.alloc((size_t)c->ntrips * 64 * nv * 16);
+            a.trip_off = c->d_trip_off.p;
+            a.words = c->d_words.p;
+            a.vals = c->d_vals.p;
+            dtype == QG_F32 ? launch(float{}, true) : launch(double{}, true);
+            QG_HIP(hipStreamSynchronize(nullptr));
+            c->ok = true;
+        }
+    }
+    nl->sphere.push_back(std::move(c));
+    return nl->sphere.back().get();
+}
+
+// Device state of the geometry just built into nl, with the entry lists of the default tile
+// heights (so that applications on caller scratch need not allocate).
+void sphere_prepare(qg_nonlocal* nl) {
+    nl->sphere.clear();
+    sphere_images(nl);
+    if (!sphere_serves(nl->gcopy, nl)) return;
+    for (int dtype : {QG_F32, QG_F64}) {
+        const int VN = dtype == QG_F32 ? 4 : 2;
+        const int ty = sphere_pick_ty((nl->gcopy.n[0] + VN - 1) / VN, nl->gcopy.n[1], 0);
+        if (ty > 0) sphere_geometry(nl, dtype, ty, true);
+    }
+}
+
+// 16-byte vectors of the 8 halo rows each thread stages
+static int sphere_halo_vectors(int nq, int tpb) { return (8 * nq + tpb - 1) / tpb; }
+
+template <class T, int NB, int NS, int NP>
+static void sphere_launch(const SphereArgs& a, const Coef8<T>& sc, const T* V, const T* psi, T* out, size_t lds,
+                          hipStream_t s) {
+    const int64_t nwg = (int64_t)a.ntile * a.nslab * ((a.nbands + NB - 1) / NB);
+    QG_REQUIRE(nwg < (1LL << 31), "too many workgroups");
+    const dim3 grid((unsigned)nwg), blk(a.tpb);
+    const bool rag = a.nx % (16 / (int)sizeof(T)) != 0;
+    const int hv = sphere_halo_vectors(a.nq, a.tpb);
+    QG_REQUIRE(hv <= (NB == 1 ? 8 : 1), "row tile too low for its halo");
+#define QG_SPHERE_GO(RAG, HV) \
+    hipLaunchKernelGGL((sphere_hpsi_kernel<T, NB, NS, NP, RAG, HV>), grid, blk, lds, s, a, sc, V, psi, out)
+    if (hv <= 1) {
+        if (rag) QG_SPHERE_GO(true, 1);
+        else QG_SPHERE_GO(false, 1);
+    } else if constexpr (NB == 1) {
+        if (hv == 2) {
+            if (rag) QG_SPHERE_GO(true, 2);
+            else QG_SPHERE_GO(false, 2);
+        } else {
+            if (rag) QG_SPHERE_GO(true, 8);
+            else QG_SPHERE_GO(false, 8);
+        }
+    }
+#undef QG_SPHERE_GO
+    QG_HIP(hipGetLastError());
+}
+
+template <class T>
+static size_t sphere_lds_of(const qg_nonlocal* nl, const SphereGeo& sg, int nb) {
+    return sphere_lds<T>(nl->gcopy.n[0], sg.ty, nb, nl->sphere_form.ns, nl->sphere_form.np, sg.max_col);
+}
+
+// Whether the apply pass of the block type runs on the entry lists prepared with the geometry
+// (with one band per workgroup at least).
+bool sphere_prepared(qg_nonlocal* nl, int dtype) {
+    if (!sphere_serves(nl->gcopy, nl)) return false;
+    const int VN = dtype == QG_F32 ? 4 : 2;
+    const int nq = (nl->gcopy.n[0] + VN - 1) / VN;
+    const int ty = sphere_pick_ty(nq, nl->gcopy.n[1], 0);
+    const SphereGeo* sg = ty > 0 ? sphere_geometry(nl, dtype, ty, false) : nullptr;
+    return sg && sg->ok && sphere_halo_vectors(nq, sg->tpb) <= 8 &&
+           (dtype == QG_F32 ? sphere_lds_of<float>(nl, *sg, 1) : sphere_lds_of<double>(nl, *sg, 1)) <= lds_limit();
+}
+
+template <class T>
+static bool sphere_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hpsi, int64_t ld_out,
+                           const double* coef, bool may_build, bool run, hipStream_t s) {
+    const qg_grid& g = h->grid;
+    qg_nonlocal* nl = h->nl;
+    constexpr int VN = 16 / sizeof(T);
+    const int dtype = sizeof(T) == 4 ? QG_F32 : QG_F64;
+    const int nq = (g.n[0] + VN - 1) / VN;
+    int ty = sphere_pick_ty(nq, g.n[1], h->plan.rows_ty);
+    if (ty == 0) return false;
+    const SphereGeo* sg = sphere_geometry(nl, dtype, ty, may_build);
+    if (!sg && h->plan.rows_ty > 0) {
+        // nothing may be built now: the tile height prepared with the geometry
+        ty = sphere_pick_ty(nq, g.n[1], 0);
+        sg = sphere_geometry(nl, dtype, ty, false);
+    }
+    if (!sg || !sg->ok) return false;
+    const bool two = nl->sphere_form.ns == 2;
+    // two bands per workgroup (an entry is loaded once for both) where that leaves two
+    // workgroups per CU
+    int nb = h->plan.rows_bands > 0 ? std::min(2, h->plan.rows_bands)
+                                    : ((int64_t)sg->ntile * ((nbands + 1) / 2) >= 512 ? 2 : 1);
+    auto lds_of = [&](int b) { return sphere_lds_of<T>(nl, *sg, b); };
+    if (nb > 1 && (sphere_halo_vectors(nq, sg->tpb) > 1 || lds_of(nb) > lds_limit())) nb = 1;
+    if (lds_of(nb) > lds_limit() || sphere_halo_vectors(nq, sg->tpb) > 8) return false;
+    if (!run) return true;
+    SphereArgs a{};
+    a.nx = g.n[0]; a.ny = g.n[1]; a.nz = g.n[2];
+    a.ty = ty;
+    a.ntile = sg->ntile;
+    // two neighbouring tiles, then all bands: the workgroups an XCD runs together share the
+    // entry lists and V in its L2 (per application of 512 FP32 bands at 120^3 the pass reads
+    // 8.0 GB so, 10.2 GB with 4 tiles, more with all)
+    a.tg = std::min(sg->ntile, 2);
+    a.nq = nq; a.tpb = sg->tpb; a.nw = sg->tpb / 64;
+    // z-slabs for about 2048 workgroups, of at least 8 planes (a slab re-reads 8), or of 3 where
+    // the workgroups are too few to fill the chip: then a workgroup's chain of planes is the time
+    // (24^3, 8 bands: 12.9 us in slabs of 8, 8.8 of 3; 40^3, 16 FP32 bands: 14.8 us of 8, 11.8 of 4)
+    const int64_t wg = (int64_t)a.ntile * ((nbands + nb - 1) / nb);
+    const int least = wg * std::max(1, g.n[2] / 8) < 512 ? 3 : 8;
+    const int nslab = (int)std::max<int64_t>(1, std::min<int64_t>((2048 + wg - 1) / wg, std::max(1, g.n[2] / least)));
+    a.tz = h->plan.rows_tz > 0 ? std::min(g.n[2], h->plan.rows_tz) : (g.n[2] + nslab - 1) / nslab;
+    a.nslab = (g.n[2] + a.tz - 1) / a.tz;
+    a.nbands = nbands;
+    a.ld_in = ld; a.ld_out = ld_out;
+    a.col_off = sg->d_col_off.p; a.col_img = sg->d_col_img.p;
+    a.images = nl->d_sphere_img.p;
+    a.trip_off = sg->d_trip_off.p;
+    a.ntrips = sg->ntrips;
+    a.vals = sg->d_vals.p; a.words = sg->d_words.p;
+    a.coef = coef; a.coef_energy = nl->d_coef_energy.p; a.atom_coef_off = nl->d_atom_coef_off.p;
+    a.atom_chan = nl->d_atom_chan.p;
+    a.ncoef = nl->geo.ncoef;
+    a.max_col = sg->max_col;
+    for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
+    const T* V = sizeof(T) == 4 ? (const T*)(const void*)h->V32.p : (const T*)(const void*)h->V64.p;
+    const Coef8<T> sc = coef8<T>(g, -0.5);
+    const size_t lds = lds_of(nb);
+    if (two) {
+        if (nb == 2) sphere_launch<T, 2, 2, 2>(a, sc, V, psi, hpsi, lds, s);
+        else sphere_launch<T, 1, 2, 2>(a, sc, V, psi, hpsi, lds, s);
+    } else {
+        if (nb == 2) sphere_launch<T, 2, 1, 1>(a, sc, V, psi, hpsi, lds, s);
+        else sphere_launch<T, 1, 1, 1>(a, sc, V, psi, hpsi, lds, s);
+    }
+    return true;
+}
+
+// H psi = V psi - 1/2 Lap8 psi + sum E c beta from the coefficients coef (nbands x ncoef), in
+// one launch; false (nothing launched) where the entry lists do not serve the grid or projector
+// set.  may_build: the lists of this tile height may be built now.  run false: only says whether
+// the call would be served.
+bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
+                              int64_t ld_out, const double* coef, bool may_build, bool run,
+                              hipStream_t s) {
+    if (!h->nl || !sphere_serves(h->grid, h->nl)) return false;
+    if (dtype == QG_F32)
+        return sphere_apply_t<float>(h, nbands, (const float*)psi, ld, (float*)hpsi, ld_out, coef, may_build,
+                                     run, s);
+    return sphere_apply_t<double>(h, nbands, (const double*)psi, ld, (double*)hpsi, ld_out, coef, may_build,
+                                  run, s);
+}
+
+}  // namespace qg
