@@ -19,9 +19,10 @@
 // backward passes of N); Adam.  Weights are kept in FP32 for training; the preconditioner
 // applies the BF16-rounded weights with FP32 accumulation.
 //
-// Convolution kernels: direct 3x3x3, one workgroup per 16 x 8 x 4 output tile and band, the
-// input tile (+1 halo, periodic wrap) and the weights staged in LDS, each lane accumulating its
-// 4 z-points x COUT channels in registers.
+// Convolution kernels: training and the FP32 weights run conv3_kernel (direct 3x3x3 FMA, one
+// workgroup per 16 x 8 x 4 output tile and band, the input tile with its periodic halo and the
+// weights staged in LDS, each lane accumulating its 4 z-points x COUT channels in registers); the
+// preconditioner's BF16 weights run conv3_split_kernel (the same sums on the matrix cores).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -251,6 +252,185 @@ __global__ __launch_bounds__(kMThreads) void conv3_mfma_kernel(ConvArgs a, const
                 float val = acc[i];
                 if constexpr (OUT_MODE == OUT_GATE) val *= 1.f + tanhf(a.ga[co] * a.v[gi] + a.gb[co]);
                 out[(int64_t)b * a.out_bs + co * a.ng + gi] = val;
+            }
+        }
+    }
+}
+
+// ----------------------------------------------------- exact-split MFMA convolution ----
+// Inference form of conv3_kernel with FP32 activations on the matrix cores.  The weights are
+// BF16-valued; each FP32 activation is cut by bit masks into three BF16 parts, x = hi + mid + lo
+// exactly (8 + 8 + 8 significand bits), so the three products per tap are exact and only the FP32
+// accumulation rounds, as in the FMA form.
+//
+// One workgroup computes a 16 x 8 x 4 output tile for a run of bands, one wavefront 16 x-points of
+// 4 y-rows and 2 z-planes, as v_mfma_f32_16x16x32_bf16 products:
+//   A (16 points x K), K = (input plane of 4) x (input channel of 8),
+//   B (K x 16),        column n = zo * 8 + co, B[(zin, ci)][n] = w[co][ci][zin - zo][dy][dx]
+//                      (zero outside the 3-tap band: 3/4 of the products are used; a non-finite
+//                      activation so reaches one plane further than its taps, which the Fourier
+//                      transforms on both sides of the network make no difference),
+// one per (dy, dx) and part.  An input row is read from LDS once per dx and part and serves the
+// three output rows it touches (LDS reads and products then take about equal time); B stays in
+// registers, the gates of the tile are formed once for all its bands, and the next band's
+// activations are loaded while the current one is multiplied.
+// An 8 -> 8 layer of 27 bands at 80^3 takes 564 us (1511 us in the FMA form, VALU-bound); products,
+// LDS reads and the splitting take ~85, ~145 and ~130 us of it, three workgroups per CU overlap
+// them in part.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+constexpr int kSX = 16, kSY = 8, kSZ = 4;
+constexpr int kSLX = kSX + 2, kSLY = kSY + 2, kSLZ = kSZ + 2;
+constexpr int kSPts = kSLX * kSLY * kSLZ;
+constexpr int kSThreads = 256;
+constexpr int kSPT = (kSPts + kSThreads - 1) / kSThreads;   // staged points per thread
+
+// the exact parts of eight channel values, packed as BF16
+__device__ __forceinline__ void split3(const float (&x)[8], bf16x8_t& hi, bf16x8_t& mid, bf16x8_t& lo) {
+    using u4_t = __attribute__((ext_vector_type(4))) uint32_t;
+    u4_t h, m, l;
+#pragma unroll
+    for (int c = 0; c < 8; c += 2) {
+        uint32_t hb[2], mb[2], lb[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float v = x[c + k];
+            hb[k] = __float_as_uint(v) & 0xffff0000u;
+            // an infinity is its own high part (inf - inf would make it NaN)
+            const float r = __builtin_isinf(v) ? 0.f : v - __uint_as_float(hb[k]);
+            mb[k] = __float_as_uint(r) & 0xffff0000u;
+            lb[k] = __float_as_uint(r - __uint_as_float(mb[k]));
+        }
+        h[c / 2] = (hb[0] >> 16) | hb[1];
+        m[c / 2] = (mb[0] >> 16) | mb[1];
+        l[c / 2] = (lb[0] >> 16) | (lb[1] & 0xffff0000u);
+    }
+    hi = __builtin_bit_cast(bf16x8_t, h);
+    mid = __builtin_bit_cast(bf16x8_t, m);
+    lo = __builtin_bit_cast(bf16x8_t, l);
+}
+
+template <int CIN, int COUT, int IN_MODE, int OUT_MODE>
+__global__ __launch_bounds__(kSThreads, 3) void conv3_split_kernel(ConvArgs a, int nb, int bl, int tiles_x, int tiles_y,
+                                                                int ntile, const float* __restrict__ w,
+                                                                const float* __restrict__ in, float* __restrict__ out) {
+    static_assert(CIN <= 8 && COUT <= 8, "at most 8 channels");
+    constexpr int CR = IN_MODE == IN_UV ? 1 : CIN;     // channels read
+    __shared__ __align__(16) __bf16 tile[3 * kSPts * 8];
+    // consecutive tiles (which share halo rows) on one XCD
+    const int nwg = gridDim.x, per = nwg >> 3, rem = nwg & 7, xcd = blockIdx.x & 7;
+    const int wg = ((xcd < rem) ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (blockIdx.x >> 3);
+    const int t = wg % ntile;
+    const int b0 = (wg / ntile) * bl, b1 = min(nb, b0 + bl);
+    const int x0 = (t % tiles_x) * kSX, y0 = (t / tiles_x) % tiles_y * kSY, z0 = t / (tiles_x * tiles_y) * kSZ;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = lane & 15, kg = lane >> 4, co = n & 7, zo = n >> 3;
+    const int zp = wave & 1, yh = wave >> 1;
+
+    bf16x8_t bw[9];
+    {
+        const int dz = kg - zo;
+#pragma unroll
+        for (int s = 0; s < 9; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                float val = 0.f;
+                if (co < COUT && j < CIN && dz >= 0 && dz <= 2) val = w[(co * CIN + j) * kTaps + dz * 9 + s];
+                bw[s][j] = (__bf16)val;
+            }
+    }
+    // staged points of this thread (periodic wrap), clamped past the tile
+    int gi[kSPT];
+    float vin[kSPT];
+#pragma unroll
+    for (int k = 0; k < kSPT; ++k) {
+        const int i = min(tid + k * kSThreads, kSPts - 1);
+        const int xx = i % kSLX, yy = (i / kSLX) % kSLY, zz = i / (kSLX * kSLY);
+        gi[k] = wrapi(x0 + xx - 1, a.nx) + a.nx * (wrapi(y0 + yy - 1, a.ny) + a.ny * wrapi(z0 + zz - 1, a.nz));
+        vin[k] = IN_MODE == IN_UV ? a.v[gi[k]] : 0.f;
+    }
+    // output points of this lane: 4 consecutive x of rows yh * 4 .. + 3, plane zp * 2 + zo
+    const int gx = x0 + 4 * kg, gz = z0 + 2 * zp + zo;
+    float g[4][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            g[r][i] = 0.f;
+            if constexpr (OUT_MODE != OUT_PLAIN) {
+                const int gy = y0 + 4 * yh + r;
+                const float vv = a.v[min(gx + i, a.nx - 1) + (int64_t)a.nx * (min(gy, a.ny - 1) + (int64_t)a.ny * min(gz, a.nz - 1))];
+                g[r][i] = OUT_MODE == OUT_GATE ? 1.f + tanhf(a.ga[co] * vv + a.gb[co]) : vv;
+            }
+        }
+    float pre[kSPT][CR];
+    auto load = [&](int b) {
+        const float* p = in + (int64_t)b * a.in_bs;
+#pragma unroll
+        for (int k = 0; k < kSPT; ++k)
+#pragma unroll
+            for (int c = 0; c < CR; ++c) pre[k][c] = p[c * a.ng + gi[k]];
+    };
+    load(b0);
+    for (int b = b0; b < b1; ++b) {
+#pragma unroll
+        for (int k = 0; k < kSPT; ++k) {
+            const int i = tid + k * kSThreads;
+            float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if constexpr (IN_MODE == IN_UV) {
+                x[0] = pre[k][0];
+                x[1] = vin[k] * pre[k][0];
+            } else {
+#pragma unroll
+                for (int c = 0; c < CR; ++c) x[c] = pre[k][c];
+            }
+            bf16x8_t hi, mid, lo;
+            split3(x, hi, mid, lo);
+            if (i < kSPts) {
+                *reinterpret_cast<bf16x8_t*>(&tile[i * 8]) = hi;
+                *reinterpret_cast<bf16x8_t*>(&tile[(kSPts + i) * 8]) = mid;
+                *reinterpret_cast<bf16x8_t*>(&tile[(2 * kSPts + i) * 8]) = lo;
+            }
+        }
+        __syncthreads();
+        load(min(b + 1, b1 - 1));
+        f32x4_t acc[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int yi = 0; yi < 6; ++yi)
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int part = 2; part >= 0; --part) {
+                    const bf16x8_t av = *reinterpret_cast<const bf16x8_t*>(
+                        &tile[(part * kSPts + ((2 * zp + kg) * kSLY + 4 * yh + yi) * kSLX + n + dx) * 8]);
+#pragma unroll
+                    for (int dy = 0; dy < 3; ++dy)
+                        if (yi - dy >= 0 && yi - dy < 4)
+                            acc[yi - dy] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[dy * 3 + dx], acc[yi - dy], 0, 0, 0);
+                }
+        __syncthreads();   // the tile is staged again for the next band
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int gy = y0 + 4 * yh + r;
+            float val[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                val[i] = acc[r][i];
+                if constexpr (OUT_MODE == OUT_GATE) val[i] *= g[r][i];
+                if constexpr (OUT_MODE == OUT_UV) val[i] += g[r][i] * __shfl(acc[r][i], lane + 1, 64);
+            }
+            const bool mine = OUT_MODE == OUT_UV ? co == 0 : co < COUT;
+            if (!mine || gy >= a.ny || gz >= a.nz) continue;
+            float* o = out + (int64_t)b * a.out_bs + (OUT_MODE == OUT_UV ? 0 : co) * a.ng + gx +
+                       (int64_t)a.nx * (gy + (int64_t)a.ny * gz);
+            if ((a.nx & 3) == 0) {
+                if (gx < a.nx) *reinterpret_cast<f32x4_t*>(o) = f32x4_t{val[0], val[1], val[2], val[3]};
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (gx + i < a.nx) o[i] = val[i];
             }
         }
     }
@@ -545,6 +725,47 @@ static void net_adjoint_mfma(qg_cnn* c, const Weights& W, int nb, const float* y
     QG_HIP(hipGetLastError());
 }
 
+// One layer of the inference network: out = post(conv(in)) for nb bands, FP32 activations,
+// BF16-valued weights.
+template <int CIN, int COUT, int IN_MODE, int OUT_MODE>
+static void launch_split(const ConvArgs& a, int nb, const float* w, const float* in, float* out, hipStream_t s) {
+    const int tx = (a.nx + kSX - 1) / kSX, ty = (a.ny + kSY - 1) / kSY, tz = (a.nz + kSZ - 1) / kSZ;
+    const int64_t ntile = (int64_t)tx * ty * tz;
+    // bands per workgroup: up to 8 (weights and gates are set up once for them) while ~2048
+    // workgroups remain
+    const int bl = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(8, nb), ntile * nb / 2048));
+    const int64_t nwg = ntile * ((nb + bl - 1) / bl);
+    QG_REQUIRE(nwg < (1LL << 31) && a.ng < (1LL << 31), "too many convolution tiles");
+    hipLaunchKernelGGL((conv3_split_kernel<CIN, COUT, IN_MODE, OUT_MODE>), dim3((unsigned)nwg), dim3(kSThreads), 0, s, a,
+                       nb, bl, tx, ty, (int)ntile, w, in, out);
+    QG_HIP(hipGetLastError());
+}
+
+// w = N u and q = N^T y with the inference weights (FP32 activations), scratch s8a/s8b
+static void net_forward_split(qg_cnn* c, const Weights& W, int nb, const float* u, float* w, float* s8a, float* s8b,
+                              hipStream_t s) {
+    const int64_t ng = c->h->grid.ng();
+    ConvArgs a = conv_args(c);
+    a.in_bs = ng; a.out_bs = kC * ng; a.ga = W.a1; a.gb = W.b1;
+    launch_split<2, kC, IN_UV, OUT_GATE>(a, nb, W.w1, u, s8a, s);
+    a.in_bs = kC * ng; a.ga = W.a2; a.gb = W.b2;
+    launch_split<kC, kC, IN_PLAIN, OUT_GATE>(a, nb, W.w2, s8a, s8b, s);
+    a.out_bs = ng;
+    launch_split<kC, 1, IN_PLAIN, OUT_PLAIN>(a, nb, W.w3, s8b, w, s);
+}
+
+static void net_adjoint_split(qg_cnn* c, const Weights& W, int nb, const float* y, float* q, float* s8a, float* s8b,
+                              hipStream_t s) {
+    const int64_t ng = c->h->grid.ng();
+    ConvArgs a = conv_args(c);
+    a.in_bs = ng; a.out_bs = kC * ng; a.ga = W.a2; a.gb = W.b2;
+    launch_split<1, kC, IN_PLAIN, OUT_GATE>(a, nb, W.t3, y, s8a, s);
+    a.in_bs = kC * ng; a.ga = W.a1; a.gb = W.b1;
+    launch_split<kC, kC, IN_PLAIN, OUT_GATE>(a, nb, W.t2, s8a, s8b, s);
+    a.out_bs = ng;
+    launch_split<kC, 2, IN_PLAIN, OUT_UV>(a, nb, W.t1, s8b, q, s);
+}
+
 // q = N^T y; when dh2/dh1 are given, the pre-gate adjoint activations are stored there and the
 // post-gate ones in da2/da1 (else scratch)
 static void net_adjoint(qg_cnn* c, const Weights& W, int nb, const float* y, float* q, float* da2, float* da1,
@@ -674,32 +895,38 @@ void cnn_precond_apply(qg_cnn* c, int dtype, int nbands, void* r, int64_t ld, hi
     QG_REQUIRE(ld == ng, "learned preconditioner expects ld == Ng");
     refresh_derived(c, s);
     const Weights W = weights(c, true);
-    // per band: u (1), two 8-channel sets, w (1), y (1)
-    const int64_t per = (2 * kC + 3) * ng;
-    const int chunk = (int)std::max<int64_t>(1, std::min<int64_t>(nbands, (1ll << 30) / (per * 4)));
-    c->ws.alloc((size_t)chunk * per);
-    float* u = c->ws.p;
-    float* s8a = u + (int64_t)chunk * ng;
-    float* s8b = s8a + (int64_t)chunk * kC * ng;
-    float* w = s8b + (int64_t)chunk * kC * ng;
-    float* y = w + (int64_t)chunk * ng;
+    // per band: y and, for an FP64 block, u as FP32 (at most 1 GiB of bands at a time); the two
+    // 8-channel sets and w likewise (80^3, 32 bands: 3.2 ms an application so, 4.1 and 5.6 ms in
+    // pieces of 256 and 128 MB that the Infinity Cache would hold: the launches get too small)
+    const int per1 = dtype == QG_F32 ? 1 : 2;
+    const int chunk = (int)std::max<int64_t>(1, std::min<int64_t>(nbands, (1ll << 30) / (per1 * ng * 4)));
+    const int sub = (int)std::max<int64_t>(1, std::min<int64_t>(chunk, (1ll << 30) / ((2 * kC + 1) * ng * 4)));
+    c->ws.alloc((size_t)chunk * per1 * ng + (size_t)sub * (2 * kC + 1) * ng);
+    float* y = c->ws.p;
+    float* u64 = y + (int64_t)chunk * ng;
+    float* s8a = y + (int64_t)chunk * per1 * ng;
+    float* s8b = s8a + (int64_t)sub * kC * ng;
+    float* w = s8b + (int64_t)sub * kC * ng;
     // u = K r in place
     precond_apply(c->h, QG_PRECOND_KINETIC, c->shift, dtype, nbands, r, ld, s);
     for (int b0 = 0; b0 < nbands; b0 += chunk) {
         const int nb = std::min(chunk, nbands - b0);
         const int64_t n = (int64_t)nb * ng;
-        if (dtype == QG_F32) {
-            QG_HIP(hipMemcpyAsync(u, (float*)r + (int64_t)b0 * ng, n * 4, hipMemcpyDeviceToDevice, s));
-        } else {
+        const float* u = (const float*)r + (int64_t)b0 * ng;
+        if (dtype != QG_F32) {
+            u = u64;
             hipLaunchKernelGGL((cnn_convert_kernel<double, float>), dim3(grid1(n)), dim3(256), 0, s,
-                               (const double*)r + (int64_t)b0 * ng, u, n, 1.0);
+                               (const double*)r + (int64_t)b0 * ng, u64, n, 1.0);
         }
-        if (c->mfma) {
-            net_forward_mfma(c, W, nb, u, w, s8a, s8b, s);
-            net_adjoint_mfma(c, W, nb, w, y, s8a, s8b, s);
-        } else {
-            net_forward(c, W, nb, u, w, nullptr, s8a, s8b, s);
-            net_adjoint(c, W, nb, w, y, s8a, s8b, nullptr, nullptr, s);
+        for (int c0 = 0; c0 < nb; c0 += sub) {
+            const int cn = std::min(sub, nb - c0);
+            if (c->mfma) {
+                net_forward_mfma(c, W, cn, u + (int64_t)c0 * ng, w, s8a, s8b, s);
+                net_adjoint_mfma(c, W, cn, w, y + (int64_t)c0 * ng, s8a, s8b, s);
+            } else {
+                net_forward_split(c, W, cn, u + (int64_t)c0 * ng, w, s8a, s8b, s);
+                net_adjoint_split(c, W, cn, w, y + (int64_t)c0 * ng, s8a, s8b, s);
+            }
         }
         precond_apply(c->h, QG_PRECOND_KINETIC, c->shift, QG_F32, nb, y, ng, s);
         if (dtype == QG_F32)
