@@ -132,6 +132,20 @@ void check_rc(int rc) {
     if (rc != QG_OK) throw Error{rc, std::string(qg_last_error())};
 }
 
+// out[b] = w_b sum_j E_j c_bj^2 of band b's coefficients, one wavefront per band
+__global__ __launch_bounds__(64) void band_energy_kernel(const double* __restrict__ c, const double* __restrict__ energy,
+                                                         int ncoef, const double* __restrict__ w, double scale,
+                                                         double* __restrict__ out) {
+    const int b = blockIdx.x;
+    double e = 0.0;
+    for (int j = threadIdx.x; j < ncoef; j += 64) {
+        const double v = c[(int64_t)b * ncoef + j];
+        e += v * v * energy[j];
+    }
+    for (int s = 32; s >= 1; s >>= 1) e += __shfl_xor(e, s, 64);
+    if (threadIdx.x == 0) out[b] = scale * w[b] * e;
+}
+
 void gradient8(const qg_grid& g, int dtype, int nbands, const void* psi, int64_t ld, void* gx, void* gy, void* gz,
                int64_t ld_out, double coef, hipStream_t s) {
     const double cx = coef / (840.0 * g.h[0]), cy = coef / (840.0 * g.h[1]), cz = coef / (840.0 * g.h[2]);
@@ -193,6 +207,52 @@ int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void*
         const qg_grid& g = nl->gcopy;
         const int64_t ng = g.ng();
         const size_t es = dtype == QG_F32 ? 4 : 8;
+        if (sphere_nonlocal_force(nl, dtype, 1, nullptr, nullptr, psi, ld, nullptr, nl->force_part, nullptr,
+                                                 false, s)) {
+            // the occupied states: their projections (in runs of consecutive bands), then forces
+            // and energies on the device
+            std::vector<int> occupied;
+            std::vector<double> host;
+            for (int b = 0; b < nbands; ++b)
+                if (occ_host[b] > 0.0) {
+                    occupied.push_back(b);
+                    host.push_back(-2.0 * occ_host[b]);
+                }
+            const int nocc = (int)occupied.size();
+            if (nocc == 0) {
+                if (energy) *energy = 0.0;
+                return;
+            }
+            // coefficients [nocc][ncoef], weights [nocc], then energies [nocc] and forces [natoms][3]
+            const size_t out_off = (size_t)nocc * ncoef + nocc;
+            const size_t nout = (size_t)nocc + (forces_host ? 3 * natoms : 0);
+            nl->force_coef.alloc(out_off + nout);
+            nl->force_idx.alloc(nocc);
+            double* c = nl->force_coef.p;
+            double* w = c + (size_t)nocc * ncoef;
+            double* res = c + out_off;
+            QG_HIP(hipMemcpyAsync(w, host.data(), nocc * sizeof(double), hipMemcpyHostToDevice, s));
+            QG_HIP(hipMemcpyAsync(nl->force_idx.p, occupied.data(), nocc * sizeof(int), hipMemcpyHostToDevice, s));
+            for (int k0 = 0; k0 < nocc;) {
+                int k1 = k0 + 1;
+                while (k1 < nocc && k1 - k0 < kMaxRun && occupied[k1] == occupied[k1 - 1] + 1) ++k1;
+                check_rc(qg_nonlocal_project(nl, dtype, k1 - k0, (const unsigned char*)psi + (size_t)occupied[k0] * ld * es,
+                                             ld, c + (size_t)k0 * ncoef, s));
+                k0 = k1;
+            }
+            if (forces_host)
+                (void)sphere_nonlocal_force(nl, dtype, nocc, nl->force_idx.p, w, psi, ld, c, nl->force_part, res + nocc,
+                                            true, s);
+            hipLaunchKernelGGL(band_energy_kernel, dim3(nocc), dim3(64), 0, s, c, nl->d_coef_energy.p, ncoef, w, -0.5, res);
+            QG_HIP(hipGetLastError());
+            host.resize(nout);
+            QG_HIP(hipMemcpyAsync(host.data(), res, nout * sizeof(double), hipMemcpyDeviceToHost, s));
+            QG_HIP(hipStreamSynchronize(s));
+            for (int k = 0; k < nocc; ++k) ev += host[k];
+            if (forces_host) std::copy(host.begin() + nocc, host.end(), forces_host);
+            if (energy) *energy = ev;
+            return;
+        }
         // bands per run: the three gradient blocks of a run take at most kGradBytes
         const int64_t per_band = 3 * ng * (int64_t)es;
         const int chunk = (int)std::max<int64_t>(

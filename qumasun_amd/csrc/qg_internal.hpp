@@ -221,6 +221,8 @@ struct SphereGeo {
     int ntrips = 1;
     bool ok = false;
     DevBuf<int> d_col_off, d_col_img, d_trip_off;
+    DevBuf<int> d_atom_ref_off;    // per atom: its (tile, column image) pairs
+    DevBuf<int2> d_atom_ref;
     DevBuf<uint32_t> d_words;
     DevBuf<unsigned char> d_vals;
 };
@@ -288,6 +290,8 @@ struct qg_nonlocal {
     // qg_nonlocal_energy_force: gradient blocks of a band run and their coefficients
     qg::DevBuf<unsigned char> force_grad;
     qg::DevBuf<double> force_coef;
+    qg::DevBuf<double> force_part;   // partial forces of the sphere force pass
+    qg::DevBuf<int> force_idx;       // occupied bands
 };
 
 namespace qg {
@@ -307,6 +311,9 @@ void sphere_prepare(qg_nonlocal* nl);
 bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
                               int64_t ld_out, const double* coef, bool may_build, bool run, hipStream_t s);
 bool sphere_prepared(qg_nonlocal* nl, int dtype);
+bool sphere_nonlocal_force(qg_nonlocal* nl, int dtype, int nocc, const int* band_idx, const double* weight,
+                           const void* psi, int64_t ld, const double* coef, DevBuf<double>& part, double* force,
+                           bool run, hipStream_t s);
 size_t lds_limit();
 double* scratch_address();
 void rows_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi, int64_t ld_out,

@@ -118,20 +118,31 @@ struct SphereArgs {
     int ncoef;
     int max_col;
     double h[3];
+    // force pass: the occupied bands and their weights -2 occ; per workgroup and column image the
+    // partial force (part[((tile * nslab + slab) * bandgroups + bandgroup) * max_col + image][3])
+    const int* band_idx;
+    const double* weight;
+    double* part;
 };
 
-// LDS bytes of an apply workgroup
+// LDS bytes of an apply workgroup; of a force workgroup with nw wavefronts (0: apply)
 template <class T>
-static size_t sphere_lds(int nx, int ty, int nb, int ns, int np, int max_col) {
+static size_t sphere_lds(int nx, int ty, int nb, int ns, int np, int max_col, int nw = 0) {
     constexpr int VN = 16 / sizeof(T);
     const size_t W = (size_t)(nx + 8 + VN - 1) / VN * VN;
-    return sizeof(T) * (2 * (size_t)nb * (ty + 8) * W + (size_t)(max_col + 1) * (4 + nb * (ns + 3 * np)));
+    const size_t b = sizeof(T) * (2 * (size_t)nb * (ty + 8) * W + (size_t)(max_col + 1) * (4 + nb * (ns + 3 * np)));
+    return (b + 15) / 16 * 16 + sizeof(double) * 3 * (size_t)nw * (max_col + 1);
 }
 
 // One workgroup of the apply pass.  NB bands; NS s and NP p channels per image; RAG: Nx is not a
 // multiple of VN (the last group of a row then overlaps its neighbour: both owners compute and
 // write the same values, and LDS is accessed by element); HV halo vectors per thread and band.
-template <class T, int NB, int NS, int NP, bool RAG, int HV>
+//
+// FORCE: instead of H psi, the nonlocal forces F_a = sum_b (-2 occ_b) sum_i v_ba(i) D psi_b(i), with
+// v_ba = sum_j E_j c_baj beta_aj the value an entry contributes to V_NL psi and D the 8th-order
+// gradient: an entry's three sums stay with its lane while consecutive planes list the same image,
+// then go to the wavefront's own LDS sums.
+template <class T, int NB, int NS, int NP, bool RAG, int HV, bool FORCE = false>
 __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>& sc, const T* __restrict__ V,
                                             const T* __restrict__ psi, T* __restrict__ out, const int wg,
                                             unsigned char* smem) {
@@ -147,6 +158,9 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
     T* planes = reinterpret_cast<T*>(smem);                    // [2][NB][ty + 8][W]
     T* imf = planes + (size_t)2 * NB * lband;                  // [max_col + 1][4]: f.x f.y f.z, n.z
     T* ec = imf + (size_t)(a.max_col + 1) * 4;                 // [max_col + 1][NB][NC]
+    // force pass: [wavefront][max_col + 1][3] sums
+    const size_t foff = (sizeof(T) * (2 * (size_t)NB * lband + (size_t)(a.max_col + 1) * (4 + NB * NC)) + 15) / 16 * 16;
+    double* facc = reinterpret_cast<double*>(smem + foff);
 
     // order: tiles of a group of tg, then bands, then slabs, then groups
     const int nbg = (a.nbands + NB - 1) / NB;
@@ -173,11 +187,12 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         // bands past the block read the last one and store nothing
-        const int band = min(b0 + b, a.nbands - 1);
+        int band = min(b0 + b, a.nbands - 1);
+        if constexpr (FORCE) band = __builtin_amdgcn_readfirstlane(a.band_idx[band]);
         rin[b] = rsrc(psi + (int64_t)band * a.ld_in, band_bytes);
-        rout[b] = rsrc(out + (int64_t)band * a.ld_out, b0 + b < a.nbands ? band_bytes : 0u);
+        if constexpr (!FORCE) rout[b] = rsrc(out + (int64_t)band * a.ld_out, b0 + b < a.nbands ? band_bytes : 0u);
     }
-    const rsrc_t rv = rsrc(V, band_bytes);
+    const rsrc_t rv = rsrc(V, FORCE ? 0u : band_bytes);
     const int vo = own ? ((y0 + r) * nx + x) * S : kOOB;
     const int lc = (r + 4) * W + 4 + x;
     const int lw = (x < 4) ? lc + nx : ((x >= nx - 4) ? lc - nx : -1);   // wrapped copy (whole vectors)
@@ -220,11 +235,15 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
             const int slot = a.atom_chan[4 * at + ch];
             if (slot >= 0) {
                 const int cb = a.atom_coef_off[at] + slot + (j < NS ? 0 : (j - NS) % 3);
-                v = (T)(a.coef_energy[cb] * a.coef[(int64_t)(b0 + b) * a.ncoef + cb]);
+                double e = a.coef_energy[cb] * a.coef[(int64_t)(b0 + b) * a.ncoef + cb];
+                if constexpr (FORCE) e *= a.weight[b0 + b];
+                v = (T)e;
             }
         }
         ec[i] = v;
     }
+    if constexpr (FORCE)
+        for (int i = tid; i < 3 * a.nw * (a.max_col + 1); i += nthr) facc[i] = 0.0;
 
     // z-queue: step k of three planes holds the planes z - 4 .. z + 4 in q[k] .. q[k + 8] and
     // loads z + 5 into q[k + 9] (step 2: into the free q[0]); the queue moves once per three planes
@@ -235,7 +254,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
         for (int d = 0; d < 8; ++d) q[b][d] = vload<T>(rin[b], vo, zoff(z0 - 4 + d));
     Row<T> hn[NB][HV], vn;
     auto load_halo = [&](int z) {
-        vn = vload<T>(rv, vo, zoff(z));
+        if constexpr (!FORCE) vn = vload<T>(rv, vo, zoff(z));
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -272,6 +291,19 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
         for (int k = 0; k < K; ++k) en[k] = load_entry(rvals, rwords, k);
     };
     load_entries(z0);
+    // force pass: the image whose sums each of the first K trips holds
+    double fa[K][3];
+    int cur[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        cur[k] = ncol;
+        fa[k][0] = fa[k][1] = fa[k][2] = 0.0;
+    }
+    auto flush = [&](int li, const double (&f)[3]) {
+        double* d = facc + 3 * ((size_t)wave * (a.max_col + 1) + li);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) __hip_atomic_fetch_add(d + k, f[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
 
     auto step = [&](auto kc, int z) {
         constexpr int k0 = decltype(kc)::value;
@@ -312,17 +344,22 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
         load_halo(zn);
         __syncthreads();
 
-        Row<T> res[NB];
+        Row<T> res[NB], gx[NB], gz[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             // V psi and the stencil: centre and z from the register queue, x and y from LDS
-            const T* Lc = Lp + b * lband + (own ? (r + 4) * W + x : 0);   // Lc[4 + i] is point x + i
-            T d[VN];
+            const T* Lc = Lp + b * lband + (own ? (r + 4) * W + x : 4 * W);   // Lc[4 + i] is point x + i
+            T d[VN], e[VN];
             const Row<T>* qb = q[b] + k0;
 #pragma unroll
             for (int i = 0; i < VN; ++i) {
-                d[i] = sc.c0 * qb[4].v[i];
-                d[i] += sc.cz[3] * (qb[8].v[i] + qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] + qb[1].v[i]) +
+                // force pass: d, e and res are the z, x and y derivatives (weights in sc)
+                if constexpr (FORCE)
+                    d[i] = sc.cz[3] * (qb[8].v[i] - qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] - qb[1].v[i]) +
+                           sc.cz[1] * (qb[6].v[i] - qb[2].v[i]) + sc.cz[0] * (qb[5].v[i] - qb[3].v[i]);
+                else
+                    d[i] = sc.c0 * qb[4].v[i];
+                if constexpr (!FORCE) d[i] += sc.cz[3] * (qb[8].v[i] + qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] + qb[1].v[i]) +
                         sc.cz[1] * (qb[6].v[i] + qb[2].v[i]) + sc.cz[0] * (qb[5].v[i] + qb[3].v[i]);
             }
             {
@@ -339,10 +376,16 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                     for (int k = 0; k < VN + 8; ++k) xsv[k] = Lc[k];
                 }
 #pragma unroll
-                for (int i = 0; i < VN; ++i)
-                    d[i] += sc.cx[3] * (xsv[i + 8] + xsv[i]) + sc.cx[2] * (xsv[i + 7] + xsv[i + 1]) +
-                            sc.cx[1] * (xsv[i + 6] + xsv[i + 2]) + sc.cx[0] * (xsv[i + 5] + xsv[i + 3]);
+                for (int i = 0; i < VN; ++i) {
+                    if constexpr (FORCE)
+                        e[i] = sc.cx[3] * (xsv[i + 8] - xsv[i]) + sc.cx[2] * (xsv[i + 7] - xsv[i + 1]) +
+                               sc.cx[1] * (xsv[i + 6] - xsv[i + 2]) + sc.cx[0] * (xsv[i + 5] - xsv[i + 3]);
+                    else
+                        d[i] += sc.cx[3] * (xsv[i + 8] + xsv[i]) + sc.cx[2] * (xsv[i + 7] + xsv[i + 1]) +
+                                sc.cx[1] * (xsv[i + 6] + xsv[i + 2]) + sc.cx[0] * (xsv[i + 5] + xsv[i + 3]);
+                }
             }
+            if constexpr (FORCE) res[b] = Row<T>{};
 #pragma unroll
             for (int m = 3; m >= 0; --m) {
                 Row<T> ym, yp;
@@ -357,17 +400,31 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                     }
                 }
 #pragma unroll
-                for (int i = 0; i < VN; ++i) d[i] += sc.cy[m] * (yp.v[i] + ym.v[i]);
+                for (int i = 0; i < VN; ++i) {
+                    if constexpr (FORCE) res[b].v[i] += sc.cy[m] * (yp.v[i] - ym.v[i]);
+                    else d[i] += sc.cy[m] * (yp.v[i] + ym.v[i]);
+                }
             }
 #pragma unroll
-            for (int i = 0; i < VN; ++i) res[b].v[i] = vcur.v[i] * qb[4].v[i] + d[i];
+            for (int i = 0; i < VN; ++i) {
+                if constexpr (FORCE) {
+                    // a point of two overlapping groups counts once
+                    const bool mine = !RAG || x + i >= xq * VN;
+                    gx[b].v[i] = mine ? e[i] : T(0);
+                    gz[b].v[i] = mine ? d[i] : T(0);
+                    if (!mine) res[b].v[i] = T(0);
+                } else {
+                    res[b].v[i] = vcur.v[i] * qb[4].v[i] + d[i];
+                }
+            }
             // one band's LDS values live at a time
             __builtin_amdgcn_sched_barrier(0);
         }
 
         // projector term: one trip per list entry, the same number for all lanes of the wavefront
         // (an entry's channels are summed before they meet the larger stencil value)
-        auto trip = [&](const Entry& e) {
+        auto trip = [&](const Entry& e, int slot) {
+            double f[3] = {0.0, 0.0, 0.0};
             const int li = (int)(e.w & 1023u);
             const int dyi = ((int)(e.w << 11)) >> 21, dxi = ((int)e.w) >> 21;
             const T* im = imf + 4 * li;
@@ -405,19 +462,41 @@ T val[VN];
                     for (int u = 0; u < VN; ++u) val[u] += e.f[NS + p].v[u] * (ayz + cx * (dx0 + (T)u * hx));
                 }
 #pragma unroll
-                for (int u = 0; u < VN; ++u) res[b].v[u] += val[u];
+                for (int u = 0; u < VN; ++u) {
+                    if constexpr (FORCE) {
+                        f[0] += (double)val[u] * (double)gx[b].v[u];
+                        f[1] += (double)val[u] * (double)res[b].v[u];
+                        f[2] += (double)val[u] * (double)gz[b].v[u];
+                    } else {
+                        res[b].v[u] += val[u];
+                    }
+                }
+            }
+            if constexpr (FORCE) {
+                if (slot < 0) {
+                    flush(li, f);
+                } else {
+                    if (li != cur[slot]) {
+                        flush(cur[slot], fa[slot]);
+                        cur[slot] = li;
+                        fa[slot][0] = fa[slot][1] = fa[slot][2] = 0.0;
+                    }
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) fa[slot][k] += f[k];
+                }
             }
         };
 #pragma unroll
         for (int k = 0; k < K; ++k)
-            if (k < n) trip(en[k]);
+            if (k < n) trip(en[k], k);
         if (n > K) {
             const rsrc_t rvals = rsrc((const unsigned char*)a.vals + (int64_t)tb * NV * 1024, (uint32_t)n * NV * 1024);
             const rsrc_t rwords = rsrc(a.words + (int64_t)tb * 64, (uint32_t)n * 256);
-            for (int k = K; k < n; ++k) trip(load_entry(rvals, rwords, k));
+            for (int k = K; k < n; ++k) trip(load_entry(rvals, rwords, k), -1);
         }
         load_entries(zn);
         // lanes without a point store out of range (dropped)
+        if constexpr (!FORCE)
 #pragma unroll
         for (int b = 0; b < NB; ++b) vstore<T>(rout[b], res[b], vo, zoff(z));
     };
@@ -436,6 +515,17 @@ T val[VN];
             q[b][8] = next;
         }
     }
+    if constexpr (FORCE) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) flush(cur[k], fa[k]);
+        __syncthreads();
+        double* part = a.part + (((size_t)tile * a.nslab + slab) * nbg + b0 / NB) * a.max_col * 3;
+        for (int i = tid; i < 3 * ncol; i += nthr) {
+            double s = 0.0;
+            for (int w = 0; w < a.nw; ++w) s += facc[(size_t)3 * w * (a.max_col + 1) + i];
+            part[i] = s;
+        }
+    }
 }
 
 template <class T, int NB, int NS, int NP, bool RAG, int HV>
@@ -443,6 +533,41 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_hpsi_kernel(SphereArgs a, 
                                                                   const T* __restrict__ psi, T* __restrict__ out) {
     extern __shared__ __align__(16) unsigned char smem[];
     sphere_body<T, NB, NS, NP, RAG, HV>(a, sc, V, psi, out, xcd_order(blockIdx.x, gridDim.x), smem);
+}
+
+// The nonlocal force pass: psi is read once (the chain of gradient blocks and their projections
+// moved psi eight times: 64 atoms, 80^3, 137 occupied FP64 bands 1.45 ms after the projection of
+// psi, 0.53 ms here).
+template <class T, int NB, int NS, int NP, bool RAG, int HV>
+__global__ __launch_bounds__(kMaxThreads) void sphere_force_kernel(SphereArgs a, Coef8<T> sc, const T* __restrict__ psi) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    sphere_body<T, NB, NS, NP, RAG, HV, true>(a, sc, nullptr, psi, nullptr, xcd_order(blockIdx.x, gridDim.x), smem);
+}
+
+// force[atom][3]: the atom's partials, over its (tile, column image) pairs and their workgroups in
+// a fixed order
+__global__ __launch_bounds__(256) void sphere_force_reduce_kernel(const double* __restrict__ part,
+                                                                  const int* __restrict__ atom_ref_off,
+                                                                  const int2* __restrict__ atom_ref, int per_tile,
+                                                                  int max_col, double* __restrict__ force) {
+    __shared__ double red[4][3];
+    const int at = blockIdx.x;
+    double f[3] = {0.0, 0.0, 0.0};
+    for (int k = atom_ref_off[at]; k < atom_ref_off[at + 1]; ++k) {
+        const int2 ref = atom_ref[k];
+        for (int w = threadIdx.x; w < per_tile; w += 256) {
+            const double* p = part + (((size_t)ref.x * per_tile + w) * max_col + ref.y) * 3;
+            for (int d = 0; d < 3; ++d) f[d] += p[d];
+        }
+    }
+    for (int d = 0; d < 3; ++d) {
+        for (int s = 32; s >= 1; s >>= 1) f[d] += __shfl_xor(f[d], s, 64);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][d] = f[d];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3)
+        force[3 * at + threadIdx.x] =
+            red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
 }
 
 // ------------------------------------------------------------------ entry lists ----
@@ -697,8 +822,21 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
         off.push_back((int)img.size());
         c->max_col = std::max(c->max_col, (int)v.size());
     }
+    // (tile, column image) pairs of every atom
+    std::vector<std::vector<int2>> refs(nl->geo.natoms);
+    for (int t = 0; t < c->ntile; ++t)
+        for (int k = 0; k < (int)col[t].size(); ++k) refs[nl->sphere_img[col[t][k]].atom].push_back(make_int2(t, k));
+    std::vector<int> ref_off(1, 0);
+    std::vector<int2> ref;
+    for (auto& v : refs) {
+        ref.insert(ref.end(), v.begin(), v.end());
+        ref_off.push_back((int)ref.size());
+    }
+    if (ref.empty()) ref.push_back(make_int2(0, 0));
     if (img.empty()) img.push_back(0);
     if (c->max_col < 1023) {
+        c->d_atom_ref_off.upload(ref_off.data(), ref_off.size());
+        c->d_atom_ref.upload(ref.data(), ref.size());
         c->d_col_off.upload(off.data(), off.size());
         c->d_col_img.upload(img.data(), img.size());
         BuildArgs a{};
@@ -811,6 +949,125 @@ bool sphere_prepared(qg_nonlocal* nl, int dtype) {
            (dtype == QG_F32 ? sphere_lds_of<float>(nl, *sg, 1) : sphere_lds_of<double>(nl, *sg, 1)) <= lds_limit();
 }
 
+// Arguments of a launch over nbands bands, nb per workgroup, except the blocks and coefficients;
+// want_tz: planes per slab (0: automatic)
+static SphereArgs sphere_args(const qg_nonlocal* nl, const SphereGeo& sg, int nbands, int nb, int want_tz) {
+    const qg_grid& g = nl->gcopy;
+    SphereArgs a{};
+    a.nx = g.n[0]; a.ny = g.n[1]; a.nz = g.n[2];
+    a.ty = sg.ty;
+    a.ntile = sg.ntile;
+    // two neighbouring tiles, then all bands: the workgroups an XCD runs together share the
+    // entry lists and V in its L2 (per application of 512 FP32 bands at 120^3 the pass reads
+    // 8.0 GB so, 10.2 GB with 4 tiles, more with all)
+    a.tg = std::min(sg.ntile, 2);
+    a.nq = sg.nq; a.tpb = sg.tpb; a.nw = sg.tpb / 64;
+    // z-slabs for about 2048 workgroups, of at least 8 planes (a slab re-reads 8), or of 3 where
+    // the workgroups are too few to fill the chip: then a workgroup's chain of planes is the time
+    // (24^3, 8 bands: 12.9 us in slabs of 8, 8.8 of 3; 40^3, 16 FP32 bands: 14.8 us of 8, 11.8 of 4)
+    const int64_t wg = (int64_t)a.ntile * ((nbands + nb - 1) / nb);
+    const int least = wg * std::max(1, g.n[2] / 8) < 512 ? 3 : 8;
+    const int nslab = (int)std::max<int64_t>(1, std::min<int64_t>((2048 + wg - 1) / wg, std::max(1, g.n[2] / least)));
+    a.tz = want_tz > 0 ? std::min(g.n[2], want_tz) : (g.n[2] + nslab - 1) / nslab;
+    a.nslab = (g.n[2] + a.tz - 1) / a.tz;
+    a.nbands = nbands;
+    a.col_off = sg.d_col_off.p; a.col_img = sg.d_col_img.p;
+    a.images = nl->d_sphere_img.p;
+    a.trip_off = sg.d_trip_off.p;
+    a.ntrips = sg.ntrips;
+    a.vals = sg.d_vals.p; a.words = sg.d_words.p;
+    a.coef_energy = nl->d_coef_energy.p; a.atom_coef_off = nl->d_atom_coef_off.p;
+    a.atom_chan = nl->d_atom_chan.p;
+    a.ncoef = nl->geo.ncoef;
+    a.max_col = sg.max_col;
+    for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
+    return a;
+}
+
+// Two bands per workgroup (an entry is loaded once for both) where that leaves two workgroups per CU
+static int sphere_pick_nb(const SphereGeo& sg, int nbands) {
+    return (int64_t)sg.ntile * ((nbands + 1) / 2) >= 512 ? 2 : 1;
+}
+
+template <class T, int NB, int NS, int NP>
+static void sphere_force_launch(const SphereArgs& a, const Coef8<T>& sc, const T* psi, size_t lds, hipStream_t s) {
+    const int64_t nwg = (int64_t)a.ntile * a.nslab * ((a.nbands + NB - 1) / NB);
+    QG_REQUIRE(nwg < (1LL << 31), "too many workgroups");
+    const dim3 grid((unsigned)nwg), blk(a.tpb);
+    const bool rag = a.nx % (16 / (int)sizeof(T)) != 0;
+    const int hv = sphere_halo_vectors(a.nq, a.tpb);
+    QG_REQUIRE(hv <= (NB == 1 ? 8 : 1), "row tile too low for its halo");
+    if (hv <= 1) {
+        if (rag) hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, true, 1>), grid, blk, lds, s, a, sc, psi);
+        else hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, false, 1>), grid, blk, lds, s, a, sc, psi);
+    } else if constexpr (NB == 1) {
+        if (rag) hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, true, 8>), grid, blk, lds, s, a, sc, psi);
+        else hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, false, 8>), grid, blk, lds, s, a, sc, psi);
+    }
+    QG_HIP(hipGetLastError());
+}
+
+template <class T>
+static bool sphere_force_t(qg_nonlocal* nl, int nocc, const int* band_idx, const double* weight, const T* psi, int64_t ld,
+                           const double* coef, DevBuf<double>& part, double* force, bool run, hipStream_t s) {
+    const qg_grid& g = nl->gcopy;
+    constexpr int VN = 16 / sizeof(T);
+    const int dtype = sizeof(T) == 4 ? QG_F32 : QG_F64;
+    const int nq = (g.n[0] + VN - 1) / VN;
+    const int ty = sphere_pick_ty(nq, g.n[1], 0);
+    const SphereGeo* sg = ty > 0 ? sphere_geometry(nl, dtype, ty, true) : nullptr;
+    if (!sg || !sg->ok || sphere_halo_vectors(nq, sg->tpb) > 8) return false;
+    const int nw = sg->tpb / 64;
+    auto lds_of = [&](int b) {
+        return sphere_lds<T>(g.n[0], ty, b, nl->sphere_form.ns, nl->sphere_form.np, sg->max_col, nw);
+    };
+    // two bands share an entry, its running sums and their LDS updates (64 atoms, 80^3, 137 FP64
+    // bands: 0.83 ms a call against 1.0 with one); 2 + 2 channels of two bands would spill
+    int nb = nl->sphere_form.ns == 2 || (int64_t)sg->ntile * ((nocc + 1) / 2) < 256 ? 1 : 2;
+    if (nb > 1 && (sphere_halo_vectors(nq, sg->tpb) > 1 || lds_of(nb) > lds_limit())) nb = 1;
+    if (lds_of(nb) > lds_limit()) return false;
+    if (!run) return true;
+    SphereArgs a = sphere_args(nl, *sg, nocc, nb, 0);
+    a.ld_in = ld;
+    a.coef = coef;
+    a.band_idx = band_idx;
+    a.weight = weight;
+    const int per_tile = a.nslab * ((nocc + nb - 1) / nb);
+    part.alloc((size_t)a.ntile * per_tile * std::max(1, a.max_col) * 3);
+    a.part = part.p;
+    // 8th-order first-difference weights, dV of the projection's dot product in them
+    Coef8<T> sc{};
+    const double w[4] = {672.0, -168.0, 32.0, -3.0};
+    for (int m = 0; m < 4; ++m) {
+        sc.cx[m] = (T)(g.dvol() * w[m] / (840.0 * g.h[0]));
+        sc.cy[m] = (T)(g.dvol() * w[m] / (840.0 * g.h[1]));
+        sc.cz[m] = (T)(g.dvol() * w[m] / (840.0 * g.h[2]));
+    }
+    const size_t lds = lds_of(nb);
+    if (nl->sphere_form.ns == 2) {
+        sphere_force_launch<T, 1, 2, 2>(a, sc, psi, lds, s);
+    } else {
+        if (nb == 2) sphere_force_launch<T, 2, 1, 1>(a, sc, psi, lds, s);
+        else sphere_force_launch<T, 1, 1, 1>(a, sc, psi, lds, s);
+    }
+    hipLaunchKernelGGL(sphere_force_reduce_kernel, dim3(nl->geo.natoms), dim3(256), 0, s, a.part, sg->d_atom_ref_off.p,
+                       sg->d_atom_ref.p, per_tile, a.max_col, force);
+    QG_HIP(hipGetLastError());
+    return true;
+}
+
+// force[atom][3] (device) = sum_b weight_b sum_j E_j c_baj dV sum_i beta_aj D psi_b over the bands
+// band_idx[0 .. nocc) of psi (device arrays), coef their projections in that order.  False (nothing
+// launched) where the entry lists do not serve the grid or projector set; run false only says so.
+bool sphere_nonlocal_force(qg_nonlocal* nl, int dtype, int nocc, const int* band_idx, const double* weight,
+                           const void* psi, int64_t ld, const double* coef, DevBuf<double>& part, double* force,
+                           bool run, hipStream_t s) {
+    if (!sphere_serves(nl->gcopy, nl)) return false;
+    if (dtype == QG_F32)
+        return sphere_force_t<float>(nl, nocc, band_idx, weight, (const float*)psi, ld, coef, part, force, run, s);
+    return sphere_force_t<double>(nl, nocc, band_idx, weight, (const double*)psi, ld, coef, part, force, run, s);
+}
+
 template <class T>
 static bool sphere_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hpsi, int64_t ld_out,
                            const double* coef, bool may_build, bool run, hipStream_t s) {
@@ -829,43 +1086,14 @@ static bool sphere_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* h
     }
     if (!sg || !sg->ok) return false;
     const bool two = nl->sphere_form.ns == 2;
-    // two bands per workgroup (an entry is loaded once for both) where that leaves two
-    // workgroups per CU
-    int nb = h->plan.rows_bands > 0 ? std::min(2, h->plan.rows_bands)
-                                    : ((int64_t)sg->ntile * ((nbands + 1) / 2) >= 512 ? 2 : 1);
+    int nb = h->plan.rows_bands > 0 ? std::min(2, h->plan.rows_bands) : sphere_pick_nb(*sg, nbands);
     auto lds_of = [&](int b) { return sphere_lds_of<T>(nl, *sg, b); };
     if (nb > 1 && (sphere_halo_vectors(nq, sg->tpb) > 1 || lds_of(nb) > lds_limit())) nb = 1;
     if (lds_of(nb) > lds_limit() || sphere_halo_vectors(nq, sg->tpb) > 8) return false;
     if (!run) return true;
-    SphereArgs a{};
-    a.nx = g.n[0]; a.ny = g.n[1]; a.nz = g.n[2];
-    a.ty = ty;
-    a.ntile = sg->ntile;
-    // two neighbouring tiles, then all bands: the workgroups an XCD runs together share the
-    // entry lists and V in its L2 (per application of 512 FP32 bands at 120^3 the pass reads
-    // 8.0 GB so, 10.2 GB with 4 tiles, more with all)
-    a.tg = std::min(sg->ntile, 2);
-    a.nq = nq; a.tpb = sg->tpb; a.nw = sg->tpb / 64;
-    // z-slabs for about 2048 workgroups, of at least 8 planes (a slab re-reads 8), or of 3 where
-    // the workgroups are too few to fill the chip: then a workgroup's chain of planes is the time
-    // (24^3, 8 bands: 12.9 us in slabs of 8, 8.8 of 3; 40^3, 16 FP32 bands: 14.8 us of 8, 11.8 of 4)
-    const int64_t wg = (int64_t)a.ntile * ((nbands + nb - 1) / nb);
-    const int least = wg * std::max(1, g.n[2] / 8) < 512 ? 3 : 8;
-    const int nslab = (int)std::max<int64_t>(1, std::min<int64_t>((2048 + wg - 1) / wg, std::max(1, g.n[2] / least)));
-    a.tz = h->plan.rows_tz > 0 ? std::min(g.n[2], h->plan.rows_tz) : (g.n[2] + nslab - 1) / nslab;
-    a.nslab = (g.n[2] + a.tz - 1) / a.tz;
-    a.nbands = nbands;
+    SphereArgs a = sphere_args(nl, *sg, nbands, nb, h->plan.rows_tz);
     a.ld_in = ld; a.ld_out = ld_out;
-    a.col_off = sg->d_col_off.p; a.col_img = sg->d_col_img.p;
-    a.images = nl->d_sphere_img.p;
-    a.trip_off = sg->d_trip_off.p;
-    a.ntrips = sg->ntrips;
-    a.vals = sg->d_vals.p; a.words = sg->d_words.p;
-    a.coef = coef; a.coef_energy = nl->d_coef_energy.p; a.atom_coef_off = nl->d_atom_coef_off.p;
-    a.atom_chan = nl->d_atom_chan.p;
-    a.ncoef = nl->geo.ncoef;
-    a.max_col = sg->max_col;
-    for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
+    a.coef = coef;
     const T* V = sizeof(T) == 4 ? (const T*)(const void*)h->V32.p : (const T*)(const void*)h->V64.p;
     const Coef8<T> sc = coef8<T>(g, -0.5);
     const size_t lds = lds_of(nb);
