@@ -1062,7 +1062,9 @@ void hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_
         const size_t es = (dtype == QG_F32) ? 4 : 8;
         const char* pin = (const char*)psi + (size_t)b0 * ld * es;
         char* pout = (char*)hpsi + (size_t)b0 * ld_out * es;
-        if (nl) {
+        if (sphere && rows_nonlocal_project(nl, dtype, nb, pin, ld, nl->d_coef.p, h->rows_part, s)) {
+            // through the entry lists
+        } else if (nl) {
             if (dtype == QG_F64) launch_project<double>(nl, nb, (const double*)pin, ld, nl->d_coef.p, s);
             else launch_project<float>(nl, nb, (const float*)pin, ld, nl->d_coef.p, s);
         }

@@ -200,6 +200,7 @@ bool build_rows_geometry(const qg_grid& g, const NlGeometry& geo, int ty, int tz
 // apply kernels see it: centre = n + f in grid points (n integer, shift included).
 struct SphereImage {
     int n[3];
+    int shift[3];        // grid-index shift (multiples of N)
     int atom;
     int b[3], e[3];      // in-grid range [b, e)
     int nparts;
@@ -225,7 +226,14 @@ struct SphereGeo {
     DevBuf<int2> d_atom_ref;
     DevBuf<uint32_t> d_words;
     DevBuf<unsigned char> d_vals;
+    // the projection's lists: slots per (tile, epoch, wavefront)
+    bool slots_ok = false;
+    DevBuf<int> d_slot_off;
+    DevBuf<uint32_t> d_slot_mask, d_slot_words;
+    DevBuf<unsigned char> d_slot_vals;
 };
+// planes of one epoch of the projection's lists
+constexpr int kProjPlanes = 8;
 
 // Caller-provided FP64 scratch of one application (projector partials, then coefficients).
 struct RowsScratch {
@@ -311,6 +319,9 @@ void sphere_prepare(qg_nonlocal* nl);
 bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
                               int64_t ld_out, const double* coef, bool may_build, bool run, hipStream_t s);
 bool sphere_prepared(qg_nonlocal* nl, int dtype);
+size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build);
+bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, const double* k, double* part,
+                    double* coef, bool may_build, hipStream_t s);
 bool sphere_nonlocal_force(qg_nonlocal* nl, int dtype, int nocc, const int* band_idx, const double* weight,
                            const void* psi, int64_t ld, const double* coef, DevBuf<double>& part, double* force,
                            bool run, hipStream_t s);

@@ -1200,17 +1200,25 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     const RowsShape sh = rows_shape(g, dtype, nbands, &h->plan);
     const RowsGeo* rg = nullptr;    // apply kernel's geometry (tile rows ty)
     const RowsGeo* rgp = nullptr;   // projection kernel's geometry (tile rows typ)
+    // both launches from the sphere entry lists where they serve
     const bool sphere = nl && sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nullptr, ws == nullptr,
                                                        false, s);
-    if (nl && sphere) {
+    const size_t sphere_part = sphere ? sphere_project_need(nl, dtype, nbands, false, ws == nullptr) : 0;
+    if (sphere) {
         if (sh.typ == 0) return false;
-        QG_REQUIRE(!ws || sh.ty == rows_shape(g, dtype, 0).ty, "the projector geometry of this launch shape is not "
-                   "prepared (qg_nonlocal_create and qg_nonlocal_update prepare the default shapes)");
+        const RowsShape def = rows_shape(g, dtype, 0);
+        QG_REQUIRE(!ws || (sh.ty == def.ty && sh.tzp == def.tzp && sh.typ == def.typ),
+                   "the projector geometry of this launch shape is not prepared (qg_nonlocal_create and "
+                   "qg_nonlocal_update prepare the default shapes)");
+    }
+    if (sphere && sphere_part == 0) {
         rgp = rows_geometry(nl, sh.typ, sh.tzp, false, ws == nullptr);
         QG_REQUIRE(rgp, "the projector geometry of this launch shape is not prepared (qg_nonlocal_create and "
                         "qg_nonlocal_update prepare the default shapes)");
         if (!rgp->ok || rgp->max_items > kProjThreads * kItemsPT) return false;
         if (rows_proj_lds<T>(*rgp, g, sh.nbp, (int)nl->geo.projs.size()) > lds_limit()) return false;
+    } else if (sphere) {
+        // no geometry of the row kernels is needed
     } else if (nl) {
         if (sh.typ == 0) return false;
         // with caller scratch nothing may be allocated: the geometry must exist already
@@ -1234,7 +1242,7 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     double* part = nullptr;
     double* coef = nullptr;
     if (nl) {
-        const size_t npart = (size_t)std::max(1, rgp->nslot) * rgp->njs * nbands;
+        const size_t npart = sphere_part ? sphere_part : (size_t)std::max(1, rgp->nslot) * rgp->njs * nbands;
         const size_t ncoef = (size_t)nbands * nl->geo.ncoef;
         if (ws) {
             QG_REQUIRE(npart + ncoef <= ws->capacity, "application exceeds the fixed scratch size");
@@ -1249,7 +1257,9 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     }
     const bool timed = h->timing && ws == nullptr;
     if (timed) QG_HIP(hipEventRecord(h->tev[0], s));
-    if (nl) {
+    if (sphere_part) {
+        (void)sphere_project(nl, dtype, nbands, psi, ld, nullptr, part, coef, ws == nullptr, s);
+    } else if (nl) {
         if (rgp->njs == 4) {
             if (rgp->pform == 2) rows_launch_project<T, 4, 2>(nl, *rgp, sh.nbp, nbands, psi, ld, part, coef, s);
             else if (rgp->pform == 1) rows_launch_project<T, 4, 1>(nl, *rgp, sh.nbp, nbands, psi, ld, part, coef, s);
@@ -1304,7 +1314,12 @@ bool rows_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, i
 bool rows_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, double* coef,
                            DevBuf<double>& part_buf, hipStream_t s) {
     const qg_grid& g = nl->gcopy;
-    if (nl->geo.ncoef == 0 || !rows_eligible(g, dtype, nl)) return false;
+    if (nl->geo.ncoef == 0) return false;
+    if (const size_t need = sphere_project_need(nl, dtype, nbands, false, true)) {
+        part_buf.alloc(need);
+        return sphere_project(nl, dtype, nbands, psi, ld, nullptr, part_buf.p, coef, true, s);
+    }
+    if (!rows_eligible(g, dtype, nl)) return false;
     const RowsShape sh = rows_shape(g, dtype, nbands);
     if (sh.typ == 0) return false;
     const RowsGeo* rg = rows_geometry(nl, sh.typ, sh.tzp, false);
@@ -1359,9 +1374,10 @@ void rows_prepare(qg_nonlocal* nl) {
         if (!rows_eligible(nl->gcopy, dtype, nl)) continue;
         const RowsShape sh = rows_shape(nl->gcopy, dtype, 0);
         if (sh.typ == 0) continue;
-        // the apply pass of the rows kernels only where the sphere entry lists do not serve
-        if (!sphere_prepared(nl, dtype)) rows_geometry(nl, sh.ty, sh.tzp, true);
-        rows_geometry(nl, sh.typ, sh.tzp, false);
+        // only where the sphere entry lists do not serve
+        const bool apply = sphere_prepared(nl, dtype);
+        if (!apply) rows_geometry(nl, sh.ty, sh.tzp, true);
+        if (!apply || sphere_project_need(nl, dtype, 1, false, false) == 0) rows_geometry(nl, sh.typ, sh.tzp, false);
     }
 }
 
@@ -1410,14 +1426,23 @@ void rows_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64
     if (nl) {
         const RowsShape sh = rows_shape(g, dtype, nbands, &h->plan);
         QG_REQUIRE(sh.typ > 0, "the projection tile does not fit this grid");
-        const RowsGeo* rgp = rows_geometry(nl, sh.typ, sh.tzp, false, false);
-        QG_REQUIRE(rgp && rgp->ok, "the projector geometry of this launch shape is not prepared (qg_nonlocal_create "
-                                   "and qg_nonlocal_update prepare the default shapes)");
-        const size_t per_band = (size_t)std::max(1, rgp->nslot) * rgp->njs + (size_t)nl->geo.ncoef;
-        QG_REQUIRE(per_band <= kScratchDoubles,
-                   "one band needs " + std::to_string(per_band) + " doubles of projector scratch, more than the fixed " +
-                       std::to_string(kScratchDoubles));
-        chunk = (int)std::min<size_t>((size_t)nbands, kScratchDoubles / per_band);
+        // bands whose partials and coefficients fit
+        auto need = [&](int nb) { return sphere_project_need(nl, dtype, nb, false, false) + (size_t)nb * nl->geo.ncoef; };
+        if (sphere_prepared(nl, dtype) && sphere_project_need(nl, dtype, 1, false, false)) {
+            while (chunk > 1 && need(chunk) > kScratchDoubles) chunk = (chunk + 1) / 2;
+            QG_REQUIRE(need(chunk) <= kScratchDoubles,
+                       "one band needs " + std::to_string(need(1)) + " doubles of projector scratch, more than the fixed " +
+                           std::to_string(kScratchDoubles));
+        } else {
+            const RowsGeo* rgp = rows_geometry(nl, sh.typ, sh.tzp, false, false);
+            QG_REQUIRE(rgp && rgp->ok, "the projector geometry of this launch shape is not prepared (qg_nonlocal_create "
+                                       "and qg_nonlocal_update prepare the default shapes)");
+            const size_t per_band = (size_t)std::max(1, rgp->nslot) * rgp->njs + (size_t)nl->geo.ncoef;
+            QG_REQUIRE(per_band <= kScratchDoubles,
+                       "one band needs " + std::to_string(per_band) +
+                           " doubles of projector scratch, more than the fixed " + std::to_string(kScratchDoubles));
+            chunk = (int)std::min<size_t>((size_t)nbands, kScratchDoubles / per_band);
+        }
     }
     const size_t es = dtype == QG_F32 ? 4 : 8;
     for (int b0 = 0; b0 < nbands; b0 += chunk) {

@@ -47,6 +47,11 @@ template <class T>
 __device__ __forceinline__ Row<T> vload(rsrc_t r, int voff, int soff) {
     return __builtin_bit_cast(Row<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
+// the same with cache policy nt, for values read once
+template <class T>
+__device__ __forceinline__ Row<T> vload_once(rsrc_t r, int voff, int soff) {
+    return __builtin_bit_cast(Row<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
 template <class T>
 __device__ __forceinline__ void vstore(rsrc_t r, const Row<T>& v, int voff, int soff) {
     // cache policy nt: the results are not read back here, and keeping them out of L2 leaves it to
@@ -305,7 +310,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
         for (int k = 0; k < 3; ++k) __hip_atomic_fetch_add(d + k, f[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
 
-    auto step = [&](auto kc, int z) {
+    auto step = [&](auto kc, int z) __attribute__((always_inline)) {
         constexpr int k0 = decltype(kc)::value;
         T* Lp = planes + (size_t)((z - z0) & 1) * NB * lband;
         const int zn = min(z + 1, z1 - 1);
@@ -570,6 +575,396 @@ __global__ __launch_bounds__(256) void sphere_force_reduce_kernel(const double* 
             red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
 }
 
+// ------------------------------------------------------------------------ projection ----
+// Bloch phases of a k-point projection: k_d h_d per grid step (real blocks: unused)
+struct SpherePhase {
+    double kh[3];
+};
+
+struct SphereProjArgs {
+    int nx, ny, nz;
+    int ty, tz, ntile, nslab, nbands;     // tz: a multiple of kProjPlanes
+    int nq, tpb, nw, nepoch;
+    int64_t ld;                 // in T elements per band (complex blocks: 2 per point)
+    const int* col_off;
+    const int* col_img;
+    const SphereImage* images;
+    const int* slot_off;        // per (tile, epoch, wavefront): first slot
+    const uint32_t* mask;       // per (tile, epoch, wavefront, plane of the epoch): slots with points
+    const void* vals;           // [slot][plane of the epoch][radial vector][lane] 16-byte vectors
+    const uint32_t* words;      // [slot][lane]
+    int max_col;
+    double h[3];
+    double* part;               // [((tile * nslab + slab) * max_col + image) * NC + c][real bands]
+};
+
+// LDS bytes of a projection workgroup: image centres, phases of the slab's planes, sums, and the
+// wavefronts' exchange buffers
+template <class T>
+static size_t sphere_proj_lds(int max_col, int tz, int nw, int nbr, int nc, bool cplx) {
+    const size_t b = sizeof(T) * (4 * (size_t)(max_col + 1) + (cplx ? 2 * (size_t)tz : 0));
+    return (b + 15) / 16 * 16 + sizeof(double) * (size_t)nw * (max_col + 1) * nc * nbr +
+           (size_t)nw * 64 * (sizeof(T) * nc * nbr + 16 + sizeof(int));
+}
+
+// c_aj = dV sum_i beta_j(i) psi(i).  A workgroup owns a tile, a slab of planes and NB bands; every
+// lane reads its own points' psi (each value once, 16 bytes a lane, two planes ahead) and adds the
+// radial values times psi to running sums.  The lists of this pass give an image the same slot
+// for all planes of an epoch (kProjPlanes planes), so a slot's sums stay in registers for the
+// epoch; per channel they are sum f psi (s), and sum f psi, sum u f psi, sum z f psi (p; u the
+// point of the lane's group, z the plane of the epoch), which at the epoch's end give
+//   c_s,  c_y = dy P0, c_z = dz0 P0 + hz Pz, c_x = dx0 P0 + hx Pu
+// and go to the wavefront's own LDS sums (FP64), and at the slab's end to one partial per
+// (workgroup, image, coefficient, band).  Slots beyond the K held at once take another walk of
+// the epoch.  No barrier inside the loop and no projector value is evaluated.
+// psi is read once; measured against the row projection (projector values evaluated per item): 120^3 /
+// 512 FP32 bands 1.0 against 1.1 ms (3.5 TB/s), 24^3 / 8 FP64 bands 12 against 38 us, 40^3 / 16 FP32
+// bands 15 against 41 us, tables on 77x41x117 / 72 FP64 bands 190 against 290 us (per-point tables).
+// CPLX: complex bands (re, im interleaved) times exp(i k.x) of the point; the two parts are then
+// two real bands (the image's own phase is applied by the reduction).
+template <class T, int NB, int NS, int NP, bool RAG, bool CPLX>
+__global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjArgs a, SpherePhase ph,
+                                                                     const T* __restrict__ psi) {
+    constexpr int VN = 16 / sizeof(T);
+    constexpr int S = sizeof(T);
+    constexpr int NC = NS + 3 * NP;
+    constexpr int NV = NS + NP;
+    constexpr int NR = CPLX ? 2 * NB : NB;      // real bands
+    constexpr int PW = CPLX ? 2 : 1;            // 16-byte vectors per lane and band
+    constexpr int K = CPLX && NS == 2 && sizeof(T) == 8 ? 2 : 4;   // slots held at once (4 would spill there)
+    constexpr int E = kProjPlanes;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    T* imf = reinterpret_cast<T*>(smem);                      // [max_col + 1][4]
+    T* ez = imf + 4 * (size_t)(a.max_col + 1);                // [tz][2]
+    const size_t aoff = (sizeof(T) * (4 * (size_t)(a.max_col + 1) + (CPLX ? 2 * (size_t)a.tz : 0)) + 15) / 16 * 16;
+    double* sums = reinterpret_cast<double*>(smem + aoff);    // [nw][max_col + 1][NC][NR]
+
+    // order: bands fastest (they share the tile's lists in an XCD's L2), then slabs, then tiles
+    const int wg = xcd_order(blockIdx.x, gridDim.x);
+    const int nbg = (a.nbands + NB - 1) / NB;
+    const int b0 = wg % nbg * NB;
+    const int slab = wg / nbg % a.nslab;
+    const int tile = wg / (nbg * a.nslab);
+    const int y0 = tile * a.ty;
+    const int rows = min(a.ty, ny - y0);
+    const int z0 = slab * a.tz, z1 = min(z0 + a.tz, nz);
+    const int tid = threadIdx.x, nthr = a.tpb;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int r = tid / a.nq, xq = tid - r * a.nq;
+    const int x = RAG ? min(xq * VN, nx - VN) : xq * VN;
+    const bool own = r < rows;
+    const int plane = nx * ny;
+    const uint32_t band_bytes = (uint32_t)((int64_t)plane * nz * S * PW);
+    rsrc_t rin[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) rin[b] = rsrc(psi + (int64_t)min(b0 + b, a.nbands - 1) * a.ld, band_bytes);
+    const int vo = own ? ((y0 + r) * nx + x) * S * PW : kOOB;
+
+    const int c0 = a.col_off[tile];
+    const int ncol = a.col_off[tile + 1] - c0;
+    for (int li = tid; li <= ncol; li += nthr) {
+        const SphereImage* im = a.images + a.col_img[c0 + max(min(li, ncol - 1), 0)];
+        const bool ok = li < ncol;
+        imf[4 * li] = ok ? (T)im->f[0] : T(0);
+        imf[4 * li + 1] = ok ? (T)im->f[1] : T(0);
+        imf[4 * li + 2] = ok ? (T)im->f[2] : T(0);
+        imf[4 * li + 3] = ok ? (T)im->n[2] : T(0);
+    }
+    T exy[VN][2];
+    if constexpr (CPLX) {
+        for (int i = tid; i < z1 - z0; i += nthr) {
+            double s, c;
+            sincos(ph.kh[2] * (double)(z0 + i), &s, &c);
+            ez[2 * i] = (T)c;
+            ez[2 * i + 1] = (T)s;
+        }
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            double s, c;
+            sincos(ph.kh[0] * (double)(x + u) + ph.kh[1] * (double)(y0 + r), &s, &c);
+            exy[u][0] = (T)c;
+            exy[u][1] = (T)s;
+        }
+    }
+    for (int i = tid; i < a.nw * (a.max_col + 1) * NC * NR; i += nthr) sums[i] = 0.0;
+    __syncthreads();
+
+    const T hx = (T)a.h[0], hy = (T)a.h[1], hz = (T)a.h[2];
+    const int ep1 = (z1 + E - 1) / E;
+    // one step: a plane of one walk (K slots from s0) of an epoch; uniform over the wavefront
+    struct Step {
+        int ep, z, s0, ns, off;     // epoch, plane, first slot of the walk, slots of the epoch, its first slot
+    };
+    const size_t lists = (size_t)tile * a.nepoch * a.nw + wave;
+    auto open = [&](int ep) {       // the first step of the first epoch from ep on that has slots
+        Step s{ep, ep * E, 0, 0, 0};
+        while (s.ep < ep1) {
+            s.off = __builtin_amdgcn_readfirstlane(a.slot_off[lists + (size_t)s.ep * a.nw]);
+            s.ns = __builtin_amdgcn_readfirstlane(a.slot_off[lists + (size_t)s.ep * a.nw + 1]) - s.off;
+            if (s.ns > 0) break;
+            ++s.ep;
+        }
+        s.z = s.ep * E;
+        return s;
+    };
+    auto next = [&](Step s) {
+        if (s.ep >= ep1) return s;
+        ++s.z;
+        if (s.z < min((s.ep + 1) * E, z1)) return s;
+        s.s0 += K;
+        s.z = s.ep * E;
+        return s.s0 < s.ns ? s : open(s.ep + 1);
+    };
+    auto mask_of = [&](const Step& s) -> uint32_t {
+        if (s.ep >= ep1) return 0u;
+        return __builtin_amdgcn_readfirstlane(a.mask[(lists + (size_t)s.ep * a.nw) * E + (s.z - s.ep * E)]) >> s.s0;
+    };
+    struct Vals {
+        Row<T> f[NV];
+    };
+    constexpr int D = 2;            // planes of psi in flight (3 and 4: no faster)
+    Row<T> p[D][NB][PW];
+    Vals en[K];
+    uint32_t wd[K];
+    auto load_psi = [&](Row<T> (&q)[NB][PW], const Step& s) {
+        const int z = min(s.z, nz - 1);     // past the last step: a load that is not used
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int h = 0; h < PW; ++h) q[b][h] = vload_once<T>(rin[b], vo + (own ? 16 * h : 0), z * plane * S * PW);
+    };
+    // a slot without points in the plane is loaded through an empty resource (zeros, no traffic)
+    auto load_vals = [&](const Step& s, uint32_t m, int k) {
+        const int64_t at = ((int64_t)(s.off + s.s0 + k) * E + (s.z - s.ep * E)) * NV * 1024;
+        const bool on = (m >> k) & 1u;
+        const rsrc_t rv = rsrc((const unsigned char*)a.vals + (on ? at : 0), on ? NV * 1024u : 0u);
+        Vals e;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) e.f[v] = vload<T>(rv, lane * 16, v * 1024);
+        return e;
+    };
+    auto load_words = [&](const Step& s) {
+        const int cnt = s.ep < ep1 ? min(K, s.ns - s.s0) : 0;
+        const rsrc_t rw = rsrc(a.words + (cnt > 0 ? (int64_t)(s.off + s.s0) * 64 : 0), (uint32_t)max(cnt, 0) * 256);
+#pragma unroll
+        for (int k = 0; k < K; ++k) wd[k] = __builtin_amdgcn_raw_buffer_load_b32(rw, lane * 4, k * 256, 0);
+    };
+
+    T acc[K][NC][NR];
+    auto clear = [&] {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int b = 0; b < NR; ++b) acc[k][c][b] = T(0);
+    };
+    clear();
+    // the sums of one walk into the wavefront's LDS sums, a slot at a time: every lane puts its CN
+    // coefficients and its image into the wavefront's buffer; then lane l owns coefficient l % CN of
+    // CN neighbouring lanes, adds up runs of one image and the runs to the sums.  (Straight atomics
+    // from every lane met on one address per image: 130 cycles an instruction, the time of the pass.)
+    constexpr int CN = NC * NR;
+    static_assert(64 % CN == 0 && CN % VN == 0, "coefficients of a slot must divide the wavefront");
+    constexpr int BS = CN + VN;                              // buffer stride: 16-byte rows, no bank conflicts
+    T* buf = reinterpret_cast<T*>(sums + (size_t)a.nw * (a.max_col + 1) * CN) + (size_t)wave * 64 * BS;
+    int* lis = reinterpret_cast<int*>(reinterpret_cast<T*>(sums + (size_t)a.nw * (a.max_col + 1) * CN) +
+                                      (size_t)a.nw * 64 * BS) + wave * 64;
+    auto flush = [&](const Step& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if (s.s0 + k < s.ns) {
+                const int li = (int)(wd[k] & 1023u);
+                const int dyi = ((int)(wd[k] << 11)) >> 21, dxi = ((int)wd[k]) >> 21;
+                const T* im = imf + 4 * li;
+                const T dx0 = hx * ((T)dxi - im[0]), dy = hy * ((T)dyi - im[1]);
+                const T dz0 = hz * (((T)(s.ep * E) - im[3]) - im[2]);
+                T c[CN];
+#pragma unroll
+                for (int b = 0; b < NR; ++b) {
+#pragma unroll
+                    for (int q = 0; q < NS; ++q) c[q * NR + b] = acc[k][q][b];
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) {
+                        const double p0 = (double)acc[k][NS + 3 * q][b];
+                        c[(NS + 3 * q) * NR + b] = (T)((double)dy * p0);
+                        c[(NS + 3 * q + 1) * NR + b] = (T)((double)dz0 * p0 + (double)hz * (double)acc[k][NS + 3 * q + 2][b]);
+                        c[(NS + 3 * q + 2) * NR + b] = (T)((double)dx0 * p0 + (double)hx * (double)acc[k][NS + 3 * q + 1][b]);
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < CN / VN; ++v) {
+                    Row<T> w;
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) w.v[u] = c[v * VN + u];
+                    *reinterpret_cast<Row<T>*>(buf + lane * BS + v * VN) = w;
+                }
+                lis[lane] = li;
+                __builtin_amdgcn_wave_barrier();
+                const int own_c = lane % CN, l0 = lane - own_c;
+                auto add = [&](int row, double v) {
+                    __hip_atomic_fetch_add(sums + ((size_t)wave * (a.max_col + 1) + row) * CN + own_c, v, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                };
+                int run = lis[l0];
+                double sum = (double)buf[l0 * BS + own_c];
+#pragma unroll
+                for (int i = 1; i < CN; ++i) {
+                    const int l = lis[l0 + i];
+                    const double v = (double)buf[(l0 + i) * BS + own_c];
+                    if (l != run) {
+                        add(run, sum);
+                        run = l;
+                        sum = 0.0;
+                    }
+                    sum += v;
+                }
+                add(run, sum);
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        clear();
+    };
+
+    Step cur = open(z0 / E), nx1 = next(cur), nx2 = next(nx1);
+    uint32_t mcur = mask_of(cur), m1 = mask_of(nx1);
+    load_psi(p[0], cur);
+    load_words(cur);
+#pragma unroll
+    for (int k = 0; k < K; ++k) en[k] = load_vals(cur, mcur, k);
+    Step far = nx1;
+#pragma unroll
+    for (int i = 1; i < D; ++i) {
+        load_psi(p[i], far);
+        far = next(far);
+    }
+    auto step = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        // the plane's values as real bands; a point of two overlapping groups counts once
+        T v[NR][VN];
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            const bool mine = !RAG || x + u >= xq * VN;
+            if constexpr (CPLX) {
+                const T cz = ez[2 * (cur.z - z0)], sz = ez[2 * (cur.z - z0) + 1];
+                const T er = exy[u][0] * cz - exy[u][1] * sz, ei = exy[u][0] * sz + exy[u][1] * cz;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const T re = p[i][b][2 * u / VN].v[2 * u % VN], im = p[i][b][2 * u / VN].v[2 * u % VN + 1];
+                    v[2 * b][u] = mine ? er * re - ei * im : T(0);
+                    v[2 * b + 1][u] = mine ? er * im + ei * re : T(0);
+                }
+            } else {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) v[b][u] = mine ? p[i][b][0].v[u] : T(0);
+            }
+        }
+        const T zr = (T)(cur.z - cur.ep * E);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if ((mcur >> k) & 1u) {
+#pragma unroll
+                for (int b = 0; b < NR; ++b) {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s)
+#pragma unroll
+                        for (int u = 0; u < VN; ++u) acc[k][s][b] += en[k].f[s].v[u] * v[b][u];
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) {
+                        T t[VN], s0 = T(0);
+#pragma unroll
+                        for (int u = 0; u < VN; ++u) {
+                            t[u] = en[k].f[NS + q].v[u] * v[b][u];
+                            s0 += t[u];
+                        }
+                        acc[k][NS + 3 * q][b] += s0;
+#pragma unroll
+                        for (int u = 1; u < VN; ++u) acc[k][NS + 3 * q + 1][b] += (T)u * t[u];
+                        acc[k][NS + 3 * q + 2][b] += zr * s0;
+                    }
+                }
+            }
+            en[k] = load_vals(nx1, m1, k);
+        }
+        if (nx1.ep != cur.ep || nx1.s0 != cur.s0) {
+            flush(cur);
+            load_words(nx1);
+        }
+        // after the next plane's values: waiting for those leaves this load in flight
+        load_psi(p[i], far);
+        far = next(far);
+        cur = nx1;
+        nx1 = nx2;
+        mcur = m1;
+        m1 = mask_of(nx1);
+        nx2 = next(nx2);
+    };
+    while (cur.ep < ep1) {
+        step(std::integral_constant<int, 0>{});
+        if (cur.ep >= ep1) break;
+        step(std::integral_constant<int, 1>{});
+    }
+    __syncthreads();
+    const int nbr = (CPLX ? 2 : 1) * a.nbands;
+    double* part = a.part + ((size_t)tile * a.nslab + slab) * a.max_col * NC * nbr;
+    for (int i = tid; i < ncol * NC * NR; i += nthr) {
+        const int b = (CPLX ? 2 : 1) * b0 + i % NR;
+        double s = 0.0;
+        for (int w = 0; w < a.nw; ++w) s += sums[(size_t)w * (a.max_col + 1) * NC * NR + i];
+        if (b < nbr) part[(size_t)(i / NR) * nbr + b] = s;
+    }
+}
+
+// coef[b * ncoef + j] = dV * sum of the atom's partials over its (tile, column image) pairs and the
+// slabs, in a fixed order; complex: times exp(-i k.h shift) of the image
+// 64 bands by 4 parts of the sum per workgroup (the parts of one coefficient are added in order), so
+// that the dependent loads of a small problem's many partials run side by side
+template <bool CPLX>
+__global__ __launch_bounds__(256) void sphere_coef_reduce_kernel(
+    const double* __restrict__ part, int nslab, int max_col, int ns, int np, int nbands, const int* __restrict__ atom_ref_off,
+    const int2* __restrict__ atom_ref, const int* __restrict__ col_off, const int* __restrict__ col_img,
+    const SphereImage* __restrict__ images, const int* __restrict__ atom_chan, const int* __restrict__ atom_coef_off,
+    SpherePhase ph, double dv, double* __restrict__ coef, int ncoef) {
+    __shared__ double red[4][64][CPLX ? 2 : 1];
+    const int nc = ns + 3 * np;
+    const int at = blockIdx.x / nc, c = blockIdx.x % nc;
+    const int lb = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int b = blockIdx.y * 64 + lb;
+    const int slot = atom_chan[4 * at + (c < ns ? c : 2 + (c - ns) / 3)];
+    if (slot < 0) return;
+    const int nbr = (CPLX ? 2 : 1) * nbands;
+    double re = 0.0, im = 0.0;
+    const int k0 = atom_ref_off[at], n = (atom_ref_off[at + 1] - k0) * nslab;
+    if (b < nbands) {
+#pragma unroll 4
+        for (int i = q; i < n; i += 4) {
+            const int2 ref = atom_ref[k0 + i / nslab];
+            const double* p = part + ((((size_t)ref.x * nslab + i % nslab) * max_col + ref.y) * nc + c) * nbr;
+            if constexpr (CPLX) {
+                const SphereImage& g = images[col_img[col_off[ref.x] + ref.y]];
+                const double sr = p[2 * b], si = p[2 * b + 1];
+                double sn, cs;
+                sincos(-(ph.kh[0] * g.shift[0] + ph.kh[1] * g.shift[1] + ph.kh[2] * g.shift[2]), &sn, &cs);
+                re += cs * sr - sn * si;
+                im += cs * si + sn * sr;
+            } else {
+                re += p[b];
+            }
+        }
+    }
+    red[q][lb][0] = re;
+    if constexpr (CPLX) red[q][lb][1] = im;
+    __syncthreads();
+    if (q != 0 || b >= nbands) return;
+    const int64_t o = (int64_t)b * ncoef + atom_coef_off[at] + slot + (c < ns ? 0 : (c - ns) % 3);
+    constexpr int W = CPLX ? 2 : 1;
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+        coef[W * o + w] = dv * (((red[0][lb][w] + red[1][lb][w]) + red[2][lb][w]) + red[3][lb][w]);
+}
+
 // ------------------------------------------------------------------ entry lists ----
 // radial function of a channel at squared distance rr (inside its cutoff), FP64:
 // RadialGrid2::GetValueByXi (RadialGrid2.h:81-136) for tables
@@ -630,6 +1025,37 @@ __device__ __forceinline__ int2 part_row(const BuildArgs& a, const DevImage& p, 
     return a.intervals[p.row_base + (y - p.b[1]) + (p.e[1] - p.b[1]) * (z - p.b[2])];
 }
 
+// radial functions of image im at the VN points from (x, y, z), per channel (f zero on entry)
+template <class T, int NS, int NP>
+__device__ __forceinline__ void radial_rows(const BuildArgs& a, const SphereImage& im, int x, int y, int z,
+                                            Row<T> (&f)[NS + NP]) {
+    constexpr int VN = 16 / sizeof(T);
+    for (int k = 0; k < im.nparts; ++k) {
+        const DevImage& p = a.parts[im.part[k]];
+        const int2 iv = part_row(a, p, y, z);
+        const double dz = a.h[2] * (double)(z - p.shift[2]) - p.R[2];
+        const double dy = a.h[1] * (double)(y - p.shift[1]) - p.R[1];
+        for (int pj = p.proj_begin; pj < p.proj_end; ++pj) {
+            const DevProj& d = a.projs[pj];
+#pragma unroll
+            for (int c = 0; c < NS + NP; ++c) {
+                // the channel of this projector: the one whose coefficient slot it fills
+                if (a.atom_chan[4 * im.atom + (c < NS ? c : 2 + c - NS)] != d.coef_rel) continue;
+                if ((d.l == 0) != (c < NS)) continue;
+#pragma unroll
+                for (int u = 0; u < VN; ++u) {
+                    if (x + u < iv.x || x + u >= iv.y) continue;
+                    const double dx = a.h[0] * (double)(x + u - p.shift[0]) - p.R[0];
+                    const double rr = dx * dx + (dy * dy + dz * dz);
+                    const double rad = radial_dev(d, a.tables, rr);
+                    if (d.l == 0) f[c].v[u] = (T)(rad * 0.28209479177387814);          // Y00
+                    else f[c].v[u] = 1.0e-14 > rr ? T(0) : (T)(rad * 0.48860251190291992 / sqrt(rr));
+                }
+            }
+        }
+    }
+}
+
 // One workgroup per (tile, plane), one thread per lane of the apply workgroup.  FILL false:
 // counts the images touching each lane's group and records the wavefront's largest count; FILL
 // true: writes the lane's entries and pads to that count with the empty image.
@@ -660,33 +1086,8 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_build_kernel(BuildArgs a) 
         if constexpr (FILL) {
             Row<T> f[NV];
 #pragma unroll
-            for (int c = 0; c < NV; ++c)
-#pragma unroll
-                for (int u = 0; u < VN; ++u) f[c].v[u] = T(0);
-            for (int k = 0; k < im.nparts; ++k) {
-                const DevImage& p = a.parts[im.part[k]];
-                const int2 iv = part_row(a, p, y, z);
-                const double dz = a.h[2] * (double)(z - p.shift[2]) - p.R[2];
-                const double dy = a.h[1] * (double)(y - p.shift[1]) - p.R[1];
-                for (int pj = p.proj_begin; pj < p.proj_end; ++pj) {
-                    const DevProj& d = a.projs[pj];
-#pragma unroll
-                    for (int c = 0; c < NV; ++c) {
-                        // the channel of this projector: the one whose coefficient slot it fills
-                        if (a.atom_chan[4 * im.atom + (c < NS ? c : 2 + c - NS)] != d.coef_rel) continue;
-                        if ((d.l == 0) != (c < NS)) continue;
-#pragma unroll
-                        for (int u = 0; u < VN; ++u) {
-                            if (x + u < iv.x || x + u >= iv.y) continue;
-                            const double dx = a.h[0] * (double)(x + u - p.shift[0]) - p.R[0];
-                            const double rr = dx * dx + (dy * dy + dz * dz);
-                            const double rad = radial_dev(d, a.tables, rr);
-                            if (d.l == 0) f[c].v[u] = (T)(rad * 0.28209479177387814);          // Y00
-                            else f[c].v[u] = 1.0e-14 > rr ? T(0) : (T)(rad * 0.48860251190291992 / sqrt(rr));
-                        }
-                    }
-                }
-            }
+            for (int c = 0; c < NV; ++c) f[c] = Row<T>{};
+            radial_rows<T, NS, NP>(a, im, x, y, z, f);
 #pragma unroll
             for (int c = 0; c < NV; ++c) vals[((size_t)(base + n) * NV + c) * 64 + lane] = f[c];
             a.words[(size_t)(base + n) * 64 + lane] = entry_word(li, x - im.n[0], y - im.n[1]);
@@ -699,6 +1100,74 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_build_kernel(BuildArgs a) 
 #pragma unroll
             for (int c = 0; c < NV; ++c) vals[((size_t)(base + n) * NV + c) * 64 + lane] = Row<T>{};
             a.words[(size_t)(base + n) * 64 + lane] = entry_word(ncol, 0, 0);
+        }
+    } else {
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) n = max(n, __shfl_xor(n, s, 64));
+        if (lane == 0) a.trips[w] = n;
+    }
+}
+
+// The projection's lists: one workgroup per (tile, epoch).  A lane gives every image that touches its
+// group in the epoch a slot, in image order.  FILL false: records the wavefront's number of slots;
+// FILL true: writes words, values of every (slot, plane) and the planes' slot masks.
+template <class T, int NS, int NP, bool FILL>
+__global__ __launch_bounds__(kMaxThreads) void sphere_slots_kernel(BuildArgs a, uint32_t* __restrict__ mask) {
+    constexpr int VN = 16 / sizeof(T);
+    constexpr int NV = NS + NP;
+    constexpr int E = kProjPlanes;
+    const int tile = blockIdx.x, ep = blockIdx.y;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int y0 = tile * a.ty;
+    const int r = tid / a.nq;
+    const int x = min((tid - r * a.nq) * VN, a.nx - VN);
+    const int y = y0 + r;
+    const bool own = r < min(a.ty, a.ny - y0);
+    const int c0 = a.col_off[tile], ncol = a.col_off[tile + 1] - c0;
+    const size_t w = ((size_t)tile * gridDim.y + ep) * a.nw + wave;
+    const int zb = ep * E, ze = min(zb + E, a.nz);
+    int n = 0;
+    const int base = FILL ? a.trip_off[w] : 0;
+    const int cnt = FILL ? a.trip_off[w + 1] - base : 0;
+    Row<T>* vals = reinterpret_cast<Row<T>*>(a.vals);
+    uint32_t has[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) has[e] = 0u;
+    for (int li = 0; own && li < ncol; ++li) {
+        const SphereImage im = a.images[a.col_img[c0 + li]];
+        uint32_t in = 0u;     // planes of the epoch where the image touches the group
+        for (int z = max(zb, im.b[2]); z < min(ze, im.e[2]); ++z)
+            for (int k = 0; k < im.nparts; ++k) {
+                const int2 iv = part_row(a, a.parts[im.part[k]], y, z);
+                if (iv.x < x + VN && iv.y > x) in |= 1u << (z - zb);
+            }
+        if (!in) continue;
+        if constexpr (FILL) {
+            for (int e = 0; e < E; ++e) {
+                Row<T> f[NV];
+#pragma unroll
+                for (int c = 0; c < NV; ++c) f[c] = Row<T>{};
+                if ((in >> e) & 1u) radial_rows<T, NS, NP>(a, im, x, y, zb + e, f);
+#pragma unroll
+                for (int c = 0; c < NV; ++c) vals[(((size_t)(base + n) * E + e) * NV + c) * 64 + lane] = f[c];
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) has[e] |= ((in >> e) & 1u) << n;
+            a.words[(size_t)(base + n) * 64 + lane] = entry_word(li, x - im.n[0], y - im.n[1]);
+        }
+        ++n;
+    }
+    if constexpr (FILL) {
+        for (; n < cnt; ++n) {
+            for (int e = 0; e < E * NV; ++e) vals[((size_t)(base + n) * E * NV + e) * 64 + lane] = Row<T>{};
+            a.words[(size_t)(base + n) * 64 + lane] = entry_word(ncol, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            uint32_t m = has[e];
+#pragma unroll
+            for (int s = 32; s >= 1; s >>= 1) m |= __shfl_xor(m, s, 64);
+            if (lane == 0) mask[w * E + e] = m;
         }
     } else {
 #pragma unroll
@@ -776,6 +1245,7 @@ static void sphere_images(qg_nonlocal* nl) {
             for (int d = 0; d < 3; ++d) {
                 const double u = im.R[d] / nl->gcopy.h[d], nn = std::rint(u);
                 s.n[d] = im.shift[d] + (int)nn;
+                s.shift[d] = im.shift[d];
                 s.f[d] = u - nn;
                 s.b[d] = im.b[d];
                 s.e[d] = im.e[d];
@@ -863,6 +1333,48 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
             }
             QG_HIP(hipGetLastError());
         };
+        // the projection's lists (a word of the masks holds 32 slots; more: the other projections serve)
+        auto build_slots = [&](SphereGeo* o, BuildArgs b) {
+            const int nep = (nz + kProjPlanes - 1) / kProjPlanes;
+            const size_t ne = (size_t)o->ntile * nep * nw;
+            std::vector<int> cnt(ne + 1, 0);
+            o->d_slot_off.alloc(ne + 1);
+            o->d_slot_mask.alloc(ne * kProjPlanes);
+            b.trips = o->d_slot_off.p;
+            auto go = [&](auto tag, bool fill) {
+                using T = decltype(tag);
+                const dim3 grid(o->ntile, nep), blk(o->tpb);
+                if (two) {
+                    if (fill) hipLaunchKernelGGL((sphere_slots_kernel<T, 2, 2, true>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
+                    else hipLaunchKernelGGL((sphere_slots_kernel<T, 2, 2, false>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
+                } else {
+                    if (fill) hipLaunchKernelGGL((sphere_slots_kernel<T, 1, 1, true>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
+                    else hipLaunchKernelGGL((sphere_slots_kernel<T, 1, 1, false>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
+                }
+                QG_HIP(hipGetLastError());
+            };
+            dtype == QG_F32 ? go(float{}, false) : go(double{}, false);
+            QG_HIP(hipMemcpy(cnt.data(), o->d_slot_off.p, ne * sizeof(int), hipMemcpyDeviceToHost));
+            int64_t sum = 0;
+            int most = 0;
+            for (size_t k = 0; k <= ne; ++k) {
+                const int n = k < ne ? cnt[k] : 0;
+                cnt[k] = (int)std::min<int64_t>(sum, INT32_MAX);
+                sum += n;
+                most = std::max(most, n);
+            }
+            const int nv = nl->sphere_form.ns + nl->sphere_form.np;
+            if (most > 32 || sum >= (1LL << 28)) return;
+            const size_t slots = (size_t)std::max<int64_t>(1, sum);
+            o->d_slot_off.upload(cnt.data(), cnt.size());
+            o->d_slot_words.alloc(slots * 64);
+            o->d_slot_vals.alloc(slots * kProjPlanes * 64 * nv * 16);
+            b.trip_off = o->d_slot_off.p;
+            b.words = o->d_slot_words.p;
+            b.vals = o->d_slot_vals.p;
+            dtype == QG_F32 ? go(float{}, true) : go(double{}, true);
+            o->slots_ok = true;
+        };
         dtype == QG_F32 ? launch(float{}, false) : launch(double{}, false);
         QG_HIP(hipMemcpy(trips.data(), c->d_trip_off.p, nwv * sizeof(int), hipMemcpyDeviceToHost));
         int64_t total = 0;
@@ -881,9 +1393,10 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
             a.words = c->d_words.p;
             a.vals = c->d_vals.p;
             dtype == QG_F32 ? launch(float{}, true) : launch(double{}, true);
-            QG_HIP(hipStreamSynchronize(nullptr));
             c->ok = true;
+            build_slots(c.get(), a);
         }
+        QG_HIP(hipStreamSynchronize(nullptr));
     }
     nl->sphere.push_back(std::move(c));
     return nl->sphere.back().get();
@@ -987,6 +1500,130 @@ static SphereArgs sphere_args(const qg_nonlocal* nl, const SphereGeo& sg, int nb
 // Two bands per workgroup (an entry is loaded once for both) where that leaves two workgroups per CU
 static int sphere_pick_nb(const SphereGeo& sg, int nbands) {
     return (int64_t)sg.ntile * ((nbands + 1) / 2) >= 512 ? 2 : 1;
+}
+
+// Launch shape of a projection over nbands bands: bands per workgroup, planes per slab, partials
+struct SphereProjShape {
+    const SphereGeo* sg = nullptr;
+    int nb = 0, tz = 0, nslab = 0;
+    size_t lds = 0, npart = 0;     // npart: doubles of the partials
+};
+
+template <class T>
+static bool sphere_proj_shape(qg_nonlocal* nl, int nbands, bool cplx, bool may_build, SphereProjShape& sh) {
+    if (!sphere_serves(nl->gcopy, nl)) return false;
+    const qg_grid& g = nl->gcopy;
+    if (cplx && g.ng() * 16 > (int64_t)kOOB - 64) return false;   // band bytes below the out-of-range offset
+    constexpr int VN = 16 / sizeof(T);
+    const int nq = (g.n[0] + VN - 1) / VN;
+    const int ty = sphere_pick_ty(nq, g.n[1], 0);
+    sh.sg = ty > 0 ? sphere_geometry(nl, sizeof(T) == 4 ? QG_F32 : QG_F64, ty, may_build) : nullptr;
+    if (!sh.sg || !sh.sg->slots_ok) return false;
+    const int nc = nl->sphere_form.ns + 3 * nl->sphere_form.np;
+    const int nw = sh.sg->tpb / 64;
+    // real bands per workgroup: 4 FP32 or 2 FP64 with 1 + 1 channels, half with 2 + 2 (their running
+    // sums fill the registers)
+    const int nbr = (sizeof(T) == 4 ? 4 : 2) / (nl->sphere_form.ns == 2 ? 2 : 1);
+    sh.nb = cplx ? std::max(1, nbr / 2) : nbr;
+    auto shape = [&] {
+        // slabs of whole epochs for ~4096 workgroups
+        const int64_t wg = (int64_t)sh.sg->ntile * ((nbands + sh.nb - 1) / sh.nb);
+        const int nep = (g.n[2] + kProjPlanes - 1) / kProjPlanes;
+        const int want = (int)std::max<int64_t>(1, std::min<int64_t>((4096 + wg - 1) / wg, nep));
+        sh.tz = (nep + want - 1) / want * kProjPlanes;
+        sh.nslab = (g.n[2] + sh.tz - 1) / sh.tz;
+        sh.lds = sphere_proj_lds<T>(sh.sg->max_col, sh.tz, nw, cplx ? 2 * sh.nb : sh.nb, nc, cplx);
+    };
+    shape();
+    if (sh.lds > lds_limit() && sh.nb > 1) {
+        sh.nb = 1;
+        shape();
+    }
+    if (sh.lds > lds_limit()) return false;
+    sh.npart = (size_t)sh.sg->ntile * sh.nslab * std::max(1, sh.sg->max_col) * nc * nbands * (cplx ? 2 : 1);
+    return true;
+}
+
+// Doubles of partials a projection of nbands bands needs; 0 where the entry lists do not serve it.
+size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build) {
+    SphereProjShape sh;
+    const bool ok = dtype == QG_F32 ? sphere_proj_shape<float>(nl, nbands, cplx, may_build, sh)
+                                    : sphere_proj_shape<double>(nl, nbands, cplx, may_build, sh);
+    return ok ? std::max<size_t>(1, sh.npart) : 0;
+}
+
+template <class T, int NB, int NS, int NP, bool CPLX>
+static void sphere_project_launch(const SphereProjArgs& a, const SpherePhase& ph, const T* psi, size_t lds, hipStream_t s) {
+    const int64_t nwg = (int64_t)a.ntile * a.nslab * ((a.nbands + NB - 1) / NB);
+    QG_REQUIRE(nwg < (1LL << 31), "too many workgroups");
+    const dim3 grid((unsigned)nwg), blk(a.tpb);
+    if (a.nx % (16 / (int)sizeof(T)) != 0)
+        hipLaunchKernelGGL((sphere_project_kernel<T, NB, NS, NP, true, CPLX>), grid, blk, lds, s, a, ph, psi);
+    else
+        hipLaunchKernelGGL((sphere_project_kernel<T, NB, NS, NP, false, CPLX>), grid, blk, lds, s, a, ph, psi);
+    QG_HIP(hipGetLastError());
+}
+
+template <class T>
+static bool sphere_project_t(qg_nonlocal* nl, int nbands, const T* psi, int64_t ld, const double* k, double* part,
+                             double* coef, bool may_build, hipStream_t s) {
+    const bool cplx = k != nullptr;
+    SphereProjShape sh;
+    if (!sphere_proj_shape<T>(nl, nbands, cplx, may_build, sh)) return false;
+    const qg_grid& g = nl->gcopy;
+    const SphereGeo& sg = *sh.sg;
+    SphereProjArgs a{};
+    a.nx = g.n[0]; a.ny = g.n[1]; a.nz = g.n[2];
+    a.ty = sg.ty; a.tz = sh.tz; a.ntile = sg.ntile; a.nslab = sh.nslab; a.nbands = nbands;
+    a.nq = sg.nq; a.tpb = sg.tpb; a.nw = sg.tpb / 64;
+    a.ld = cplx ? 2 * ld : ld;
+    a.col_off = sg.d_col_off.p; a.col_img = sg.d_col_img.p; a.images = nl->d_sphere_img.p;
+    a.nepoch = (g.n[2] + kProjPlanes - 1) / kProjPlanes;
+    a.slot_off = sg.d_slot_off.p; a.mask = sg.d_slot_mask.p;
+    a.vals = sg.d_slot_vals.p; a.words = sg.d_slot_words.p;
+    a.max_col = std::max(1, sg.max_col);
+    for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
+    a.part = part;
+    SpherePhase ph{};
+    if (cplx)
+        for (int d = 0; d < 3; ++d) ph.kh[d] = k[d] * g.h[d];
+    constexpr int F = sizeof(T) == 4 ? 4 : 2;    // real bands with 1 + 1 channels
+    const bool two = nl->sphere_form.ns == 2;
+#define QG_SPHERE_PROJ(NB, NS, NP, C) sphere_project_launch<T, NB, NS, NP, C>(a, ph, psi, sh.lds, s)
+    if (cplx) {
+        if (two) QG_SPHERE_PROJ(1, 2, 2, true);
+        else if (sh.nb == F / 2) QG_SPHERE_PROJ(F / 2, 1, 1, true);
+        else QG_SPHERE_PROJ(1, 1, 1, true);
+    } else if (two) {
+        if (sh.nb == F / 2) QG_SPHERE_PROJ(F / 2, 2, 2, false);
+        else QG_SPHERE_PROJ(1, 2, 2, false);
+    } else {
+        if (sh.nb == F) QG_SPHERE_PROJ(F, 1, 1, false);
+        else QG_SPHERE_PROJ(1, 1, 1, false);
+    }
+#undef QG_SPHERE_PROJ
+    const int nc = nl->sphere_form.ns + 3 * nl->sphere_form.np;
+    const dim3 rgrid((unsigned)(nl->geo.natoms * nc), (unsigned)((nbands + 63) / 64));
+    QG_REQUIRE(rgrid.y <= 65535, "too many bands in one projection");
+    auto reduce = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, rgrid, dim3(256), 0, s, part, sh.nslab, a.max_col, nl->sphere_form.ns,
+                           nl->sphere_form.np, nbands, sg.d_atom_ref_off.p, sg.d_atom_ref.p, a.col_off, a.col_img,
+                           a.images, nl->d_atom_chan.p, nl->d_atom_coef_off.p, ph, g.dvol(), coef, nl->geo.ncoef);
+    };
+    if (cplx) reduce(sphere_coef_reduce_kernel<true>);
+    else reduce(sphere_coef_reduce_kernel<false>);
+    QG_HIP(hipGetLastError());
+    return true;
+}
+
+// coef[b * ncoef + j] = dV sum beta_j psi_b through the entry lists, part holding
+// sphere_project_need doubles; k non-null: complex blocks (dtype the type of a part, ld and coef in
+// complex elements) with the Bloch phases of k.  False (nothing launched) where not served.
+bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, const double* k, double* part,
+                    double* coef, bool may_build, hipStream_t s) {
+    if (dtype == QG_F32)
+        return sphere_project_t<float>(nl, nbands, (const float*)psi, ld, k, part, coef, may_build, s);
+    return sphere_project_t<double>(nl, nbands, (const double*)psi, ld, k, part, coef, may_build, s);
 }
 
 template <class T, int NB, int NS, int NP>
