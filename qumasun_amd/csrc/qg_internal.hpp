@@ -221,16 +221,20 @@ struct SphereGeo {
     int max_col = 0;     // most sphere images of one tile column
     int ntrips = 1;
     bool ok = false;
-    DevBuf<int> d_col_off, d_col_img, d_trip_off;
-    DevBuf<int> d_atom_ref_off;    // per atom: its (tile, column image) pairs
-    DevBuf<int2> d_atom_ref;
-    DevBuf<uint32_t> d_words;
-    DevBuf<unsigned char> d_vals;
-    // the projection's lists: slots per (tile, epoch, wavefront)
-    bool slots_ok = false;
-    DevBuf<int> d_slot_off;
-    DevBuf<uint32_t> d_slot_mask, d_slot_words;
-    DevBuf<unsigned char> d_slot_vals;
+    bool slots_ok = false;   // the projection's lists, slots per (tile, epoch, wavefront), are there
+    const int* col_off = nullptr;
+    const int* col_img = nullptr;
+    const int* atom_ref_off = nullptr;    // per atom: its (tile, column image) pairs
+    const int2* atom_ref = nullptr;
+    const int* trip_off = nullptr;
+    const int* slot_off = nullptr;
+    const uint32_t* slot_mask = nullptr;
+    const uint32_t* words = nullptr;
+    const uint32_t* slot_words = nullptr;
+    const void* vals = nullptr;
+    const void* slot_vals = nullptr;
+    DevBuf<int> meta, counts;             // what the pointers above point into
+    DevBuf<unsigned char> lists;
 };
 // planes of one epoch of the projection's lists
 constexpr int kProjPlanes = 8;
@@ -315,6 +319,7 @@ bool rows_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* p
 bool rows_laplacian_apply(const qg_grid& g, int dtype, int nbands, const void* psi, int64_t ld, void* out,
                           int64_t ld_out, double coef, int accumulate, hipStream_t s);
 void rows_prepare(qg_nonlocal* nl);
+bool rows_serve(const qg_nonlocal* nl, int dtype);
 void sphere_prepare(qg_nonlocal* nl);
 bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
                               int64_t ld_out, const double* coef, bool may_build, bool run, hipStream_t s);

@@ -962,6 +962,8 @@ static bool rows_eligible(const qg_grid& g, int dtype, const qg_nonlocal* nl) {
     return true;
 }
 
+bool rows_serve(const qg_nonlocal* nl, int dtype) { return rows_eligible(nl->gcopy, dtype, nl); }
+
 static int rows_nthr(const qg_grid& g, int dtype, int ty, int nbw) {
     const int VN = dtype == QG_F32 ? 4 : 2;
     return nbw * round64i(std::max(ty, 8) * (g.n[0] / VN));

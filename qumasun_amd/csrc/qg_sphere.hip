@@ -1076,7 +1076,8 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_build_kernel(BuildArgs a) 
     const int base = FILL ? a.trip_off[w] : 0;
     Row<T>* vals = reinterpret_cast<Row<T>*>(a.vals);
     for (int li = 0; own && li < ncol; ++li) {
-        const SphereImage im = a.images[a.col_img[c0 + li]];
+        const SphereImage& im = a.images[a.col_img[c0 + li]];
+        if (y < im.b[1] || y >= im.e[1] || x + VN <= im.b[0] || x >= im.e[0] || z < im.b[2] || z >= im.e[2]) continue;
         bool touch = false;
         for (int k = 0; k < im.nparts; ++k) {
             const int2 iv = part_row(a, a.parts[im.part[k]], y, z);
@@ -1110,7 +1111,8 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_build_kernel(BuildArgs a) 
 
 // The projection's lists: one workgroup per (tile, epoch).  A lane gives every image that touches its
 // group in the epoch a slot, in image order.  FILL false: records the wavefront's number of slots;
-// FILL true: writes words, values of every (slot, plane) and the planes' slot masks.
+// FILL true (a workgroup per plane of the epoch): writes words, values of every (slot, plane) and the
+// planes' slot masks.
 template <class T, int NS, int NP, bool FILL>
 __global__ __launch_bounds__(kMaxThreads) void sphere_slots_kernel(BuildArgs a, uint32_t* __restrict__ mask) {
     constexpr int VN = 16 / sizeof(T);
@@ -1130,45 +1132,42 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_slots_kernel(BuildArgs a, 
     const int base = FILL ? a.trip_off[w] : 0;
     const int cnt = FILL ? a.trip_off[w + 1] - base : 0;
     Row<T>* vals = reinterpret_cast<Row<T>*>(a.vals);
-    uint32_t has[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) has[e] = 0u;
+    const int e = blockIdx.z;     // filling: one plane of the epoch
+    uint32_t has = 0u;
     for (int li = 0; own && li < ncol; ++li) {
-        const SphereImage im = a.images[a.col_img[c0 + li]];
+        const SphereImage& im = a.images[a.col_img[c0 + li]];
+        if (y < im.b[1] || y >= im.e[1] || x + VN <= im.b[0] || x >= im.e[0] || ze <= im.b[2] || zb >= im.e[2]) continue;
         uint32_t in = 0u;     // planes of the epoch where the image touches the group
-        for (int z = max(zb, im.b[2]); z < min(ze, im.e[2]); ++z)
-            for (int k = 0; k < im.nparts; ++k) {
-                const int2 iv = part_row(a, a.parts[im.part[k]], y, z);
-                if (iv.x < x + VN && iv.y > x) in |= 1u << (z - zb);
+        for (int k = 0; k < im.nparts; ++k) {
+            const DevImage& part = a.parts[im.part[k]];
+#pragma unroll
+            for (int d = 0; d < E; ++d) {
+                const int2 iv = part_row(a, part, y, zb + d);
+                if (iv.x < x + VN && iv.y > x) in |= 1u << d;
             }
+        }
         if (!in) continue;
         if constexpr (FILL) {
-            for (int e = 0; e < E; ++e) {
-                Row<T> f[NV];
+            Row<T> f[NV];
 #pragma unroll
-                for (int c = 0; c < NV; ++c) f[c] = Row<T>{};
-                if ((in >> e) & 1u) radial_rows<T, NS, NP>(a, im, x, y, zb + e, f);
+            for (int c = 0; c < NV; ++c) f[c] = Row<T>{};
+            if ((in >> e) & 1u) radial_rows<T, NS, NP>(a, im, x, y, zb + e, f);
 #pragma unroll
-                for (int c = 0; c < NV; ++c) vals[(((size_t)(base + n) * E + e) * NV + c) * 64 + lane] = f[c];
-            }
-#pragma unroll
-            for (int e = 0; e < E; ++e) has[e] |= ((in >> e) & 1u) << n;
-            a.words[(size_t)(base + n) * 64 + lane] = entry_word(li, x - im.n[0], y - im.n[1]);
+            for (int c = 0; c < NV; ++c) vals[(((size_t)(base + n) * E + e) * NV + c) * 64 + lane] = f[c];
+            has |= ((in >> e) & 1u) << n;
+            if (e == 0) a.words[(size_t)(base + n) * 64 + lane] = entry_word(li, x - im.n[0], y - im.n[1]);
         }
         ++n;
     }
     if constexpr (FILL) {
         for (; n < cnt; ++n) {
-            for (int e = 0; e < E * NV; ++e) vals[((size_t)(base + n) * E * NV + e) * 64 + lane] = Row<T>{};
-            a.words[(size_t)(base + n) * 64 + lane] = entry_word(ncol, 0, 0);
+#pragma unroll
+            for (int c = 0; c < NV; ++c) vals[(((size_t)(base + n) * E + e) * NV + c) * 64 + lane] = Row<T>{};
+            if (e == 0) a.words[(size_t)(base + n) * 64 + lane] = entry_word(ncol, 0, 0);
         }
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            uint32_t m = has[e];
-#pragma unroll
-            for (int s = 32; s >= 1; s >>= 1) m |= __shfl_xor(m, s, 64);
-            if (lane == 0) mask[w * E + e] = m;
-        }
+        for (int s = 32; s >= 1; s >>= 1) has |= __shfl_xor(has, s, 64);
+        if (lane == 0) mask[w * E + e] = has;
     } else {
 #pragma unroll
         for (int s = 32; s >= 1; s >>= 1) n = max(n, __shfl_xor(n, s, 64));
@@ -1302,99 +1301,92 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
         ref.insert(ref.end(), v.begin(), v.end());
         ref_off.push_back((int)ref.size());
     }
-    if (ref.empty()) ref.push_back(make_int2(0, 0));
-    if (img.empty()) img.push_back(0);
     if (c->max_col < 1023) {
-        c->d_atom_ref_off.upload(ref_off.data(), ref_off.size());
-        c->d_atom_ref.upload(ref.data(), ref.size());
-        c->d_col_off.upload(off.data(), off.size());
-        c->d_col_img.upload(img.data(), img.size());
+        // one upload for the index arrays, one read and one write of the counts, one allocation for the
+        // lists: their number is what a small cell's set-up costs
+        std::vector<int> meta(off);
+        auto put = [&](const int* p, size_t n) {
+            const size_t at = (meta.size() + 1) / 2 * 2;
+            meta.resize(at + std::max<size_t>(n, 2), 0);
+            std::copy(p, p + n, meta.begin() + at);
+            return at;
+        };
+        const size_t at_img = put(img.data(), img.size()), at_roff = put(ref_off.data(), ref_off.size());
+        const size_t at_ref = put(reinterpret_cast<const int*>(ref.data()), 2 * ref.size());
+        c->meta.alloc(meta.size());
+        QG_HIP(hipMemcpyAsync(c->meta.p, meta.data(), meta.size() * sizeof(int), hipMemcpyHostToDevice, nullptr));
+        c->col_off = c->meta.p;
+        c->col_img = c->meta.p + at_img;
+        c->atom_ref_off = c->meta.p + at_roff;
+        c->atom_ref = reinterpret_cast<const int2*>(c->meta.p + at_ref);
+        const int nep = (nz + kProjPlanes - 1) / kProjPlanes;
+        const size_t nwv = (size_t)c->ntile * nz * nw, ne = (size_t)c->ntile * nep * nw;
+        std::vector<int> cnt(nwv + 1 + ne + 1, 0);
+        c->counts.alloc(cnt.size() + ne * kProjPlanes);
+        c->trip_off = c->counts.p;
+        c->slot_off = c->counts.p + nwv + 1;
+        uint32_t* mask = reinterpret_cast<uint32_t*>(c->counts.p + cnt.size());
+        c->slot_mask = mask;
         BuildArgs a{};
         a.nx = g.n[0]; a.ny = g.n[1]; a.nz = nz;
         a.ty = ty; a.ntile = c->ntile; a.nq = c->nq; a.tpb = c->tpb; a.nw = nw;
         for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
-        a.col_off = c->d_col_off.p; a.col_img = c->d_col_img.p;
+        a.col_off = c->col_off; a.col_img = c->col_img;
         a.images = nl->d_sphere_img.p; a.parts = nl->d_images.p; a.intervals = nl->d_intervals.p;
         a.projs = nl->d_projs.p; a.tables = nl->d_tables.p; a.atom_chan = nl->d_atom_chan.p;
-        const size_t nwv = (size_t)c->ntile * nz * nw;
-        std::vector<int> trips(nwv + 1, 0);
-        c->d_trip_off.alloc(nwv + 1);
-        a.trips = c->d_trip_off.p;
+        BuildArgs s = a;     // the projection's lists
+        a.trips = c->counts.p;
+        s.trips = c->counts.p + nwv + 1;
         const bool two = nl->sphere_form.ns == 2;
-        auto launch = [&](auto tag, bool fill) {
+        auto build = [&](auto tag, auto fill, bool slots) {
             using T = decltype(tag);
-            const dim3 grid(c->ntile, nz), blk(c->tpb);
+            constexpr bool F = decltype(fill)::value;
+            const dim3 blk(c->tpb), tg(c->ntile, nz), sgr(c->ntile, nep, F ? kProjPlanes : 1);
             if (two) {
-                if (fill) hipLaunchKernelGGL((sphere_build_kernel<T, 2, 2, true>), grid, blk, 0, nullptr, a);
-                else hipLaunchKernelGGL((sphere_build_kernel<T, 2, 2, false>), grid, blk, 0, nullptr, a);
+                hipLaunchKernelGGL((sphere_build_kernel<T, 2, 2, F>), tg, blk, 0, nullptr, a);
+                if (slots) hipLaunchKernelGGL((sphere_slots_kernel<T, 2, 2, F>), sgr, blk, 0, nullptr, s, mask);
             } else {
-                if (fill) hipLaunchKernelGGL((sphere_build_kernel<T, 1, 1, true>), grid, blk, 0, nullptr, a);
-                else hipLaunchKernelGGL((sphere_build_kernel<T, 1, 1, false>), grid, blk, 0, nullptr, a);
+                hipLaunchKernelGGL((sphere_build_kernel<T, 1, 1, F>), tg, blk, 0, nullptr, a);
+                if (slots) hipLaunchKernelGGL((sphere_slots_kernel<T, 1, 1, F>), sgr, blk, 0, nullptr, s, mask);
             }
             QG_HIP(hipGetLastError());
         };
-        // the projection's lists (a word of the masks holds 32 slots; more: the other projections serve)
-        auto build_slots = [&](SphereGeo* o, BuildArgs b) {
-            const int nep = (nz + kProjPlanes - 1) / kProjPlanes;
-            const size_t ne = (size_t)o->ntile * nep * nw;
-            std::vector<int> cnt(ne + 1, 0);
-            o->d_slot_off.alloc(ne + 1);
-            o->d_slot_mask.alloc(ne * kProjPlanes);
-            b.trips = o->d_slot_off.p;
-            auto go = [&](auto tag, bool fill) {
-                using T = decltype(tag);
-                const dim3 grid(o->ntile, nep), blk(o->tpb);
-                if (two) {
-                    if (fill) hipLaunchKernelGGL((sphere_slots_kernel<T, 2, 2, true>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
-                    else hipLaunchKernelGGL((sphere_slots_kernel<T, 2, 2, false>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
-                } else {
-                    if (fill) hipLaunchKernelGGL((sphere_slots_kernel<T, 1, 1, true>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
-                    else hipLaunchKernelGGL((sphere_slots_kernel<T, 1, 1, false>), grid, blk, 0, nullptr, b, o->d_slot_mask.p);
-                }
-                QG_HIP(hipGetLastError());
-            };
-            dtype == QG_F32 ? go(float{}, false) : go(double{}, false);
-            QG_HIP(hipMemcpy(cnt.data(), o->d_slot_off.p, ne * sizeof(int), hipMemcpyDeviceToHost));
+        dtype == QG_F32 ? build(float{}, std::false_type{}, true) : build(double{}, std::false_type{}, true);
+        QG_HIP(hipMemcpy(cnt.data(), c->counts.p, cnt.size() * sizeof(int), hipMemcpyDeviceToHost));
+        // counts -> offsets; a word of the masks holds 32 slots (more: the other projections serve)
+        auto scan = [](int* v, size_t n, int& most) {
             int64_t sum = 0;
-            int most = 0;
-            for (size_t k = 0; k <= ne; ++k) {
-                const int n = k < ne ? cnt[k] : 0;
-                cnt[k] = (int)std::min<int64_t>(sum, INT32_MAX);
-                sum += n;
-                most = std::max(most, n);
+            for (size_t k = 0; k <= n; ++k) {
+                const int m = k < n ? v[k] : 0;
+                v[k] = (int)std::min<int64_t>(sum, INT32_MAX);
+                sum += m;
+                most = std::max(most, m);
             }
-            const int nv = nl->sphere_form.ns + nl->sphere_form.np;
-            if (most > 32 || sum >= (1LL << 28)) return;
-            const size_t slots = (size_t)std::max<int64_t>(1, sum);
-            o->d_slot_off.upload(cnt.data(), cnt.size());
-            o->d_slot_words.alloc(slots * 64);
-            o->d_slot_vals.alloc(slots * kProjPlanes * 64 * nv * 16);
-            b.trip_off = o->d_slot_off.p;
-            b.words = o->d_slot_words.p;
-            b.vals = o->d_slot_vals.p;
-            dtype == QG_F32 ? go(float{}, true) : go(double{}, true);
-            o->slots_ok = true;
+            return sum;
         };
-        dtype == QG_F32 ? launch(float{}, false) : launch(double{}, false);
-        QG_HIP(hipMemcpy(trips.data(), c->d_trip_off.p, nwv * sizeof(int), hipMemcpyDeviceToHost));
-        int64_t total = 0;
-        for (size_t k = 0; k <= nwv; ++k) {
-            const int n = k < nwv ? trips[k] : 0;
-            trips[k] = (int)std::min<int64_t>(total, INT32_MAX);
-            total += n;
-        }
-        const int nv = nl->sphere_form.ns + nl->sphere_form.np;
-        if (total < (1LL << 30)) {
-            c->ntrips = (int)std::max<int64_t>(1, total);
-            c->d_trip_off.upload(trips.data(), trips.size());
-            c->d_words.alloc((size_t)c->ntrips * 64);
-            c->d_vals.alloc((size_t)c->ntrips * 64 * nv * 16);
-            a.trip_off = c->d_trip_off.p;
-            a.words = c->d_words.p;
-            a.vals = c->d_vals.p;
-            dtype == QG_F32 ? launch(float{}, true) : launch(double{}, true);
+        int most_trips = 0, most_slots = 0;
+        const int64_t trips = scan(cnt.data(), nwv, most_trips), slots = scan(cnt.data() + nwv + 1, ne, most_slots);
+        if (trips < (1LL << 30)) {
+            const size_t nv = nl->sphere_form.ns + nl->sphere_form.np;
+            c->slots_ok = most_slots <= 32 && slots < (1LL << 28);
+            c->ntrips = (int)std::max<int64_t>(1, trips);
+            const size_t nt = c->ntrips, ns = c->slots_ok ? (size_t)std::max<int64_t>(1, slots) : 0;
+            QG_HIP(hipMemcpyAsync(c->counts.p, cnt.data(), cnt.size() * sizeof(int), hipMemcpyHostToDevice, nullptr));
+            c->lists.alloc(1024 * nv * (nt + ns * kProjPlanes) + 256 * (nt + ns));
+            unsigned char* v = c->lists.p;
+            c->vals = v;
+            c->slot_vals = v + 1024 * nv * nt;
+            uint32_t* w = reinterpret_cast<uint32_t*>(v + 1024 * nv * (nt + ns * kProjPlanes));
+            c->words = w;
+            c->slot_words = w + 64 * nt;
+            a.trip_off = c->trip_off;
+            a.words = w;
+            a.vals = v;
+            s.trip_off = c->slot_off;
+            s.words = w + 64 * nt;
+            s.vals = v + 1024 * nv * nt;
+            dtype == QG_F32 ? build(float{}, std::true_type{}, c->slots_ok) : build(double{}, std::true_type{}, c->slots_ok);
             c->ok = true;
-            build_slots(c.get(), a);
         }
         QG_HIP(hipStreamSynchronize(nullptr));
     }
@@ -1403,7 +1395,8 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
 }
 
 // Device state of the geometry just built into nl, with the entry lists of the default tile
-// heights (so that applications on caller scratch need not allocate).
+// heights where the allocation-free application may need them (other lists are built at their first
+// use).
 void sphere_prepare(qg_nonlocal* nl) {
     nl->sphere.clear();
     sphere_images(nl);
@@ -1411,7 +1404,7 @@ void sphere_prepare(qg_nonlocal* nl) {
     for (int dtype : {QG_F32, QG_F64}) {
         const int VN = dtype == QG_F32 ? 4 : 2;
         const int ty = sphere_pick_ty((nl->gcopy.n[0] + VN - 1) / VN, nl->gcopy.n[1], 0);
-        if (ty > 0) sphere_geometry(nl, dtype, ty, true);
+        if (ty > 0 && rows_serve(nl, dtype)) sphere_geometry(nl, dtype, ty, true);
     }
 }
 
@@ -1484,11 +1477,11 @@ static SphereArgs sphere_args(const qg_nonlocal* nl, const SphereGeo& sg, int nb
     a.tz = want_tz > 0 ? std::min(g.n[2], want_tz) : (g.n[2] + nslab - 1) / nslab;
     a.nslab = (g.n[2] + a.tz - 1) / a.tz;
     a.nbands = nbands;
-    a.col_off = sg.d_col_off.p; a.col_img = sg.d_col_img.p;
+    a.col_off = sg.col_off; a.col_img = sg.col_img;
     a.images = nl->d_sphere_img.p;
-    a.trip_off = sg.d_trip_off.p;
+    a.trip_off = sg.trip_off;
     a.ntrips = sg.ntrips;
-    a.vals = sg.d_vals.p; a.words = sg.d_words.p;
+    a.vals = sg.vals; a.words = sg.words;
     a.coef_energy = nl->d_coef_energy.p; a.atom_coef_off = nl->d_atom_coef_off.p;
     a.atom_chan = nl->d_atom_chan.p;
     a.ncoef = nl->geo.ncoef;
@@ -1577,10 +1570,10 @@ static bool sphere_project_t(qg_nonlocal* nl, int nbands, const T* psi, int64_t 
     a.ty = sg.ty; a.tz = sh.tz; a.ntile = sg.ntile; a.nslab = sh.nslab; a.nbands = nbands;
     a.nq = sg.nq; a.tpb = sg.tpb; a.nw = sg.tpb / 64;
     a.ld = cplx ? 2 * ld : ld;
-    a.col_off = sg.d_col_off.p; a.col_img = sg.d_col_img.p; a.images = nl->d_sphere_img.p;
+    a.col_off = sg.col_off; a.col_img = sg.col_img; a.images = nl->d_sphere_img.p;
     a.nepoch = (g.n[2] + kProjPlanes - 1) / kProjPlanes;
-    a.slot_off = sg.d_slot_off.p; a.mask = sg.d_slot_mask.p;
-    a.vals = sg.d_slot_vals.p; a.words = sg.d_slot_words.p;
+    a.slot_off = sg.slot_off; a.mask = sg.slot_mask;
+    a.vals = sg.slot_vals; a.words = sg.slot_words;
     a.max_col = std::max(1, sg.max_col);
     for (int d = 0; d < 3; ++d) a.h[d] = g.h[d];
     a.part = part;
@@ -1607,7 +1600,7 @@ static bool sphere_project_t(qg_nonlocal* nl, int nbands, const T* psi, int64_t 
     QG_REQUIRE(rgrid.y <= 65535, "too many bands in one projection");
     auto reduce = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, rgrid, dim3(256), 0, s, part, sh.nslab, a.max_col, nl->sphere_form.ns,
-                           nl->sphere_form.np, nbands, sg.d_atom_ref_off.p, sg.d_atom_ref.p, a.col_off, a.col_img,
+                           nl->sphere_form.np, nbands, sg.atom_ref_off, sg.atom_ref, a.col_off, a.col_img,
                            a.images, nl->d_atom_chan.p, nl->d_atom_coef_off.p, ph, g.dvol(), coef, nl->geo.ncoef);
     };
     if (cplx) reduce(sphere_coef_reduce_kernel<true>);
@@ -1687,8 +1680,8 @@ static bool sphere_force_t(qg_nonlocal* nl, int nocc, const int* band_idx, const
         if (nb == 2) sphere_force_launch<T, 2, 1, 1>(a, sc, psi, lds, s);
         else sphere_force_launch<T, 1, 1, 1>(a, sc, psi, lds, s);
     }
-    hipLaunchKernelGGL(sphere_force_reduce_kernel, dim3(nl->geo.natoms), dim3(256), 0, s, a.part, sg->d_atom_ref_off.p,
-                       sg->d_atom_ref.p, per_tile, a.max_col, force);
+    hipLaunchKernelGGL(sphere_force_reduce_kernel, dim3(nl->geo.natoms), dim3(256), 0, s, a.part, sg->atom_ref_off,
+                       sg->atom_ref, per_tile, a.max_col, force);
     QG_HIP(hipGetLastError());
     return true;
 }
