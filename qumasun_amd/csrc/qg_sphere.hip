@@ -363,9 +363,8 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                     d[i] = sc.cz[3] * (qb[8].v[i] - qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] - qb[1].v[i]) +
                            sc.cz[1] * (qb[6].v[i] - qb[2].v[i]) + sc.cz[0] * (qb[5].v[i] - qb[3].v[i]);
                 else
-                    d[i] = sc.c0 * qb[4].v[i];
-                if constexpr (!FORCE) d[i] += sc.cz[3] * (qb[8].v[i] + qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] + qb[1].v[i]) +
-                        sc.cz[1] * (qb[6].v[i] + qb[2].v[i]) + sc.cz[0] * (qb[5].v[i] + qb[3].v[i]);
+                    d[i] = sc.cz[3] * (qb[8].v[i] + qb[0].v[i]) + sc.cz[2] * (qb[7].v[i] + qb[1].v[i]) +
+                           sc.cz[1] * (qb[6].v[i] + qb[2].v[i]) + sc.cz[0] * (qb[5].v[i] + qb[3].v[i]);
             }
             {
                 T xsv[VN + 8];
@@ -419,7 +418,8 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                     gz[b].v[i] = mine ? d[i] : T(0);
                     if (!mine) res[b].v[i] = T(0);
                 } else {
-                    res[b].v[i] = vcur.v[i] * qb[4].v[i] + d[i];
+                    // the large centre term last: the sums before it round at their own size
+                    res[b].v[i] = vcur.v[i] * qb[4].v[i] + (sc.c0 * qb[4].v[i] + d[i]);
                 }
             }
             // one band's LDS values live at a time
@@ -1218,7 +1218,6 @@ static SphereForm sphere_form(const NlGeometry& geo, std::vector<int>& chan) {
 }
 
 bool sphere_serves(const qg_grid& g, const qg_nonlocal* nl) {
-    if (env_int("QG_SPHERE", 1) == 0) return false;
     if (g.n[0] < 8 || g.n[0] > 1024 || g.n[2] < 8) return false;
     if (g.ng() * 8 > (int64_t)kOOB - 64) return false;   // band bytes below the out-of-range offset
     return nl->geo.ncoef > 0 && !nl->geo.images.empty() && nl->sphere_form.ns > 0;
