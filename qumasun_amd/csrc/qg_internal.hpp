@@ -352,7 +352,12 @@ struct qg_ham {
     qg::DevBuf<double> rows_part;  // projector partials of the row path
     qg::DevBuf<double> rows_coef;  // projector coefficients of the row path
     int tchunks = 0;
+    hipStream_t side = nullptr;    // second stream of a batch this handle leads a share of
+    hipEvent_t side_ev[2] = {};
     ~qg_ham() {
+        for (auto& e : side_ev)
+            if (e) (void)hipEventDestroy(e);
+        if (side) (void)hipStreamDestroy(side);
         for (auto& e : tev)
             if (e) (void)hipEventDestroy(e);
         if (lobpcg) qg::lobpcg_state_free(lobpcg);
