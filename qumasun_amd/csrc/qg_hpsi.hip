@@ -1367,7 +1367,7 @@ static bool sphere_cell(const BatchReq& r, int dtype, hipStream_t s) {
 // The batch as one H psi per cell, the cells dealt over the caller's stream and one of the first
 // handle of the second share (largest cell first, each to the share with the least work so far): the
 // sphere passes of a small cell leave most of the chip idle, and two of them run side by side.
-// Returns with the work done.  8 uneven cells (16-128 FP32 bands, 40^3-80^3): 577 us against 1033 us
+// Returns with the work done.  8 uneven cells (16-128 FP32 bands, 40^3-80^3): 543 us against 1034 us
 // for the persistent table-kernel launches; all on one stream 732 us, on four 660 us.
 static void batch_streams_apply(std::vector<BatchReq> reqs, int dtype, hipStream_t s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

@@ -324,6 +324,8 @@ void sphere_prepare(qg_nonlocal* nl);
 bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
                               int64_t ld_out, const double* coef, bool may_build, bool run, hipStream_t s);
 bool sphere_prepared(qg_nonlocal* nl, int dtype);
+bool sphere_kpoint_apply(qg_ham* h, const double* k, int dtype, int nbands, const void* psi, int64_t ld, void* out,
+                         int64_t ld_out, DevBuf<double>& part, double* coef, hipStream_t s);
 size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build);
 bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, const double* k, double* part,
                     double* coef, bool may_build, hipStream_t s);

@@ -65,6 +65,7 @@ struct qg_kpoint {
     qg::DevBuf<double2> phase64;
     qg::DevBuf<float2> phase32;
     qg::DevBuf<double2> coef;   // projector coefficients [nb][ncoef]
+    qg::DevBuf<double> part;    // projector partials of the sphere lists
     // the projector table entries of every grid point (CSR over grid points): entries of point
     // g are pt_ent[pt_off[g] .. pt_off[g+1]), each a table point and its atom's first coefficient
     qg::DevBuf<int> pt_off, pt_ent, pt_cb;
@@ -509,6 +510,14 @@ template <class T>
 void kpoint_apply(qg_kpoint* kp, int nbands, const void* psi, int64_t ld, void* out, int64_t ld_out, hipStream_t s) {
     qg_ham* h = kp->h;
     const qg_grid& g = h->grid;
+    // projection and one fused apply pass where the sphere entry lists serve
+    if (h->nl && h->nl->geo.ncoef > 0) {
+        QG_REQUIRE(h->nl->geo.max_coef_per_atom <= 8, "k-point projectors: at most 8 coefficients per atom");
+        kp->coef.alloc((size_t)nbands * h->nl->geo.ncoef);
+        if (sphere_kpoint_apply(h, kp->k, sizeof(T) == 4 ? QG_F32 : QG_F64, nbands, psi, ld, out, ld_out, kp->part,
+                                reinterpret_cast<double*>(kp->coef.p), s))
+            return;
+    }
     const double coef = -0.5;
     KStencil<T> ks;
     const double k2 = kp->k[0] * kp->k[0] + kp->k[1] * kp->k[1] + kp->k[2] * kp->k[2];
@@ -982,7 +991,11 @@ int qg_kpoint_create(qg_ham* h, double kx, double ky, double kz, qg_kpoint** out
         kp->k[1] = ky;
         kp->k[2] = kz;
         try {
-            build_phases(kp);
+            // the sphere lists of both precisions, or the phase tables of the table kernels
+            bool lists = h->nl && h->nl->geo.ncoef > 0;
+            for (int dtype : {QG_F32, QG_F64})
+                lists = lists && sphere_kpoint_apply(h, kp->k, dtype, 0, nullptr, 0, nullptr, 0, kp->part, nullptr, nullptr);
+            if (!lists) build_phases(kp);
         } catch (...) {
             delete kp;
             throw;

@@ -945,8 +945,9 @@ __global__ __launch_bounds__(256) void sphere_coef_reduce_kernel(
             if constexpr (CPLX) {
                 const SphereImage& g = images[col_img[col_off[ref.x] + ref.y]];
                 const double sr = p[2 * b], si = p[2 * b + 1];
-                double sn, cs;
-                sincos(-(ph.kh[0] * g.shift[0] + ph.kh[1] * g.shift[1] + ph.kh[2] * g.shift[2]), &sn, &cs);
+                double sn = 0.0, cs = 1.0;
+                if (g.shift[0] | g.shift[1] | g.shift[2])
+                    sincos(-(ph.kh[0] * g.shift[0] + ph.kh[1] * g.shift[1] + ph.kh[2] * g.shift[2]), &sn, &cs);
                 re += cs * sr - sn * si;
                 im += cs * si + sn * sr;
             } else {
@@ -963,6 +964,372 @@ __global__ __launch_bounds__(256) void sphere_coef_reduce_kernel(
 #pragma unroll
     for (int w = 0; w < W; ++w)
         coef[W * o + w] = dv * (((red[0][lb][w] + red[1][lb][w]) + red[2][lb][w]) + red[3][lb][w]);
+}
+
+// -------------------------------------------------------------------------- k points ----
+// H_k u = coef [L8 - |k|^2 + 2 i k . D8] u + V u + sum_j E_j conj(P_j) c_j for one complex band per
+// workgroup (re, im interleaved), the structure of sphere_body with the two parts in place of two
+// bands: a part of a point is a fixed element of the lane's two 16-byte vectors, so the z-queue holds
+// the block's own layout; LDS holds the parts in separate planes.
+// The phase of P_j = beta_j exp(i k.x_u), x_u the image-frame coordinate, is the grid point's
+// exp(i k.h i) times the image's exp(-i k.h shift): the second sits in the staged E c, the first is
+// applied once per point to the sum over its images.
+// One pass replaces stencil, projection gather and their read-modify-write: 64 atoms, 80^3, 64
+// complex128 bands 465 us against 398 (stencil) + 347 (gather); occupancy (two halves of the
+// z-queue, ~200 VGPRs) and L2 traffic of halo rows and lists bound it.
+template <class T>
+struct SphereKStencil {
+    T c0;
+    T a[3][4], b[3][4];     // second- and first-difference weights of offsets 1..4
+};
+
+template <class T>
+static size_t sphere_kpoint_lds(int nx, int ty, int tz, int ns, int np, int max_col) {
+    return sphere_lds<T>(nx, ty, 2, ns, np, max_col) + sizeof(T) * 2 * (size_t)tz;
+}
+
+template <class T, int NS, int NP, bool RAG, int HV>
+__global__ __launch_bounds__(kMaxThreads) void sphere_kpoint_kernel(SphereArgs a, SphereKStencil<T> ks, SpherePhase ph,
+                                                                    const T* __restrict__ V, const T* __restrict__ psi,
+                                                                    T* __restrict__ out) {
+    constexpr int VN = 16 / sizeof(T);
+    constexpr int S = sizeof(T);
+    constexpr int NC = NS + 3 * NP;
+    constexpr int NV = NS + NP;
+    constexpr int K = 3;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const int W = RAG ? (nx + 8 + VN - 1) / VN * VN : nx + 8;
+    const int ty = a.ty;
+    const int lband = (ty + 8) * W;
+    const int nthr = a.tpb;
+    T* planes = reinterpret_cast<T*>(smem);                    // [2][re, im][ty + 8][W]
+    T* imf = planes + (size_t)4 * lband;                       // [max_col + 1][4]
+    T* ec = imf + (size_t)(a.max_col + 1) * 4;                 // [max_col + 1][re, im][NC]
+    T* ez = ec + (size_t)(a.max_col + 1) * 2 * NC;             // [tz][2]
+
+    const int wg = xcd_order(blockIdx.x, gridDim.x);
+    const int grp = wg / (a.tg * a.nbands * a.nslab);
+    const int in_grp = wg - grp * (a.tg * a.nbands * a.nslab);
+    const int tgw = min(a.tg, a.ntile - grp * a.tg);
+    const int tile = grp * a.tg + in_grp % tgw;
+    const int rest = in_grp / tgw;
+    const int slab = rest / a.nbands;
+    const int band = rest - slab * a.nbands;
+    const int y0 = tile * ty;
+    const int rows = min(ty, ny - y0);
+    const int z0 = slab * a.tz, z1 = min(z0 + a.tz, nz);
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int nq = a.nq;
+    const int r = tid / nq, xq = tid - r * nq;
+    const int x = RAG ? min(xq * VN, nx - VN) : xq * VN;
+    const bool own = r < rows;
+    const int plane = nx * ny;
+    const uint32_t v_bytes = (uint32_t)((int64_t)plane * nz * S);
+    const rsrc_t rin = rsrc(psi + (int64_t)band * a.ld_in, 2 * v_bytes);
+    const rsrc_t rout = rsrc(out + (int64_t)band * a.ld_out, 2 * v_bytes);
+    const rsrc_t rv = rsrc(V, v_bytes);
+    const int pt = (y0 + r) * nx + x;
+    const int vo = own ? pt * S : kOOB;                        // V
+    const int vc[2] = {own ? 2 * pt * S : kOOB, own ? 2 * pt * S + 16 : kOOB};
+    const int lc = (r + 4) * W + 4 + x;
+    const int lw = (x < 4) ? lc + nx : ((x >= nx - 4) ? lc - nx : -1);
+    int ho[HV][2], hl[HV];
+#pragma unroll
+    for (int k = 0; k < HV; ++k) {
+        const int v = tid + k * nthr;
+        ho[k][0] = ho[k][1] = kOOB;
+        hl[k] = -1;
+        if (v < 8 * nq) {
+            const int hr = v / nq, hq = v - hr * nq;
+            const int hx = RAG ? min(hq * VN, nx - VN) : hq * VN;
+            int gy = (hr < 4) ? y0 - 4 + hr : y0 + rows + (hr - 4);
+            gy = ((gy % ny) + ny) % ny;
+            ho[k][0] = 2 * (gy * nx + hx) * S;
+            ho[k][1] = ho[k][0] + 16;
+            hl[k] = ((hr < 4) ? hr : rows + hr) * W + 4 + hx;
+        }
+    }
+    auto wrapz = [&](int z) { return (z < 0 ? z + nz : (z >= nz ? z - nz : z)) * plane * S; };
+    const T hx = (T)a.h[0], hy = (T)a.h[1], hz = (T)a.h[2];
+
+    const int c0 = a.col_off[tile];
+    const int ncol = a.col_off[tile + 1] - c0;
+    for (int li = tid; li <= ncol; li += nthr) {
+        const SphereImage* im = a.images + a.col_img[c0 + max(min(li, ncol - 1), 0)];
+        const bool ok = li < ncol;
+        imf[4 * li] = ok ? (T)im->f[0] : T(0);
+        imf[4 * li + 1] = ok ? (T)im->f[1] : T(0);
+        imf[4 * li + 2] = ok ? (T)im->f[2] : T(0);
+        imf[4 * li + 3] = ok ? (T)im->n[2] : T(0);
+    }
+    for (int i = tid; i < (ncol + 1) * NC; i += nthr) {
+        const int li = i / NC, j = i % NC;
+        double er = 0.0, ei = 0.0;
+        if (li < ncol) {
+            const SphereImage& im = a.images[a.col_img[c0 + li]];
+            const int slot = a.atom_chan[4 * im.atom + (j < NS ? j : 2 + (j - NS) / 3)];
+            if (slot >= 0) {
+                const int cb = a.atom_coef_off[im.atom] + slot + (j < NS ? 0 : (j - NS) % 3);
+                const double e = a.coef_energy[cb];
+                const double cr = e * a.coef[2 * ((int64_t)band * a.ncoef + cb)];
+                const double ci = e * a.coef[2 * ((int64_t)band * a.ncoef + cb) + 1];
+                double sn, cs;
+                sincos(ph.kh[0] * im.shift[0] + ph.kh[1] * im.shift[1] + ph.kh[2] * im.shift[2], &sn, &cs);
+                er = cr * cs - ci * sn;
+                ei = cr * sn + ci * cs;
+            }
+        }
+        ec[(size_t)li * 2 * NC + j] = (T)er;
+        ec[(size_t)li * 2 * NC + NC + j] = (T)ei;
+    }
+    for (int i = tid; i < z1 - z0; i += nthr) {
+        double s, c;
+        sincos(ph.kh[2] * (double)(z0 + i), &s, &c);
+        ez[2 * i] = (T)c;
+        ez[2 * i + 1] = (T)s;
+    }
+    T exy[VN][2];
+#pragma unroll
+    for (int u = 0; u < VN; ++u) {
+        double s, c;
+        sincos(ph.kh[0] * (double)(x + u) + ph.kh[1] * (double)(y0 + r), &s, &c);
+        exy[u][0] = (T)c;
+        exy[u][1] = (T)s;
+    }
+
+    // part c of point u of a pair of vectors
+#define QG_PART(pair, c, u) ((pair)[(2 * (u) + (c)) / VN].v[(2 * (u) + (c)) % VN])
+    struct Pair {
+        Row<T> h[2];
+    };
+    Pair q[11];     // the z-queue of sphere_body
+    auto load_pair = [&](const int (&off)[2], int zo) {
+        Pair p;
+        p.h[0] = vload<T>(rin, off[0], 2 * zo);
+        p.h[1] = vload<T>(rin, off[1], 2 * zo);
+        return p;
+    };
+#pragma unroll
+    for (int d = 0; d < 9; ++d) q[d] = load_pair(vc, wrapz(z0 - 4 + d));
+    Pair hn[HV];
+    Row<T> vn;
+    auto load_halo = [&](int z) {
+        vn = vload<T>(rv, vo, wrapz(z));
+#pragma unroll
+        for (int k = 0; k < HV; ++k) hn[k] = load_pair(ho[k], wrapz(z));
+    };
+    load_halo(z0);
+    struct Entry {
+        Row<T> f[NV];
+        uint32_t w;
+    };
+    Entry en[K];
+    const int* toff = a.trip_off + (size_t)tile * nz * a.nw + wave;
+    int tb, n;
+    auto load_entry = [&](rsrc_t rvals, rsrc_t rwords, int k) {
+        Entry e;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) e.f[v] = vload<T>(rvals, lane * 16, (k * NV + v) * 1024);
+        e.w = __builtin_amdgcn_raw_buffer_load_b32(rwords, lane * 4, k * 256, 0);
+        return e;
+    };
+    auto load_entries = [&](int z) {
+        tb = __builtin_amdgcn_readfirstlane(toff[(size_t)z * a.nw]);
+        n = __builtin_amdgcn_readfirstlane(toff[(size_t)z * a.nw + 1]) - tb;
+        const rsrc_t rvals = rsrc((const unsigned char*)a.vals + (int64_t)tb * NV * 1024, (uint32_t)n * NV * 1024);
+        const rsrc_t rwords = rsrc(a.words + (int64_t)tb * 64, (uint32_t)n * 256);
+#pragma unroll
+        for (int k = 0; k < K; ++k) en[k] = load_entry(rvals, rwords, k);
+    };
+    load_entries(z0);
+    auto stage = [&](T* L, int at, const Pair& p, int c) __attribute__((always_inline)) {
+        if constexpr (!RAG) {
+            Row<T> w;
+#pragma unroll
+            for (int u = 0; u < VN; ++u) w.v[u] = QG_PART(p.h, c, u);
+            *reinterpret_cast<Row<T>*>(L + at) = w;
+        } else {
+#pragma unroll
+            for (int u = 0; u < VN; ++u) L[at + u] = QG_PART(p.h, c, u);
+        }
+    };
+
+    auto step = [&](auto kc, int z) __attribute__((always_inline)) {
+        constexpr int k0 = decltype(kc)::value;
+        T* Lp = planes + (size_t)((z - z0) & 1) * 2 * lband;
+        const int zn = min(z + 1, z1 - 1);
+        const Row<T> vcur = vn;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            T* Lb = Lp + c * lband;
+            if (own) {
+                stage(Lb, lc, q[k0 + 4], c);
+                if constexpr (!RAG) {
+                    if (lw >= 0) stage(Lb, lw, q[k0 + 4], c);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) {
+                        if (x + u < 4) Lb[lc + u + nx] = QG_PART(q[k0 + 4].h, c, u);
+                        if (x + u >= nx - 4) Lb[lc + u - nx] = QG_PART(q[k0 + 4].h, c, u);
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < HV; ++k)
+                if (hl[k] >= 0) stage(Lb, hl[k], hn[k], c);
+        }
+        q[k0 < 2 ? k0 + 9 : 0] = load_pair(vc, wrapz(z + 5));
+        load_halo(zn);
+        __syncthreads();
+
+        // the stencil: d[c] collects part c; a first difference of one part enters the other
+        T d[2][VN];
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) d[c][u] = T(0);
+#pragma unroll
+            for (int m = 3; m >= 0; --m)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const T up = QG_PART(q[k0 + 5 + m].h, c, u), dn = QG_PART(q[k0 + 3 - m].h, c, u);
+                    d[c][u] += ks.a[2][m] * (up + dn);
+                    d[1 - c][u] += (c == 0 ? ks.b[2][m] : -ks.b[2][m]) * (up - dn);
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const T* Lc = Lp + c * lband + (own ? (r + 4) * W + x : 4 * W);   // Lc[4 + i] is point x + i
+            T xsv[VN + 8];
+            if constexpr (!RAG) {
+#pragma unroll
+                for (int k = 0; k < (VN + 8) / VN; ++k) {
+                    const Row<T> w = *reinterpret_cast<const Row<T>*>(Lc + k * VN);
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) xsv[k * VN + u] = w.v[u];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < VN + 8; ++k) xsv[k] = Lc[k];
+            }
+#pragma unroll
+            for (int u = 0; u < VN; ++u)
+#pragma unroll
+                for (int m = 3; m >= 0; --m) {
+                    d[c][u] += ks.a[0][m] * (xsv[u + 5 + m] + xsv[u + 3 - m]);
+                    d[1 - c][u] += (c == 0 ? ks.b[0][m] : -ks.b[0][m]) * (xsv[u + 5 + m] - xsv[u + 3 - m]);
+                }
+#pragma unroll
+            for (int m = 3; m >= 0; --m) {
+                Row<T> ym, yp;
+                if constexpr (!RAG) {
+                    ym = *reinterpret_cast<const Row<T>*>(Lc + 4 - (m + 1) * W);
+                    yp = *reinterpret_cast<const Row<T>*>(Lc + 4 + (m + 1) * W);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < VN; ++i) {
+                        ym.v[i] = Lc[4 + i - (m + 1) * W];
+                        yp.v[i] = Lc[4 + i + (m + 1) * W];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < VN; ++u) {
+                    d[c][u] += ks.a[1][m] * (yp.v[u] + ym.v[u]);
+                    d[1 - c][u] += (c == 0 ? ks.b[1][m] : -ks.b[1][m]) * (yp.v[u] - ym.v[u]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            const T cv = ks.c0 + vcur.v[u];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) d[c][u] += cv * QG_PART(q[k0 + 4].h, c, u);
+        }
+        // keep the stencil here: moved behind the projector term it would hold its operands for it
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int u = 0; u < VN; ++u) asm volatile("" : "+v"(d[c][u]));
+
+        T nl[2][VN];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int u = 0; u < VN; ++u) nl[c][u] = T(0);
+        auto trip = [&](const Entry& e) __attribute__((always_inline)) {
+            const int li = (int)(e.w & 1023u);
+            const int dyi = ((int)(e.w << 11)) >> 21, dxi = ((int)e.w) >> 21;
+            const T* im = imf + 4 * li;
+            T fx, fy, fz, nzf;
+            if constexpr (VN == 4) {
+                const Row<T> w = *reinterpret_cast<const Row<T>*>(im);
+                fx = w.v[0]; fy = w.v[1]; fz = w.v[2]; nzf = w.v[3];
+            } else {
+                const Row<T> w0 = *reinterpret_cast<const Row<T>*>(im), w1 = *reinterpret_cast<const Row<T>*>(im + 2);
+                fx = w0.v[0]; fy = w0.v[1]; fz = w1.v[0]; nzf = w1.v[1];
+            }
+            const T dx0 = hx * ((T)dxi - fx), dy = hy * ((T)dyi - fy), dz = hz * (((T)z - nzf) - fz);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                T c[NC];
+                const Row<T>* ep = reinterpret_cast<const Row<T>*>(ec + ((size_t)li * 2 + b) * NC);
+#pragma unroll
+                for (int k = 0; k < NC / VN; ++k) {
+                    const Row<T> w = ep[k];
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) c[k * VN + u] = w.v[u];
+                }
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) nl[b][u] += e.f[s].v[u] * c[s];
+#pragma unroll
+                for (int p = 0; p < NP; ++p) {
+                    const T ayz = c[NS + 3 * p] * dy + c[NS + 3 * p + 1] * dz;
+#pragma unroll
+                    for (int u = 0; u < VN; ++u)
+                        nl[b][u] += e.f[NS + p].v[u] * (ayz + c[NS + 3 * p + 2] * (dx0 + (T)u * hx));
+                }
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (k < n) trip(en[k]);
+        if (n > K) {
+            const rsrc_t rvals = rsrc((const unsigned char*)a.vals + (int64_t)tb * NV * 1024, (uint32_t)n * NV * 1024);
+            const rsrc_t rwords = rsrc(a.words + (int64_t)tb * 64, (uint32_t)n * 256);
+            for (int k = K; k < n; ++k) trip(load_entry(rvals, rwords, k));
+        }
+        load_entries(zn);
+        // conj(phase) of the point times the sum of its images
+        const T cz = ez[2 * (z - z0)], sz = ez[2 * (z - z0) + 1];
+        Pair o;
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            const T er = exy[u][0] * cz - exy[u][1] * sz, ei = exy[u][0] * sz + exy[u][1] * cz;
+            QG_PART(o.h, 0, u) = d[0][u] + (er * nl[0][u] + ei * nl[1][u]);
+            QG_PART(o.h, 1, u) = d[1][u] + (er * nl[1][u] - ei * nl[0][u]);
+        }
+        vstore<T>(rout, o.h[0], vc[0], 2 * wrapz(z));
+        vstore<T>(rout, o.h[1], vc[1], 2 * wrapz(z));
+    };
+    for (int z = z0;;) {
+        step(std::integral_constant<int, 0>{}, z);
+        if (++z >= z1) break;
+        step(std::integral_constant<int, 1>{}, z);
+        if (++z >= z1) break;
+        step(std::integral_constant<int, 2>{}, z);
+        if (++z >= z1) break;
+        const Pair next = q[0];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) q[d] = q[d + 3];
+        q[8] = next;
+    }
+#undef QG_PART
 }
 
 // ------------------------------------------------------------------ entry lists ----
@@ -1195,6 +1562,14 @@ static int sphere_pick_ty(int nq, int ny, int want) {
         if (score > bests) { bests = score; best = ty; }
     }
     return best;
+}
+
+// Tile rows of the complex passes: 4 wavefronts where that leaves 6 rows or more (two workgroups of
+// ~175 VGPRs a CU instead of one: 64 atoms, 80^3, 64 complex128 bands 709 us with 6 rows, 812 with 12),
+// the real passes' height otherwise
+static int sphere_kpoint_ty(int nq, int ny) {
+    const int four = std::min(ny, 256 / std::max(1, nq));
+    return four >= 6 && four < sphere_pick_ty(nq, ny, 0) ? four : sphere_pick_ty(nq, ny, 0);
 }
 
 static SphereForm sphere_form(const NlGeometry& geo, std::vector<int>& chan) {
@@ -1508,7 +1883,7 @@ static bool sphere_proj_shape(qg_nonlocal* nl, int nbands, bool cplx, bool may_b
     if (cplx && g.ng() * 16 > (int64_t)kOOB - 64) return false;   // band bytes below the out-of-range offset
     constexpr int VN = 16 / sizeof(T);
     const int nq = (g.n[0] + VN - 1) / VN;
-    const int ty = sphere_pick_ty(nq, g.n[1], 0);
+    const int ty = cplx ? sphere_kpoint_ty(nq, g.n[1]) : sphere_pick_ty(nq, g.n[1], 0);
     sh.sg = ty > 0 ? sphere_geometry(nl, sizeof(T) == 4 ? QG_F32 : QG_F64, ty, may_build) : nullptr;
     if (!sh.sg || !sh.sg->slots_ok) return false;
     const int nc = nl->sphere_form.ns + 3 * nl->sphere_form.np;
@@ -1749,6 +2124,76 @@ bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi,
                                      run, s);
     return sphere_apply_t<double>(h, nbands, (const double*)psi, ld, (double*)hpsi, ld_out, coef, may_build,
                                   run, s);
+}
+
+template <class T, int NS, int NP>
+static void sphere_kpoint_launch(const SphereArgs& a, const SphereKStencil<T>& ks, const SpherePhase& ph, const T* V,
+                                 const T* psi, T* out, size_t lds, int hv, hipStream_t s) {
+    const int64_t nwg = (int64_t)a.ntile * a.nslab * a.nbands;
+    QG_REQUIRE(nwg < (1LL << 31), "too many workgroups");
+    const dim3 grid((unsigned)nwg), blk(a.tpb);
+    const bool rag = a.nx % (16 / (int)sizeof(T)) != 0;
+    if (hv <= 1) {
+        if (rag) hipLaunchKernelGGL((sphere_kpoint_kernel<T, NS, NP, true, 1>), grid, blk, lds, s, a, ks, ph, V, psi, out);
+        else hipLaunchKernelGGL((sphere_kpoint_kernel<T, NS, NP, false, 1>), grid, blk, lds, s, a, ks, ph, V, psi, out);
+    } else {
+        if (rag) hipLaunchKernelGGL((sphere_kpoint_kernel<T, NS, NP, true, 2>), grid, blk, lds, s, a, ks, ph, V, psi, out);
+        else hipLaunchKernelGGL((sphere_kpoint_kernel<T, NS, NP, false, 2>), grid, blk, lds, s, a, ks, ph, V, psi, out);
+    }
+    QG_HIP(hipGetLastError());
+}
+
+template <class T>
+static bool sphere_kpoint_t(qg_ham* h, const double* k, int nbands, const T* psi, int64_t ld, T* out, int64_t ld_out,
+                            DevBuf<double>& part, double* coef, hipStream_t s) {
+    qg_nonlocal* nl = h->nl;
+    const qg_grid& g = h->grid;
+    constexpr int VN = 16 / sizeof(T);
+    const int dtype = sizeof(T) == 4 ? QG_F32 : QG_F64;
+    const size_t need = sphere_project_need(nl, dtype, std::max(1, nbands), true, true);
+    if (need == 0) return false;
+    const int nq = (g.n[0] + VN - 1) / VN;
+    const int ty = sphere_kpoint_ty(nq, g.n[1]);
+    const SphereGeo* sg = sphere_geometry(nl, dtype, ty, true);
+    const int hv = sphere_halo_vectors(nq, sg->tpb);
+    if (!sg->ok || hv > 2) return false;
+    if (sphere_kpoint_lds<T>(g.n[0], ty, g.n[2], nl->sphere_form.ns, nl->sphere_form.np, sg->max_col) > lds_limit())
+        return false;
+    if (nbands == 0) return true;
+    SphereArgs a = sphere_args(nl, *sg, nbands, 1, 0);
+    const size_t lds = sphere_kpoint_lds<T>(g.n[0], ty, a.tz, nl->sphere_form.ns, nl->sphere_form.np, sg->max_col);
+    part.alloc(need);
+    (void)sphere_project(nl, dtype, nbands, psi, ld, k, part.p, coef, true, s);
+    a.ld_in = 2 * ld; a.ld_out = 2 * ld_out;
+    a.coef = coef;
+    const double cf = -0.5, k2 = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
+    SphereKStencil<T> ks;
+    ks.c0 = (T)(-14350.0 / 5040.0 * cf * (1.0 / (g.h[0] * g.h[0]) + 1.0 / (g.h[1] * g.h[1]) + 1.0 / (g.h[2] * g.h[2])) -
+                cf * k2);
+    const double w2[4] = {8064.0, -1008.0, 128.0, -9.0}, w1[4] = {672.0, -168.0, 32.0, -3.0};
+    for (int d = 0; d < 3; ++d)
+        for (int m = 0; m < 4; ++m) {
+            ks.a[d][m] = (T)(w2[m] * cf / (5040.0 * g.h[d] * g.h[d]));
+            ks.b[d][m] = (T)(2.0 * cf * k[d] * w1[m] / (840.0 * g.h[d]));
+        }
+    SpherePhase ph;
+    for (int d = 0; d < 3; ++d) ph.kh[d] = k[d] * g.h[d];
+    const T* V = sizeof(T) == 4 ? (const T*)(const void*)h->V32.p : (const T*)(const void*)h->V64.p;
+    if (nl->sphere_form.ns == 2) sphere_kpoint_launch<T, 2, 2>(a, ks, ph, V, psi, out, lds, hv, s);
+    else sphere_kpoint_launch<T, 1, 1>(a, ks, ph, V, psi, out, lds, hv, s);
+    return true;
+}
+
+// H_k of complex blocks (interleaved; dtype the type of a part, ld in complex elements): projection
+// into coef (complex, nbands x ncoef) and one apply pass.  False (nothing launched) where the entry
+// lists do not serve; nbands 0: prepares the lists and says so.
+bool sphere_kpoint_apply(qg_ham* h, const double* k, int dtype, int nbands, const void* psi, int64_t ld, void* out,
+                         int64_t ld_out, DevBuf<double>& part, double* coef, hipStream_t s) {
+    if (!h->nl || !sphere_serves(h->grid, h->nl)) return false;
+    if (h->grid.ng() * (dtype == QG_F32 ? 8 : 16) > (int64_t)kOOB - 64) return false;
+    if (dtype == QG_F32)
+        return sphere_kpoint_t<float>(h, k, nbands, (const float*)psi, ld, (float*)out, ld_out, part, coef, s);
+    return sphere_kpoint_t<double>(h, k, nbands, (const double*)psi, ld, (double*)out, ld_out, part, coef, s);
 }
 
 }  // namespace qg
