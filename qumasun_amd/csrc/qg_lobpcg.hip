@@ -141,37 +141,55 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     return t;
 }
 
-// out[k] = sum_i a[k*ld + i] * b[k*ld + i]  (one workgroup per band, FP64 accumulation)
+// Points of one workgroup of the column sums: a band is cut into ranges, so that a block of any number
+// of bands fills the chip, and the ranges' sums are added in their order.  One workgroup per band took
+// 854 (coldot of a block with itself) and 1074 us (residual) at 512,000 points x 144 FP64 bands, ranges
+// take 126 and 335 us (floors at 4.68 TB/s 126 and 378).
+constexpr int64_t kColRange = 8192;
+
+// part[k][range] = sum_i a[k*ld + i] * b[k*ld + i] (FP64 accumulation)
 template <class T>
-__global__ __launch_bounds__(256) void coldot_kernel(const T* a, const T* b, int64_t ld, int64_t n, double* out) {
+__global__ __launch_bounds__(256) void coldot_kernel(const T* a, const T* b, int64_t ld, int64_t n, double* part) {
     __shared__ double red[4];
-    const int k = blockIdx.x;
+    const int k = blockIdx.y;
     const T* pa = a + (int64_t)k * ld;
     const T* pb = b + (int64_t)k * ld;
+    const int64_t i0 = blockIdx.x * kColRange, i1 = min(n, i0 + kColRange);
     double s = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) s += (double)pa[i] * (double)pb[i];
+#pragma unroll 4
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) s += (double)pa[i] * (double)pb[i];
     s = block_sum(s, red);
-    if (threadIdx.x == 0) out[k] = s;
+    if (threadIdx.x == 0) part[(int64_t)k * gridDim.x + blockIdx.x] = s;
 }
 
-// r[k] = ax[k] - e[k] x[k]; norm2[k] = ||r[k]||^2
+// r[k] = ax[k] - e[k] x[k]; part[k][range] = the range's share of ||r[k]||^2
 template <class T>
 __global__ __launch_bounds__(256) void residual_kernel(const T* ax, const T* x, const double* e, T* r, int64_t ld,
-                                                       int64_t n, double* norm2) {
+                                                       int64_t n, double* part) {
     __shared__ double red[4];
-    const int k = blockIdx.x;
+    const int k = blockIdx.y;
     const double ek = e[k];
     const T* pa = ax + (int64_t)k * ld;
     const T* px = x + (int64_t)k * ld;
     T* pr = r + (int64_t)k * ld;
+    const int64_t i0 = blockIdx.x * kColRange, i1 = min(n, i0 + kColRange);
     double s = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+#pragma unroll 4
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) {
         const T v = (T)(pa[i] - (T)ek * px[i]);
         pr[i] = v;
         s += (double)v * (double)v;
     }
     s = block_sum(s, red);
-    if (threadIdx.x == 0) norm2[k] = s;
+    if (threadIdx.x == 0) part[(int64_t)k * gridDim.x + blockIdx.x] = s;
+}
+
+// out[k] = sum over the ranges of part[k]
+__global__ __launch_bounds__(64) void colsum_kernel(const double* part, int ranges, double* out) {
+    double s = 0.0;
+    for (int i = threadIdx.x; i < ranges; i += 64) s += part[(int64_t)blockIdx.x * ranges + i];
+    for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // C[m + ldc n] = sum_c W[c][m + N n] (split-K partial Gram products)
@@ -277,7 +295,7 @@ struct LobpcgState {
     DevBuf<double> Sa, Sb;        // 3N x 3N + 4 N x N scratch each (reference layout)
     DevBuf<double> A3, B3, D, E;  // nb x nb eigenproblem
     DevBuf<int> info;
-    DevBuf<double> eig, norm_a, norm_b, res2;
+    DevBuf<double> eig, norm_a, norm_b, res2, col_part;
     DevBuf<float> C32, G32, gram_ws;
     DevBuf<unsigned char> split_ws;
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -290,6 +308,28 @@ struct LobpcgState {
 };
 
 void lobpcg_state_free(LobpcgState* s) { delete s; }
+
+static int col_ranges(int64_t K) { return (int)((K + kColRange - 1) / kColRange); }
+
+// out[k] = a_k . b_k for N bands of K points
+template <class T>
+static void coldot(LobpcgState& st, const T* a, const T* b, int64_t K, int N, double* out, hipStream_t s) {
+    const int nr = col_ranges(K);
+    if (nr > 1) st.col_part.alloc((int64_t)nr * N);
+    double* part = nr > 1 ? st.col_part.p : out;
+    hipLaunchKernelGGL((coldot_kernel<T>), dim3(nr, N), dim3(256), 0, s, a, b, K, K, part);
+    if (nr > 1) hipLaunchKernelGGL(colsum_kernel, dim3(N), dim3(64), 0, s, part, nr, out);
+}
+
+// r_k = ax_k - eig_k x_k, res2[k] = ||r_k||^2
+template <class T>
+static void block_residual(LobpcgState& st, const T* ax, const T* x, T* r, int64_t K, int N, hipStream_t s) {
+    const int nr = col_ranges(K);
+    if (nr > 1) st.col_part.alloc((int64_t)nr * N);
+    double* part = nr > 1 ? st.col_part.p : st.res2.p;
+    hipLaunchKernelGGL((residual_kernel<T>), dim3(nr, N), dim3(256), 0, s, ax, x, st.eig.p, r, K, K, part);
+    if (nr > 1) hipLaunchKernelGGL(colsum_kernel, dim3(N), dim3(64), 0, s, part, nr, st.res2.p);
+}
 
 // shift of the kinetic preconditioner: the run's own, or the fallback of a learned run
 static double kinetic_shift(const qg_lobpcg_opts& o) {
@@ -475,8 +515,8 @@ static void run_lobpcg(qg_ham* h, const qg_lobpcg_opts& o, int N, double* eig_ho
     } else {
         hpsi(P, AP);
     }
-    hipLaunchKernelGGL((coldot_kernel<T>), dim3(N), dim3(256), 0, s, X, AX, K, K, st.eig.p);
-    hipLaunchKernelGGL((residual_kernel<T>), dim3(N), dim3(256), 0, s, AX, X, st.eig.p, R, K, K, st.res2.p);
+    coldot<T>(st, X, AX, K, N, st.eig.p, s);
+    block_residual<T>(st, AX, X, R, K, N, s);
     std::vector<double> ev(n3), nx(N), np(N), r2(N);
     QG_HIP(hipMemcpyAsync(eig_host, st.eig.p, N * 8, hipMemcpyDeviceToHost, s));
     QG_HIP(hipMemcpyAsync(r2.data(), st.res2.p, N * 8, hipMemcpyDeviceToHost, s));
@@ -522,11 +562,11 @@ static void run_lobpcg(qg_ham* h, const qg_lobpcg_opts& o, int N, double* eig_ho
         }
         const bool use_p = p_valid;
         if (robust) {
-            hipLaunchKernelGGL((coldot_kernel<T>), dim3(N), dim3(256), 0, s, R, R, K, K, st.norm_a.p);
+            coldot<T>(st, R, R, K, N, st.norm_a.p, s);
             hipLaunchKernelGGL((colscale_kernel<T>), dim3(grid_for(K) / 4 + 1, N), dim3(256), 0, s, R, (T*)nullptr,
                                st.norm_a.p, K, K);
             if (use_p) {
-                hipLaunchKernelGGL((coldot_kernel<T>), dim3(N), dim3(256), 0, s, P, P, K, K, st.norm_b.p);
+                coldot<T>(st, P, P, K, N, st.norm_b.p, s);
                 hipLaunchKernelGGL((colscale_kernel<T>), dim3(grid_for(K) / 4 + 1, N), dim3(256), 0, s, P, AP,
                                    st.norm_b.p, K, K);
             }
@@ -574,7 +614,7 @@ static void run_lobpcg(qg_ham* h, const qg_lobpcg_opts& o, int N, double* eig_ho
             // discard this step: X and AX stay, P and AP are dropped, R = AX - X E again
             QG_HIP(hipMemsetAsync(P, 0, blk, s));
             QG_HIP(hipMemsetAsync(AP, 0, blk, s));
-            hipLaunchKernelGGL((residual_kernel<T>), dim3(N), dim3(256), 0, s, AX, X, st.eig.p, R, K, K, st.res2.p);
+            block_residual<T>(st, AX, X, R, K, N, s);
             p_valid = false;
             large_diff = true;   // full Gram on the next iteration
             ++stats.rollbacks;
@@ -603,7 +643,7 @@ static void run_lobpcg(qg_ham* h, const qg_lobpcg_opts& o, int N, double* eig_ho
         if (use_p) op.update(P, Cp, Cp32, nb, 1.0, Tm);
         QG_HIP(hipMemcpyAsync(P, Tm, blk, hipMemcpyDeviceToDevice, s));
         op.update(X, Cx, Cx32, nb, 1.0, Tm);
-        hipLaunchKernelGGL((coldot_kernel<T>), dim3(N), dim3(256), 0, s, Tm, Tm, K, K, st.norm_a.p);
+        coldot<T>(st, Tm, Tm, K, N, st.norm_a.p, s);
         QG_HIP(hipMemcpyAsync(nx.data(), st.norm_a.p, N * 8, hipMemcpyDeviceToHost, s));
         sync();
         stats.t_update += sector_end(t0, 16, 1);
@@ -645,7 +685,7 @@ static void run_lobpcg(qg_ham* h, const qg_lobpcg_opts& o, int N, double* eig_ho
             if (robust)   // renormalise X (and AX with it); norm_a holds ||x'||^2
                 hipLaunchKernelGGL((colscale_kernel<T>), dim3(grid_for(K) / 4 + 1, N), dim3(256), 0, s, X, AX,
                                    st.norm_a.p, K, K);
-            hipLaunchKernelGGL((residual_kernel<T>), dim3(N), dim3(256), 0, s, AX, X, st.eig.p, R, K, K, st.res2.p);
+            block_residual<T>(st, AX, X, R, K, N, s);
             sync();
             stats.t_update += sector_end(t0, 16, 1);
             t0 = sector_begin();
@@ -976,7 +1016,7 @@ static void run_lobpcg_ortho(qg_ham* h, const qg_lobpcg_opts& o, int N, double* 
     // largest band residual, and the block's residual norm sqrt(sum over bands)
     double totres = 0.0;
     auto residual = [&](double& maxres) {
-        hipLaunchKernelGGL((residual_kernel<T>), dim3(N), dim3(256), 0, s, AX, X, st.eig.p, W, K, K, st.res2.p);
+        block_residual<T>(st, AX, X, W, K, N, s);
         std::vector<double> r2(N);
         QG_HIP(hipMemcpyAsync(r2.data(), st.res2.p, N * 8, hipMemcpyDeviceToHost, s));
         QG_HIP(hipMemcpyAsync(eig_host, st.eig.p, N * 8, hipMemcpyDeviceToHost, s));
@@ -1096,7 +1136,7 @@ static void run_lobpcg_ortho(qg_ham* h, const qg_lobpcg_opts& o, int N, double* 
         std::swap(P, Tm);                                      // P = P', Tm = free
         hipLaunchKernelGGL(diag_copy_kernel, dim3((N + 255) / 256), dim3(256), 0, s, st.D.p, st.eig.p, N);
         // keep X normalised against rounding
-        hipLaunchKernelGGL((coldot_kernel<T>), dim3(N), dim3(256), 0, s, X, X, K, K, st.norm_a.p);
+        coldot<T>(st, X, X, K, N, st.norm_a.p, s);
         hipLaunchKernelGGL((colscale_kernel<T>), dim3(grid_for(K) / 4 + 1, N), dim3(256), 0, s, X, (T*)nullptr,
                            st.norm_a.p, K, K);
         sync();
