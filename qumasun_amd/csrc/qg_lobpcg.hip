@@ -109,6 +109,10 @@ static void batch_service_leave(BatchService* b, hipStream_t s) {
 void gram_bf16(const float* A, const float* B, int64_t K, int M, int N, int64_t lda, int64_t ldb,
                double* C, int ldc, float* partial, size_t partial_floats, hipStream_t s, bool split);
 size_t gram_bf16_workspace(int64_t K, int M, int N);
+size_t gram64_workspace(int64_t K, int M, int N);
+bool gram64_serves(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N);
+void gram64(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N, double* C, int ldc,
+            double* ws, size_t ws_bytes, hipStream_t s);
 
 #define QG_BLAS(call)                                                                        \
     do {                                                                                     \
@@ -248,17 +252,25 @@ static int64_t gram_chunks(int64_t K, int want = 0) {
 }
 template <class T>
 static size_t gram_workspace(int64_t K, int M, int N, int want = 0) {
-    return (size_t)(gram_chunks<T>(K, want) + 1) * M * N * sizeof(T);
+    const size_t own = sizeof(T) == 8 ? gram64_workspace(K, M, N) : 0;
+    return std::max(own, (size_t)(gram_chunks<T>(K, want) + 1) * M * N * sizeof(T));
 }
 
 // C (M x N, FP64, column stride ldc) = A^T B over K rows; A: M columns of length K (column m
 // at A + m lda), B: N columns (ld ldb).  The Gram blocks of the Rayleigh-Ritz matrices
-// (MakeMatrix_d_blas, lobpcg_d_multi_mpi.h:192-250): split-K over the rows as one
-// strided-batched library GEMM in the block precision (enough parallel work for small M, N),
-// then the chunks summed in FP64.
+// (MakeMatrix_d_blas, lobpcg_d_multi_mpi.h:192-250).  FP64: the matrix-core kernel of
+// qg_dense64.hip (faster at every size measured there), unless the caller chose the number of
+// chunks or a column is not 16-byte aligned.  Otherwise split-K over the rows as one strided-batched library GEMM in the block
+// precision (enough parallel work for small M, N), then the chunks summed in FP64.
 template <class T>
 static void gram_splitk(rocblas_handle hb, hipStream_t s, const T* A, int64_t lda, const T* B, int64_t ldb, int64_t K,
                         int M, int N, double* C, int ldc, T* ws, size_t ws_bytes, int want_chunks = 0) {
+    if constexpr (sizeof(T) == 8) {
+        if (want_chunks <= 0 && gram64_serves(A, lda, B, ldb, K, M, N)) {
+            gram64(A, lda, B, ldb, K, M, N, C, ldc, ws, ws_bytes, s);
+            return;
+        }
+    }
     const int64_t nch = gram_chunks<T>(K, want_chunks);
     const int64_t kc = K / nch;
     const int64_t rem = K - nch * kc;
@@ -364,7 +376,9 @@ struct Ops {
                        nch);
     }
     static size_t split_workspace(int64_t K, int N, int nb_max = 0, int want = 0) {
-        return gram_workspace<T>(K, N, nb_max > 0 ? nb_max : N, want);
+        size_t need = 0;
+        for (int nb = N; nb <= std::max(N, nb_max); nb += N) need = std::max(need, gram_workspace<T>(K, N, nb, want));
+        return need;
     }
     // Out = A * Cm + beta * Out, A: K x N (ld K), Cm: N x N FP64 (ld ldc) / FP32 copy for T = float
     void update(const T* A, const double* Cm, const float* Cm32, int ldc, double beta, T* Out) {
