@@ -113,6 +113,8 @@ size_t gram64_workspace(int64_t K, int M, int N);
 bool gram64_serves(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N);
 void gram64(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N, double* C, int ldc,
             double* ws, size_t ws_bytes, hipStream_t s);
+bool update64(const double* A, int64_t lda, const double* C, int ldc, int64_t K, int N, double alpha, double beta,
+              double* out, int64_t ldo, hipStream_t s);
 
 #define QG_BLAS(call)                                                                        \
     do {                                                                                     \
@@ -384,6 +386,7 @@ struct Ops {
     void update(const T* A, const double* Cm, const float* Cm32, int ldc, double beta, T* Out) {
         if constexpr (sizeof(T) == 8) {
             const double one = 1.0;
+            if (update64(A, K, Cm, ldc, K, N, one, beta, Out, K, s)) return;
             QG_BLAS(rocblas_dgemm(st.blas, rocblas_operation_none, rocblas_operation_none, (int)K, N, N, &one, A,
                                   (int)K, Cm, ldc, &beta, Out, (int)K));
         } else {
@@ -925,6 +928,7 @@ static void run_lobpcg_ortho(qg_ham* h, const qg_lobpcg_opts& o, int N, double* 
     // Out = alpha A C + beta Out, C: N x N FP64 (ld ldc), A: K x N
     auto upd = [&](const T* A, const double* C, int ldc, double alpha, double beta, T* Out) {
         if constexpr (sizeof(T) == 8) {
+            if (update64(A, K, C, ldc, K, N, alpha, beta, Out, K, s)) return;
             QG_BLAS(rocblas_dgemm(st.blas, rocblas_operation_none, rocblas_operation_none, (int)K, N, N, &alpha, A,
                                   (int)K, C, ldc, &beta, Out, (int)K));
         } else {

@@ -1,6 +1,6 @@
 // qg_rows.hip — H·psi on MI355X (gfx950) with 16-byte row vectors: a tile-centric projector
 // dot-product kernel and a stencil + local potential + projector-apply kernel that writes each
-// H psi value exactly once.
+// H psi value exactly once.  AUTO plans use them where the sphere lists (qg_sphere.hip) do not serve.
 //
 // Reference semantics (QUMASUN source/):
 //   out += coef Lap8 psi, periodic            GridDifference8th.h:83-185
