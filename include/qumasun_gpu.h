@@ -157,8 +157,8 @@ int qg_gradient8_apply(const qg_grid* g, int dtype, int nbands, const void* psi,
  * with occ_host[b] > 0, *energy = sum_b occ_b sum_{a,j} E_j c_baj^2 and, when forces_host is not
  * NULL, forces_host[3a + d] = sum_b sum_j E_j c_baj (-2 occ_b) dV sum beta_aj d_d psi_b with the
  * 8th-order gradient (set, not accumulated).  psi: nbands band-major device vectors.  The handle
- * keeps the gradient scratch of a run of bands (at most 4 GiB) between calls, so calls on one
- * handle must not overlap. */
+ * keeps scratch between calls (partial forces, or where the sphere lists do not serve the gradient
+ * of a run of bands, at most 4 GiB), so calls on one handle must not overlap. */
 int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld,
                              const double* occ_host, double* energy, double* forces_host, void* stream);
 
@@ -263,9 +263,9 @@ int qg_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int6
                          void* hpsi, int64_t ld_out, void* stream);
 /* Same result as qg_hamiltonian_apply with no device memory allocated or freed, for callers
  * that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  No counterpart in the reference.  It runs the row kernels only (Nx a
- * multiple of 4 in FP32 or of 2 in FP64, 8 <= Nx <= 1024, Gaussian projectors with l <= 1)
- * and keeps the projector partials and coefficients in one fixed 64 MiB device array per GPU,
+ * forbid hipMalloc).  No counterpart in the reference.  It serves what the row kernels
+ * serve (Nx a multiple of 4 in FP32 or of 2 in FP64, 8 <= Nx <= 1024, Gaussian projectors with
+ * l <= 1; the sphere passes where they do) and keeps the projector partials and coefficients in one fixed 64 MiB device array per GPU,
  * processing the bands in chunks that fit it; QG_ERR_ARG when one band does not fit or the
  * projector geometry is not prepared (qg_nonlocal_create/update prepare it).  Calls on one GPU
  * share that array: calls that overlap on one GPU (other streams, other threads) race. */
@@ -364,7 +364,8 @@ typedef struct qg_lobpcg_opts {
     void* watch_user;
     int orth;                /* QG_ORTH_* (orthonormal basis only) */
     int gram_chunks;         /* K chunks of the split-K library Gram products (each chunk summed
-                                in the block precision, the chunks in FP64); 0: 64 in FP64,
+                                in the block precision, the chunks in FP64); 0: this engine's
+                                matrix-core kernel in FP64 (64 chunks where it does not serve),
                                 chunks of at most ~6,750 terms in FP32 (256 at 120^3: longer FP32
                                 partial sums stalled the FP32 phase at 512 bands) */
     double reortho;          /* orthonormal basis: a second orthonormalisation pass runs when the
@@ -473,9 +474,10 @@ int qg_hamiltonian_set_cnn(qg_ham* h, qg_cnn* c);
 
 /* ------------------------------------------------- batches of uneven cells ---- */
 /* H psi for ncells independent cells (each its own Hamiltonian, grid, atoms and band count;
- * psi[c], hpsi[c] band-major device blocks with ld == Ng of that cell) in persistent launches:
- * one projection launch and one fused stencil/V/projector launch per round of Infinity-Cache
- * sized band chunks, covering every cell.  Same results as qg_hamiltonian_apply per cell.
+ * psi[c], hpsi[c] band-major device blocks with ld == Ng of that cell): the cells' own launches
+ * over two streams where the sphere lists serve every cell, otherwise persistent launches, one
+ * projection launch and one fused stencil/V/projector launch per round of Infinity-Cache sized
+ * band chunks, covering every cell.  Returns with the work done.  Same results as qg_hamiltonian_apply per cell.
  * The cells must share the projector slot count (cells with different tile plans run in
  * one stencil launch per plan).  No
  * counterpart in the reference (which runs one cell per process). */
