@@ -47,11 +47,6 @@ template <class T>
 __device__ __forceinline__ Row<T> vload(rsrc_t r, int voff, int soff) {
     return __builtin_bit_cast(Row<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
-// the same with cache policy nt, for values read once
-template <class T>
-__device__ __forceinline__ Row<T> vload_once(rsrc_t r, int voff, int soff) {
-    return __builtin_bit_cast(Row<T>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
 template <class T>
 __device__ __forceinline__ void vstore(rsrc_t r, const Row<T>& v, int voff, int soff) {
     // cache policy nt: the results are not read back here, and keeping them out of L2 leaves it to
@@ -733,7 +728,7 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjA
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int h = 0; h < PW; ++h) q[b][h] = vload_once<T>(rin[b], vo + (own ? 16 * h : 0), z * plane * S * PW);
+            for (int h = 0; h < PW; ++h) q[b][h] = vload<T>(rin[b], vo + (own ? 16 * h : 0), z * plane * S * PW);
     };
     // a slot without points in the plane is loaded through an empty resource (zeros, no traffic)
     auto load_vals = [&](const Step& s, uint32_t m, int k) {
