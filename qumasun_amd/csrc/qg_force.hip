@@ -207,7 +207,9 @@ int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void*
         const qg_grid& g = nl->gcopy;
         const int64_t ng = g.ng();
         const size_t es = dtype == QG_F32 ? 4 : 8;
-        if (sphere_nonlocal_force(nl, dtype, 1, nullptr, nullptr, psi, ld, nullptr, nl->force_part, nullptr,
+        // FP64 states: one pass over psi.  FP32 states keep the chain below and its kernels: the FP64 forces
+        // of FP32 arithmetic follow its order of rounding (another order moves them by 6e-7)
+        if (dtype == QG_F64 && sphere_nonlocal_force(nl, dtype, 1, nullptr, nullptr, psi, ld, nullptr, nl->force_part, nullptr,
                                                  false, s)) {
             // the occupied states: their projections (in runs of consecutive bands), then forces
             // and energies on the device
@@ -275,14 +277,14 @@ int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void*
             while (k1 < occupied.size() && (int)(k1 - k0) < chunk && occupied[k1] == occupied[k1 - 1] + 1) ++k1;
             const int b0 = occupied[k0], nb = (int)(k1 - k0);
             const unsigned char* p = (const unsigned char*)psi + (size_t)b0 * ld * es;
-            check_rc(qg_nonlocal_project(nl, dtype, nb, p, ld, c, s));
+            nonlocal_project(nl, dtype, nb, p, ld, c, dtype == QG_F64, s);
             if (forces_host) {
                 // the three gradient blocks back to back: one projection of 3 nb bands
                 unsigned char* gx = nl->force_grad.p;
                 unsigned char* gy = gx + (size_t)nb * ng * es;
                 unsigned char* gz = gy + (size_t)nb * ng * es;
                 gradient8(g, dtype, nb, p, ld, gx, gy, gz, ng, 1.0, s);
-                check_rc(qg_nonlocal_project(nl, dtype, 3 * nb, gx, ng, d, s));
+                nonlocal_project(nl, dtype, 3 * nb, gx, ng, d, dtype == QG_F64, s);
                 QG_HIP(hipMemcpyAsync(hd.data(), d, (size_t)3 * nb * ncoef * 8, hipMemcpyDeviceToHost, s));
             }
             QG_HIP(hipMemcpyAsync(hc.data(), c, (size_t)nb * ncoef * 8, hipMemcpyDeviceToHost, s));

@@ -1408,6 +1408,13 @@ static void batch_streams_apply(std::vector<BatchReq> reqs, int dtype, hipStream
     QG_HIP(hipStreamSynchronize(s));
 }
 
+void nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, double* coef, bool lists,
+                      hipStream_t s) {
+    if (rows_nonlocal_project(nl, dtype, nbands, psi, ld, coef, nl->rows_part, s, lists)) return;
+    if (dtype == QG_F64) launch_project<double>(nl, nbands, (const double*)psi, ld, coef, s);
+    else launch_project<float>(nl, nbands, (const float*)psi, ld, coef, s);
+}
+
 void batch_hamiltonian_apply(const std::vector<BatchReq>& reqs, int dtype, hipStream_t s,
                              DevBuf<unsigned char>& scratch, DevBuf<double>& coefs) {
     if (reqs.empty()) return;
@@ -1623,12 +1630,7 @@ int qg_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi,
         QG_REQUIRE(ld >= nl->gcopy.ng(), "leading dimension smaller than the grid");
         if (nbands == 0 || nl->geo.ncoef == 0) return;
         QG_REQUIRE(psi && coef, "null pointer");
-        hipStream_t s = as_stream(stream);
-        if (rows_nonlocal_project(nl, dtype, nbands, psi, ld, coef, nl->rows_part, s)) return;
-        if (dtype == QG_F64)
-            launch_project<double>(nl, nbands, (const double*)psi, ld, coef, s);
-        else
-            launch_project<float>(nl, nbands, (const float*)psi, ld, coef, s);
+        nonlocal_project(nl, dtype, nbands, psi, ld, coef, true, as_stream(stream));
     });
 }
 

@@ -315,7 +315,10 @@ void precond_state_free(PrecondPlan*);
 bool rows_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
                             int64_t ld_out, hipStream_t s, RowsScratch* scratch);
 bool rows_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, double* coef,
-                           DevBuf<double>& part_buf, hipStream_t s);
+                           DevBuf<double>& part_buf, hipStream_t s, bool lists = true);
+// c of a band block, from the sphere lists where they serve (lists) or by the row and table kernels
+void nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, double* coef, bool lists,
+                      hipStream_t s);
 bool rows_laplacian_apply(const qg_grid& g, int dtype, int nbands, const void* psi, int64_t ld, void* out,
                           int64_t ld_out, double coef, int accumulate, hipStream_t s);
 void rows_prepare(qg_nonlocal* nl);

@@ -1314,10 +1314,10 @@ bool rows_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, i
 // coef_dev[b * ncoef + j] for a band block through the tile-centric projection; false when
 // the row path does not serve this projector set.
 bool rows_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, double* coef,
-                           DevBuf<double>& part_buf, hipStream_t s) {
+                           DevBuf<double>& part_buf, hipStream_t s, bool lists) {
     const qg_grid& g = nl->gcopy;
     if (nl->geo.ncoef == 0) return false;
-    if (const size_t need = sphere_project_need(nl, dtype, nbands, false, true)) {
+    if (const size_t need = lists ? sphere_project_need(nl, dtype, nbands, false, true) : 0) {
         part_buf.alloc(need);
         return sphere_project(nl, dtype, nbands, psi, ld, nullptr, part_buf.p, coef, true, s);
     }
