@@ -9,6 +9,7 @@
 #include <memory>
 #include <mutex>
 #include "../../include/qumasun_gpu.h"
+#include "qg_sphere_plan.hpp"
 
 namespace qg {
 
@@ -236,9 +237,6 @@ struct SphereGeo {
     DevBuf<int> meta, counts;             // what the pointers above point into
     DevBuf<unsigned char> lists;
 };
-// planes of one epoch of the projection's lists
-constexpr int kProjPlanes = 8;
-
 // Caller-provided FP64 scratch of one application (projector partials, then coefficients).
 struct RowsScratch {
     double* base;
@@ -329,9 +327,9 @@ bool sphere_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi,
 bool sphere_prepared(qg_nonlocal* nl, int dtype);
 bool sphere_kpoint_apply(qg_ham* h, const double* k, int dtype, int nbands, const void* psi, int64_t ld, void* out,
                          int64_t ld_out, DevBuf<double>& part, double* coef, hipStream_t s);
-size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build);
+size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build, size_t most = SIZE_MAX);
 bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, const double* k, double* part,
-                    double* coef, bool may_build, hipStream_t s);
+                    double* coef, bool may_build, hipStream_t s, size_t most = SIZE_MAX);
 bool sphere_nonlocal_force(qg_nonlocal* nl, int dtype, int nocc, const int* band_idx, const double* weight,
                            const void* psi, int64_t ld, const double* coef, DevBuf<double>& part, double* force,
                            bool run, hipStream_t s);

@@ -1205,7 +1205,10 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     // both launches from the sphere entry lists where they serve
     const bool sphere = nl && sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nullptr, ws == nullptr,
                                                        false, s);
-    const size_t sphere_part = sphere ? sphere_project_need(nl, dtype, nbands, false, ws == nullptr) : 0;
+    // doubles of partials there is room for
+    const size_t most = !ws || !nl ? SIZE_MAX
+                                   : ws->capacity - std::min(ws->capacity, (size_t)nbands * nl->geo.ncoef);
+    const size_t sphere_part = sphere ? sphere_project_need(nl, dtype, nbands, false, ws == nullptr, most) : 0;
     if (sphere) {
         if (sh.typ == 0) return false;
         const RowsShape def = rows_shape(g, dtype, 0);
@@ -1260,7 +1263,7 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     const bool timed = h->timing && ws == nullptr;
     if (timed) QG_HIP(hipEventRecord(h->tev[0], s));
     if (sphere_part) {
-        (void)sphere_project(nl, dtype, nbands, psi, ld, nullptr, part, coef, ws == nullptr, s);
+        (void)sphere_project(nl, dtype, nbands, psi, ld, nullptr, part, coef, ws == nullptr, s, most);
     } else if (nl) {
         if (rgp->njs == 4) {
             if (rgp->pform == 2) rows_launch_project<T, 4, 2>(nl, *rgp, sh.nbp, nbands, psi, ld, part, coef, s);
@@ -1428,13 +1431,13 @@ void rows_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64
     if (nl) {
         const RowsShape sh = rows_shape(g, dtype, nbands, &h->plan);
         QG_REQUIRE(sh.typ > 0, "the projection tile does not fit this grid");
-        // bands whose partials and coefficients fit
-        auto need = [&](int nb) { return sphere_project_need(nl, dtype, nb, false, false) + (size_t)nb * nl->geo.ncoef; };
-        if (sphere_prepared(nl, dtype) && sphere_project_need(nl, dtype, 1, false, false)) {
-            while (chunk > 1 && need(chunk) > kScratchDoubles) chunk = (chunk + 1) / 2;
-            QG_REQUIRE(need(chunk) <= kScratchDoubles,
-                       "one band needs " + std::to_string(need(1)) + " doubles of projector scratch, more than the fixed " +
-                           std::to_string(kScratchDoubles));
+        // bands whose partials and coefficients fit; a band's least need is one slab of partials
+        const size_t one_band = sphere_prepared(nl, dtype) ? sphere_project_need(nl, dtype, 1, false, false, 0) : 0;
+        if (one_band) {
+            chunk = sphere_chunk_bands(nbands, one_band, nl->geo.ncoef, kScratchDoubles);
+            QG_REQUIRE(chunk > 0, "one band needs " + std::to_string(one_band + nl->geo.ncoef) +
+                                      " doubles of projector scratch, more than the fixed " +
+                                      std::to_string(kScratchDoubles));
         } else {
             const RowsGeo* rgp = rows_geometry(nl, sh.typ, sh.tzp, false, false);
             QG_REQUIRE(rgp && rgp->ok, "the projector geometry of this launch shape is not prepared (qg_nonlocal_create "

@@ -1872,7 +1872,7 @@ struct SphereProjShape {
 };
 
 template <class T>
-static bool sphere_proj_shape(qg_nonlocal* nl, int nbands, bool cplx, bool may_build, SphereProjShape& sh) {
+static bool sphere_proj_shape(qg_nonlocal* nl, int nbands, bool cplx, bool may_build, size_t most, SphereProjShape& sh) {
     if (!sphere_serves(nl->gcopy, nl)) return false;
     const qg_grid& g = nl->gcopy;
     if (cplx && g.ng() * 16 > (int64_t)kOOB - 64) return false;   // band bytes below the out-of-range offset
@@ -1887,13 +1887,12 @@ static bool sphere_proj_shape(qg_nonlocal* nl, int nbands, bool cplx, bool may_b
     // sums fill the registers)
     const int nbr = (sizeof(T) == 4 ? 4 : 2) / (nl->sphere_form.ns == 2 ? 2 : 1);
     sh.nb = cplx ? std::max(1, nbr / 2) : nbr;
+    const size_t per_slab = (size_t)sh.sg->ntile * std::max(1, sh.sg->max_col) * nc * nbands * (cplx ? 2 : 1);
     auto shape = [&] {
-        // slabs of whole epochs for ~4096 workgroups
-        const int64_t wg = (int64_t)sh.sg->ntile * ((nbands + sh.nb - 1) / sh.nb);
-        const int nep = (g.n[2] + kProjPlanes - 1) / kProjPlanes;
-        const int want = (int)std::max<int64_t>(1, std::min<int64_t>((4096 + wg - 1) / wg, nep));
-        sh.tz = (nep + want - 1) / want * kProjPlanes;
-        sh.nslab = (g.n[2] + sh.tz - 1) / sh.tz;
+        const SphereSlabs sl =
+            sphere_project_slabs(g.n[2], (int64_t)sh.sg->ntile * ((nbands + sh.nb - 1) / sh.nb), per_slab, most);
+        sh.tz = sl.tz;
+        sh.nslab = sl.nslab;
         sh.lds = sphere_proj_lds<T>(sh.sg->max_col, sh.tz, nw, cplx ? 2 * sh.nb : sh.nb, nc, cplx);
     };
     shape();
@@ -1902,15 +1901,17 @@ static bool sphere_proj_shape(qg_nonlocal* nl, int nbands, bool cplx, bool may_b
         shape();
     }
     if (sh.lds > lds_limit()) return false;
-    sh.npart = (size_t)sh.sg->ntile * sh.nslab * std::max(1, sh.sg->max_col) * nc * nbands * (cplx ? 2 : 1);
+    sh.npart = per_slab * sh.nslab;
     return true;
 }
 
 // Doubles of partials a projection of nbands bands needs; 0 where the entry lists do not serve it.
-size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build) {
+// most: the doubles there are; the slabs are fewer where they would need more (more than `most` is
+// returned only where one slab does not fit).
+size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build, size_t most) {
     SphereProjShape sh;
-    const bool ok = dtype == QG_F32 ? sphere_proj_shape<float>(nl, nbands, cplx, may_build, sh)
-                                    : sphere_proj_shape<double>(nl, nbands, cplx, may_build, sh);
+    const bool ok = dtype == QG_F32 ? sphere_proj_shape<float>(nl, nbands, cplx, may_build, most, sh)
+                                    : sphere_proj_shape<double>(nl, nbands, cplx, may_build, most, sh);
     return ok ? std::max<size_t>(1, sh.npart) : 0;
 }
 
@@ -1928,10 +1929,10 @@ static void sphere_project_launch(const SphereProjArgs& a, const SpherePhase& ph
 
 template <class T>
 static bool sphere_project_t(qg_nonlocal* nl, int nbands, const T* psi, int64_t ld, const double* k, double* part,
-                             double* coef, bool may_build, hipStream_t s) {
+                             double* coef, bool may_build, size_t most, hipStream_t s) {
     const bool cplx = k != nullptr;
     SphereProjShape sh;
-    if (!sphere_proj_shape<T>(nl, nbands, cplx, may_build, sh)) return false;
+    if (!sphere_proj_shape<T>(nl, nbands, cplx, may_build, most, sh)) return false;
     const qg_grid& g = nl->gcopy;
     const SphereGeo& sg = *sh.sg;
     SphereProjArgs a{};
@@ -1979,13 +1980,13 @@ static bool sphere_project_t(qg_nonlocal* nl, int nbands, const T* psi, int64_t 
 }
 
 // coef[b * ncoef + j] = dV sum beta_j psi_b through the entry lists, part holding
-// sphere_project_need doubles; k non-null: complex blocks (dtype the type of a part, ld and coef in
+// sphere_project_need doubles (of the same `most`); k non-null: complex blocks (dtype the type of a part, ld and coef in
 // complex elements) with the Bloch phases of k.  False (nothing launched) where not served.
 bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, const double* k, double* part,
-                    double* coef, bool may_build, hipStream_t s) {
+                    double* coef, bool may_build, hipStream_t s, size_t most) {
     if (dtype == QG_F32)
-        return sphere_project_t<float>(nl, nbands, (const float*)psi, ld, k, part, coef, may_build, s);
-    return sphere_project_t<double>(nl, nbands, (const double*)psi, ld, k, part, coef, may_build, s);
+        return sphere_project_t<float>(nl, nbands, (const float*)psi, ld, k, part, coef, may_build, most, s);
+    return sphere_project_t<double>(nl, nbands, (const double*)psi, ld, k, part, coef, may_build, most, s);
 }
 
 template <class T, int NB, int NS, int NP>
