@@ -21,6 +21,10 @@
 //   sum_s f_s (E c)_s + sum_p f_p [(E c)_y dy + (E c)_z dz + (E c)_x dx]
 // to it from registers, so the term needs no exponentials, no LDS exchange, no barrier and no
 // atomics, and every radial form (Gaussian or tabulated) costs the same.
+//
+// Infinities and NaN: those of psi outside every sphere reach no projection and no force.  A coefficient
+// that is not finite (one inside its sphere) makes its spheres' points so, and with them the other points
+// of the groups they touch (zero times the coefficient), at most VN - 1 beyond a sphere's end.
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -424,7 +428,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
         // projector term: one trip per list entry, the same number for all lanes of the wavefront
         // (an entry's channels are summed before they meet the larger stencil value)
         auto trip = [&](const Entry& e, int slot) {
-            double f[3] = {0.0, 0.0, 0.0};
+            double f[3];
             const int li = (int)(e.w & 1023u);
             const int dyi = ((int)(e.w << 11)) >> 21, dxi = ((int)e.w) >> 21;
             const T* im = imf + 4 * li;
@@ -437,41 +441,56 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                 fx = w0.v[0]; fy = w0.v[1]; fz = w1.v[0]; nzf = w1.v[1];
             }
             const T dx0 = hx * ((T)dxi - fx), dy = hy * ((T)dyi - fy), dz = hz * (((T)z - nzf) - fz);
+            // inside: leave out points outside the image
+            auto bands = [&](auto inside) __attribute__((always_inline)) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                T c[NC];
-                const Row<T>* ep = reinterpret_cast<const Row<T>*>(ec + ((size_t)li * NB + b) * NC);
+                for (int k = 0; k < 3; ++k) f[k] = 0.0;
 #pragma unroll
-                for (int k = 0; k < NC / VN; ++k) {
-                    const Row<T> w = ep[k];
+                for (int b = 0; b < NB; ++b) {
+                    T c[NC];
+                    const Row<T>* ep = reinterpret_cast<const Row<T>*>(ec + ((size_t)li * NB + b) * NC);
 #pragma unroll
-                    for (int u = 0; u < VN; ++u) c[k * VN + u] = w.v[u];
-                }
-T val[VN];
+                    for (int k = 0; k < NC / VN; ++k) {
+                        const Row<T> w = ep[k];
 #pragma unroll
-                for (int u = 0; u < VN; ++u) val[u] = e.f[0].v[u] * c[0];
+                        for (int u = 0; u < VN; ++u) c[k * VN + u] = w.v[u];
+                    }
+                    T val[VN];
 #pragma unroll
-                for (int s = 1; s < NS; ++s)
+                    for (int u = 0; u < VN; ++u) val[u] = e.f[0].v[u] * c[0];
 #pragma unroll
-                    for (int u = 0; u < VN; ++u) val[u] += e.f[s].v[u] * c[s];
+                    for (int s = 1; s < NS; ++s)
 #pragma unroll
-                for (int p = 0; p < NP; ++p) {
-                    const T cy = c[NS + 3 * p], cz = c[NS + 3 * p + 1], cx = c[NS + 3 * p + 2];
-                    const T ayz = cy * dy + cz * dz;
+                        for (int u = 0; u < VN; ++u) val[u] += e.f[s].v[u] * c[s];
 #pragma unroll
-                    for (int u = 0; u < VN; ++u) val[u] += e.f[NS + p].v[u] * (ayz + cx * (dx0 + (T)u * hx));
-                }
+                    for (int p = 0; p < NP; ++p) {
+                        const T cy = c[NS + 3 * p], cz = c[NS + 3 * p + 1], cx = c[NS + 3 * p + 2];
+                        const T ayz = cy * dy + cz * dz;
 #pragma unroll
-                for (int u = 0; u < VN; ++u) {
-                    if constexpr (FORCE) {
-                        f[0] += (double)val[u] * (double)gx[b].v[u];
-                        f[1] += (double)val[u] * (double)res[b].v[u];
-                        f[2] += (double)val[u] * (double)gz[b].v[u];
-                    } else {
-                        res[b].v[u] += val[u];
+                        for (int u = 0; u < VN; ++u) val[u] += e.f[NS + p].v[u] * (ayz + cx * (dx0 + (T)u * hx));
+                    }
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) {
+                        if constexpr (FORCE) {
+                            if constexpr (decltype(inside)::value) {
+                                bool on = false;
+#pragma unroll
+                                for (int v = 0; v < NV; ++v) on = on || e.f[v].v[u] != T(0);
+                                if (!on) continue;
+                            }
+                            f[0] += (double)val[u] * (double)gx[b].v[u];
+                            f[1] += (double)val[u] * (double)res[b].v[u];
+                            f[2] += (double)val[u] * (double)gz[b].v[u];
+                        } else {
+                            res[b].v[u] += val[u];
+                        }
                     }
                 }
-            }
+            };
+            bands(std::false_type{});
+            // a list's zero times an infinite or undefined gradient is not zero
+            if constexpr (FORCE)
+                if (__ballot(!__builtin_isfinite(f[0] + f[1] + f[2])) != 0) bands(std::true_type{});
             if constexpr (FORCE) {
                 if (slot < 0) {
                     flush(li, f);
@@ -757,6 +776,26 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjA
                 for (int b = 0; b < NR; ++b) acc[k][c][b] = T(0);
     };
     clear();
+    // the plane's values of the lane's points as real bands; a point of two overlapping groups counts once
+    auto values = [&](const Row<T> (&q)[NB][PW], int z, T (&v)[NR][VN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < VN; ++u) {
+            const bool mine = !RAG || x + u >= xq * VN;
+            if constexpr (CPLX) {
+                const T cz = ez[2 * (z - z0)], sz = ez[2 * (z - z0) + 1];
+                const T er = exy[u][0] * cz - exy[u][1] * sz, ei = exy[u][0] * sz + exy[u][1] * cz;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const T re = q[b][2 * u / VN].v[2 * u % VN], im = q[b][2 * u / VN].v[2 * u % VN + 1];
+                    v[2 * b][u] = mine ? er * re - ei * im : T(0);
+                    v[2 * b + 1][u] = mine ? er * im + ei * re : T(0);
+                }
+            } else {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) v[b][u] = mine ? q[b][0].v[u] : T(0);
+            }
+        }
+    };
     // the sums of one walk into the wavefront's LDS sums, a slot at a time: every lane puts its CN
     // coefficients and its image into the wavefront's buffer; then lane l owns coefficient l % CN of
     // CN neighbouring lanes, adds up runs of one image and the runs to the sums.  (Straight atomics
@@ -777,16 +816,56 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjA
                 const T dx0 = hx * ((T)dxi - im[0]), dy = hy * ((T)dyi - im[1]);
                 const T dz0 = hz * (((T)(s.ep * E) - im[3]) - im[2]);
                 T c[CN];
+                auto coefficients = [&]() __attribute__((always_inline)) {
+                    T all = T(0);
 #pragma unroll
-                for (int b = 0; b < NR; ++b) {
+                    for (int b = 0; b < NR; ++b) {
 #pragma unroll
-                    for (int q = 0; q < NS; ++q) c[q * NR + b] = acc[k][q][b];
+                        for (int q = 0; q < NS; ++q) c[q * NR + b] = acc[k][q][b];
 #pragma unroll
-                    for (int q = 0; q < NP; ++q) {
-                        const double p0 = (double)acc[k][NS + 3 * q][b];
-                        c[(NS + 3 * q) * NR + b] = (T)((double)dy * p0);
-                        c[(NS + 3 * q + 1) * NR + b] = (T)((double)dz0 * p0 + (double)hz * (double)acc[k][NS + 3 * q + 2][b]);
-                        c[(NS + 3 * q + 2) * NR + b] = (T)((double)dx0 * p0 + (double)hx * (double)acc[k][NS + 3 * q + 1][b]);
+                        for (int q = 0; q < NP; ++q) {
+                            const double p0 = (double)acc[k][NS + 3 * q][b];
+                            c[(NS + 3 * q) * NR + b] = (T)((double)dy * p0);
+                            c[(NS + 3 * q + 1) * NR + b] =
+                                (T)((double)dz0 * p0 + (double)hz * (double)acc[k][NS + 3 * q + 2][b]);
+                            c[(NS + 3 * q + 2) * NR + b] =
+                                (T)((double)dx0 * p0 + (double)hx * (double)acc[k][NS + 3 * q + 1][b]);
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < CN; ++i) all += c[i];
+                    return __builtin_isfinite(all);
+                };
+                if (__ballot(!coefficients()) != 0) {
+                    // a list's zero times an infinity or NaN at a point outside the image is not zero: the
+                    // slot's epoch once more, point by point, without those
+#pragma unroll
+                    for (int i = 0; i < CN; ++i) c[i] = T(0);
+                    for (Step t{s.ep, s.ep * E, s.s0, s.ns, s.off}; t.z < min((s.ep + 1) * E, z1); ++t.z) {
+                        Row<T> q[NB][PW];
+                        load_psi(q, t);
+                        const Vals e = load_vals(t, mask_of(t), k);
+                        T v[NR][VN];
+                        values(q, t.z, v);
+                        const T dz = hz * (((T)t.z - im[3]) - im[2]);
+#pragma unroll
+                        for (int u = 0; u < VN; ++u) {
+                            const T dx = dx0 + (T)u * hx;
+#pragma unroll
+                            for (int b = 0; b < NR; ++b) {
+#pragma unroll
+                                for (int q = 0; q < NS; ++q)
+                                    if (e.f[q].v[u] != T(0)) c[q * NR + b] += e.f[q].v[u] * v[b][u];
+#pragma unroll
+                                for (int q = 0; q < NP; ++q)
+                                    if (e.f[NS + q].v[u] != T(0)) {
+                                        const T w = e.f[NS + q].v[u] * v[b][u];
+                                        c[(NS + 3 * q) * NR + b] += w * dy;
+                                        c[(NS + 3 * q + 1) * NR + b] += w * dz;
+                                        c[(NS + 3 * q + 2) * NR + b] += w * dx;
+                                    }
+                            }
+                        }
                     }
                 }
 #pragma unroll
@@ -837,25 +916,8 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjA
     }
     auto step = [&](auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        // the plane's values as real bands; a point of two overlapping groups counts once
         T v[NR][VN];
-#pragma unroll
-        for (int u = 0; u < VN; ++u) {
-            const bool mine = !RAG || x + u >= xq * VN;
-            if constexpr (CPLX) {
-                const T cz = ez[2 * (cur.z - z0)], sz = ez[2 * (cur.z - z0) + 1];
-                const T er = exy[u][0] * cz - exy[u][1] * sz, ei = exy[u][0] * sz + exy[u][1] * cz;
-#pragma unroll
-                for (int b = 0; b < NB; ++b) {
-                    const T re = p[i][b][2 * u / VN].v[2 * u % VN], im = p[i][b][2 * u / VN].v[2 * u % VN + 1];
-                    v[2 * b][u] = mine ? er * re - ei * im : T(0);
-                    v[2 * b + 1][u] = mine ? er * im + ei * re : T(0);
-                }
-            } else {
-#pragma unroll
-                for (int b = 0; b < NB; ++b) v[b][u] = mine ? p[i][b][0].v[u] : T(0);
-            }
-        }
+        values(p[i], cur.z, v);
         const T zr = (T)(cur.z - cur.ep * E);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
