@@ -140,7 +140,8 @@ static size_t sphere_lds(int nx, int ty, int nb, int ns, int np, int max_col, in
 
 // One workgroup of the apply pass.  NB bands; NS s and NP p channels per image; RAG: Nx is not a
 // multiple of VN (the last group of a row then overlaps its neighbour: both owners compute and
-// write the same values, and LDS is accessed by element); HV halo vectors per thread and band.
+// write the same values, to the bit, so a point's x displacement is formed from its own grid index
+// and not from its group's; LDS is accessed by element); HV halo vectors per thread and band.
 //
 // FORCE: instead of H psi, the nonlocal forces F_a = sum_b (-2 occ_b) sum_i v_ba(i) D psi_b(i), with
 // v_ba = sum_j E_j c_baj beta_aj the value an entry contributes to V_NL psi and D the 8th-order
@@ -441,6 +442,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                 fx = w0.v[0]; fy = w0.v[1]; fz = w1.v[0]; nzf = w1.v[1];
             }
             const T dx0 = hx * ((T)dxi - fx), dy = hy * ((T)dyi - fy), dz = hz * (((T)z - nzf) - fz);
+            auto dx = [&](int u) { return RAG && !FORCE ? hx * ((T)(dxi + u) - fx) : dx0 + (T)u * hx; };
             // inside: leave out points outside the image
             auto bands = [&](auto inside) __attribute__((always_inline)) {
 #pragma unroll
@@ -467,7 +469,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
                         const T cy = c[NS + 3 * p], cz = c[NS + 3 * p + 1], cx = c[NS + 3 * p + 2];
                         const T ayz = cy * dy + cz * dz;
 #pragma unroll
-                        for (int u = 0; u < VN; ++u) val[u] += e.f[NS + p].v[u] * (ayz + cx * (dx0 + (T)u * hx));
+                        for (int u = 0; u < VN; ++u) val[u] += e.f[NS + p].v[u] * (ayz + cx * dx(u));
                     }
 #pragma unroll
                     for (int u = 0; u < VN; ++u) {
@@ -1330,6 +1332,8 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_kpoint_kernel(SphereArgs a
                 fx = w0.v[0]; fy = w0.v[1]; fz = w1.v[0]; nzf = w1.v[1];
             }
             const T dx0 = hx * ((T)dxi - fx), dy = hy * ((T)dyi - fy), dz = hz * (((T)z - nzf) - fz);
+            // as in sphere_body: the same bits from both owners of a point
+            auto dx = [&](int u) { return RAG ? hx * ((T)(dxi + u) - fx) : dx0 + (T)u * hx; };
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 T c[NC];
@@ -1349,7 +1353,7 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_kpoint_kernel(SphereArgs a
                     const T ayz = c[NS + 3 * p] * dy + c[NS + 3 * p + 1] * dz;
 #pragma unroll
                     for (int u = 0; u < VN; ++u)
-                        nl[b][u] += e.f[NS + p].v[u] * (ayz + c[NS + 3 * p + 2] * (dx0 + (T)u * hx));
+                        nl[b][u] += e.f[NS + p].v[u] * (ayz + c[NS + 3 * p + 2] * dx(u));
                 }
             }
         };
