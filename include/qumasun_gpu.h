@@ -265,20 +265,26 @@ int qg_hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int6
  * that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  No counterpart in the reference.  It serves what the row kernels
  * serve (Nx a multiple of 4 in FP32 or of 2 in FP64, 8 <= Nx <= 1024, Gaussian projectors with
- * l <= 1; the sphere passes where they do) and keeps the projector partials and coefficients in one fixed 64 MiB device array per GPU,
- * processing the bands in chunks that fit it; QG_ERR_ARG when one band does not fit or the
+ * l <= 1), through the sphere passes where those serve too and the plan does not ask for the row
+ * kernels, and keeps the projector partials and coefficients in one fixed 64 MiB device array per
+ * GPU, processing the bands in chunks that fit it; QG_ERR_ARG when one band does not fit or the
  * projector geometry is not prepared (qg_nonlocal_create/update prepare it).  Calls on one GPU
  * share that array: calls that overlap on one GPU (other streams, other threads) race. */
 int qg_hamiltonian_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld,
                                  void* hpsi, int64_t ld_out, void* stream);
-/* Kernel plan of a Hamiltonian's H psi (no counterpart in the reference).  The row kernels
- * (a tile-centric projection launch and one stencil + V + projector launch) serve grids with
- * Nx a multiple of 4 (FP32) or 2 (FP64), 8 <= Nx <= 1024, and Gaussian projectors with l <= 1;
- * the table kernels serve everything.  Zero fields are chosen automatically from the grid and
- * the band count.  The QG_ROWS_* environment variables override the shape fields (measurement
+/* Kernel plan of a Hamiltonian's H psi (no counterpart in the reference).  Three families:
+ * - the sphere passes (projector values from entry lists) serve 8 <= Nx <= 1024, Nz >= 8 and atoms
+ *   of at most two s and two p channels, Gaussian or tabulated;
+ * - the row kernels (a tile-centric projection launch and one stencil + V + projector launch) serve
+ *   Nx a multiple of 4 (FP32) or 2 (FP64), 8 <= Nx <= 1024, and Gaussian projectors with l <= 1;
+ * - the table kernels serve everything.
+ * Zero fields are chosen automatically from the grid and the band count.  The shape fields are the
+ * row kernels'; the sphere passes take rows_ty, rows_tz and rows_bands (4 as 2) for their apply pass.
+ * The QG_ROWS_* environment variables override the shape fields of the row kernels (measurement
  * switches). */
-#define QG_KERNELS_AUTO 0     /* row kernels where they serve, table kernels otherwise */
-#define QG_KERNELS_ROWS 1     /* row kernels only (QG_ERR_ARG where they do not serve) */
+#define QG_KERNELS_AUTO 0     /* the first of the three that serves */
+#define QG_KERNELS_ROWS 1     /* row kernels only (QG_ERR_ARG where they do not serve); the geometry
+                                 they need is built by qg_hamiltonian_set_plan and later updates */
 #define QG_KERNELS_TABLES 2   /* table kernels */
 typedef struct qg_hpsi_plan {
     int kernels;      /* QG_KERNELS_* */
@@ -483,10 +489,11 @@ int qg_hamiltonian_set_cnn(qg_ham* h, qg_cnn* c);
  * counterpart in the reference (which runs one cell per process). */
 int qg_batch_hamiltonian_apply(int ncells, qg_ham* const* hams, int dtype, const int* nbands,
                                const void* const* psi, void* const* hpsi, void* stream);
-/* Autotuner: times the fused H psi of h on nbands zero bands for candidate tile shapes (rows
- * per tile x points per thread; fixed_ppt != 0 pins the latter) and records the fastest for
- * this grid shape and dtype; later applications on grids of that shape use it (unless the
- * QG_PLAN_TY / QG_PLAN_PPT environment overrides are set). */
+/* Autotuner of the table kernels: times their fused H psi of h on nbands zero bands for candidate
+ * tile shapes (rows per tile x points per thread; fixed_ppt != 0 pins the latter) and records the
+ * fastest for this grid shape and dtype; later applications of the table kernels on grids of that
+ * shape (a QG_KERNELS_TABLES plan, or where neither the sphere passes nor the row kernels serve) use
+ * it (unless the QG_PLAN_TY / QG_PLAN_PPT environment overrides are set). */
 int qg_autotune_hamiltonian(qg_ham* h, int dtype, int nbands, int fixed_ppt, int* ty, int* ppt,
                             double* best_ms);
 /* LOBPCG for ncells independent cells (arguments per cell as in qg_lobpcg_d_multi).  batched

@@ -1032,8 +1032,9 @@ static int chunk_bands(const qg_grid& g, int dtype, int nbands, bool split) {
 // H psi for a band block, used by qg_hamiltonian_apply and the LOBPCG driver.
 void hamiltonian_apply(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi,
                        int64_t ld_out, hipStream_t s) {
-    // the row kernels (one projection pass, one stencil + V + projector pass) where they
-    // serve the grid and projector set; the table kernels below otherwise
+    // the sphere passes or the row kernels (one projection pass, one stencil + V + projector pass)
+    // where the latter serve the grid and projector set; the table kernels below, or the sphere passes
+    // on other grids and sets, otherwise
     if (rows_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, s, nullptr)) return;
     const qg_grid& g = h->grid;
     qg_nonlocal* nl = (h->nl && h->nl->geo.ncoef > 0) ? h->nl : nullptr;
@@ -1355,7 +1356,7 @@ static void batch_apply_t(const std::vector<BatchReq>& reqs, hipStream_t s, DevB
     QG_HIP(hipStreamSynchronize(s));
 }
 
-// Whether the cell's projection and apply both run on the sphere lists (or it has no projectors).
+// Whether the cell's projection and apply both run on the sphere lists.
 static bool sphere_cell(const BatchReq& r, int dtype, hipStream_t s) {
     if (r.h->plan.kernels != QG_KERNELS_AUTO) return false;
     if (!r.h->nl || r.h->nl->geo.ncoef == 0) return false;
@@ -1728,6 +1729,12 @@ int qg_hamiltonian_set_plan(qg_ham* h, const qg_hpsi_plan* plan) {
         QG_REQUIRE(p.rows_bands == 0 || p.rows_bands == 1 || p.rows_bands == 2 || p.rows_bands == 4,
                    "bands per workgroup must be 1, 2 or 4");
         QG_REQUIRE(p.rows_nbp == 0 || p.rows_nbp == 4 || p.rows_nbp == 8, "projection bands must be 4 or 8");
+        // the allocation-free application expects the row kernels' geometry to be there, now and after every
+        // qg_nonlocal_update
+        if (p.kernels == QG_KERNELS_ROWS && h->nl && !h->nl->rows_wanted) {
+            h->nl->rows_wanted = true;
+            rows_prepare(h->nl);
+        }
         h->plan = p;
     });
 }

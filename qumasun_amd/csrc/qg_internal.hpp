@@ -286,6 +286,7 @@ struct qg_nonlocal {
     qg::DevBuf<int64_t> d_img_tbl_off;
     // row-kernel geometry, one per (tile rows, projection slab) shape in use
     std::vector<std::unique_ptr<qg::RowsGeo>> rows;
+    bool rows_wanted = false;       // a Hamiltonian's plan asks for the row kernels: prepare their geometry
     std::mutex rows_mu;             // guards the creation of entries of `rows` and `sphere`
     // sphere apply kernels: images, channel slots and entry lists per (tile rows, type) in use
     qg::SphereForm sphere_form;

@@ -1202,9 +1202,9 @@ static bool rows_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* hps
     const RowsShape sh = rows_shape(g, dtype, nbands, &h->plan);
     const RowsGeo* rg = nullptr;    // apply kernel's geometry (tile rows ty)
     const RowsGeo* rgp = nullptr;   // projection kernel's geometry (tile rows typ)
-    // both launches from the sphere entry lists where they serve
-    const bool sphere = nl && sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nullptr, ws == nullptr,
-                                                       false, s);
+    // both launches from the sphere entry lists where they serve, unless the plan asks for the row kernels
+    const bool sphere = nl && h->plan.kernels != QG_KERNELS_ROWS &&
+                        sphere_hamiltonian_apply(h, dtype, nbands, psi, ld, hpsi, ld_out, nullptr, ws == nullptr, false, s);
     // doubles of partials there is room for
     const size_t most = !ws || !nl ? SIZE_MAX
                                    : ws->capacity - std::min(ws->capacity, (size_t)nbands * nl->geo.ncoef);
@@ -1371,16 +1371,16 @@ bool rows_laplacian_apply(const qg_grid& g, int dtype, int nbands, const void* p
     return true;
 }
 
-// Builds the row geometry of the default launch shapes (FP32 and FP64) of nl, so that
-// applications find it ready (and applications on caller scratch need not allocate).
+// Builds the row geometry of the default launch shapes (FP32 and FP64) of nl, where applications may
+// need it, so that they find it ready (and applications on caller scratch need not allocate).
 void rows_prepare(qg_nonlocal* nl) {
     if (nl->geo.ncoef == 0) return;
     for (int dtype : {QG_F32, QG_F64}) {
         if (!rows_eligible(nl->gcopy, dtype, nl)) continue;
         const RowsShape sh = rows_shape(nl->gcopy, dtype, 0);
         if (sh.typ == 0) continue;
-        // only where the sphere entry lists do not serve
-        const bool apply = sphere_prepared(nl, dtype);
+        // only where the sphere entry lists do not serve, or a plan asks for the row kernels
+        const bool apply = !nl->rows_wanted && sphere_prepared(nl, dtype);
         if (!apply) rows_geometry(nl, sh.ty, sh.tzp, true);
         if (!apply || sphere_project_need(nl, dtype, 1, false, false) == 0) rows_geometry(nl, sh.typ, sh.tzp, false);
     }
@@ -1432,7 +1432,8 @@ void rows_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64
         const RowsShape sh = rows_shape(g, dtype, nbands, &h->plan);
         QG_REQUIRE(sh.typ > 0, "the projection tile does not fit this grid");
         // bands whose partials and coefficients fit; a band's least need is one slab of partials
-        const size_t one_band = sphere_prepared(nl, dtype) ? sphere_project_need(nl, dtype, 1, false, false, 0) : 0;
+        const bool lists = h->plan.kernels != QG_KERNELS_ROWS && sphere_prepared(nl, dtype);
+        const size_t one_band = lists ? sphere_project_need(nl, dtype, 1, false, false, 0) : 0;
         if (one_band) {
             chunk = sphere_chunk_bands(nbands, one_band, nl->geo.ncoef, kScratchDoubles);
             QG_REQUIRE(chunk > 0, "one band needs " + std::to_string(one_band + nl->geo.ncoef) +
