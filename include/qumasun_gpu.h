@@ -125,7 +125,12 @@ typedef struct qg_nonlocal qg_nonlocal;
  * (in species order).  Replaces PseudoPotIntegrator_mpi::UpdatePosition
  * (PseudoPotOperator_mpi_v2.h:231-248) for one process holding the whole grid:
  * GridForSphere boxes (GridSubgrid.h:483-492), their periodic overlap blocks
- * (GridSubgrid.h:381-430) and the projector/Ylm values on them. */
+ * (GridSubgrid.h:381-430) and the projector/Ylm values on them.
+ * Device memory beside those: the entry lists of the sphere passes, with the geometry for FP32 and
+ * FP64 where qg_hamiltonian_apply_noalloc serves the cell, at first use otherwise and for k points
+ * and plans of another tile height (216 atoms on 120^3, both precisions: 250 MB).  All lists of a
+ * handle take at most a sixteenth of the device's memory; those beyond it, or that the device has no
+ * memory for, are left out, and the row or table kernels serve in their place. */
 int qg_nonlocal_create(const qg_grid* g, int natoms, const double* xyz_host,
                        const int* species_host, int nspecies, const int* nproj_host,
                        const qg_proj_spec* specs, qg_nonlocal** out);

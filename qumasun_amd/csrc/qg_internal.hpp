@@ -76,6 +76,19 @@ struct DevBuf {
         QG_HIP(hipMalloc(&p, count * sizeof(T)));
         n = count;
     }
+    // false where the device has not the memory
+    bool try_alloc(size_t count) {
+        release();
+        const hipError_t e = hipMalloc(&p, count * sizeof(T));
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        QG_HIP(e);
+        n = count;
+        return true;
+    }
     void upload(const T* host, size_t count, hipStream_t s = nullptr) {
         alloc(count);
         if (count) QG_HIP(hipMemcpyAsync(p, host, count * sizeof(T), hipMemcpyHostToDevice, s));
@@ -294,6 +307,7 @@ struct qg_nonlocal {
     qg::DevBuf<qg::SphereImage> d_sphere_img;
     qg::DevBuf<int> d_atom_chan;
     std::vector<std::unique_ptr<qg::SphereGeo>> sphere;
+    size_t sphere_bytes = 0;        // of the lists of all of them
     qg::DevBuf<double> rows_part;   // projector partials of qg_nonlocal_project
     // geometry generation: bumped by every (re)build of the projector geometry, so state derived
     // from it elsewhere (the k-point phase tables) knows when to rebuild

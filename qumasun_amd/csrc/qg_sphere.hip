@@ -273,6 +273,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
     // of exactly the plane's trips, so that those past its last one cost no traffic and every
     // plane issues the same number of loads
     constexpr int K = 3;
+    static_assert(K <= kSphereAhead, "the lists' slack covers the loads ahead");
     struct Entry {
         Row<T> f[NV];
         uint32_t w;
@@ -648,6 +649,7 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjA
     constexpr int NR = CPLX ? 2 * NB : NB;      // real bands
     constexpr int PW = CPLX ? 2 : 1;            // 16-byte vectors per lane and band
     constexpr int K = CPLX && NS == 2 && sizeof(T) == 8 ? 2 : 4;   // slots held at once (4 would spill there)
+    static_assert(K <= kSphereAhead, "the lists' slack covers the loads ahead");
     constexpr int E = kProjPlanes;
     extern __shared__ __align__(16) unsigned char smem[];
     const int nx = a.nx, ny = a.ny, nz = a.nz;
@@ -1056,6 +1058,7 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_kpoint_kernel(SphereArgs a
     constexpr int NC = NS + 3 * NP;
     constexpr int NV = NS + NP;
     constexpr int K = 3;
+    static_assert(K <= kSphereAhead, "the lists' slack covers the loads ahead");
     extern __shared__ __align__(16) unsigned char smem[];
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const int W = RAG ? (nx + 8 + VN - 1) / VN * VN : nx + 8;
@@ -1700,7 +1703,28 @@ static void sphere_images(qg_nonlocal* nl) {
     nl->d_atom_chan.upload(chan.data(), chan.size());
 }
 
-// Entry lists of tile rows ty for the block type, built on the device on first use.
+// Bytes the lists of one projector set may take, all its tile heights and types together: a sixteenth of
+// the device's memory (18 GB of 288; 216 atoms on 120^3 take 250 MB in both types).  QG_SPHERE_KB: another number of
+// KiB (measurement switch).
+static size_t sphere_list_budget() {
+    const int kb = env_int("QG_SPHERE_KB", -1);
+    if (kb >= 0) return (size_t)kb << 10;
+    static std::mutex mu;
+    static size_t total[64] = {};
+    int dev = 0;
+    QG_HIP(hipGetDevice(&dev));
+    if (dev < 0 || dev >= 64) return (size_t)4 << 30;
+    std::lock_guard<std::mutex> lk(mu);
+    if (!total[dev]) {
+        size_t free = 0;
+        QG_HIP(hipMemGetInfo(&free, &total[dev]));
+    }
+    return total[dev] / 16;
+}
+
+// Entry lists of tile rows ty for the block type, built on the device on first use.  Lists beyond the
+// budget, or that the device has no memory for, are left out until the next update of the nuclei: the
+// row or table kernels serve in their place (ok, slots_ok false).
 static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build) {
     std::lock_guard<std::mutex> lk(nl->rows_mu);
     for (auto& c : nl->sphere)
@@ -1801,25 +1825,35 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
         };
         int most_trips = 0, most_slots = 0;
         const int64_t trips = scan(cnt.data(), nwv, most_trips), slots = scan(cnt.data() + nwv + 1, ne, most_slots);
-        if (trips < (1LL << 30)) {
-            const size_t nv = nl->sphere_form.ns + nl->sphere_form.np;
-            c->slots_ok = most_slots <= 32 && slots < (1LL << 28);
-            c->ntrips = (int)std::max<int64_t>(1, trips);
-            const size_t nt = c->ntrips, ns = c->slots_ok ? (size_t)std::max<int64_t>(1, slots) : 0;
+        const int nv = nl->sphere_form.ns + nl->sphere_form.np;
+        const size_t nt = (size_t)std::max<int64_t>(1, trips);
+        const bool may_slots = most_slots <= 32 && slots < (1LL << 28);
+        const size_t budget = sphere_list_budget(), room = budget - std::min(budget, nl->sphere_bytes);
+        int fit = trips < (1LL << 30)
+                      ? sphere_lists_that_fit(nv, nt, may_slots ? (size_t)std::max<int64_t>(1, slots) : 0, room)
+                      : 0;
+        if (fit == 2 && !may_slots) fit = 1;
+        SphereListLayout l{};
+        for (; fit > 0; --fit) {
+            l = sphere_list_layout(nv, nt, fit == 2 ? (size_t)std::max<int64_t>(1, slots) : 0);
+            if (c->lists.try_alloc(l.bytes)) break;
+        }
+        if (fit > 0) {
+            c->slots_ok = fit == 2;
+            c->ntrips = (int)nt;
+            nl->sphere_bytes += l.bytes;
             QG_HIP(hipMemcpyAsync(c->counts.p, cnt.data(), cnt.size() * sizeof(int), hipMemcpyHostToDevice, nullptr));
-            c->lists.alloc(1024 * nv * (nt + ns * kProjPlanes) + 256 * (nt + ns));
             unsigned char* v = c->lists.p;
-            c->vals = v;
-            c->slot_vals = v + 1024 * nv * nt;
-            uint32_t* w = reinterpret_cast<uint32_t*>(v + 1024 * nv * (nt + ns * kProjPlanes));
-            c->words = w;
-            c->slot_words = w + 64 * nt;
+            c->vals = v + l.vals;
+            c->slot_vals = v + l.slot_vals;
+            c->words = reinterpret_cast<uint32_t*>(v + l.words);
+            c->slot_words = reinterpret_cast<uint32_t*>(v + l.slot_words);
             a.trip_off = c->trip_off;
-            a.words = w;
-            a.vals = v;
+            a.words = const_cast<uint32_t*>(c->words);
+            a.vals = const_cast<void*>(c->vals);
             s.trip_off = c->slot_off;
-            s.words = w + 64 * nt;
-            s.vals = v + 1024 * nv * nt;
+            s.words = const_cast<uint32_t*>(c->slot_words);
+            s.vals = const_cast<void*>(c->slot_vals);
             dtype == QG_F32 ? build(float{}, std::true_type{}, c->slots_ok) : build(double{}, std::true_type{}, c->slots_ok);
             c->ok = true;
         }
@@ -1834,6 +1868,7 @@ static SphereGeo* sphere_geometry(qg_nonlocal* nl, int dtype, int ty, bool build
 // use).
 void sphere_prepare(qg_nonlocal* nl) {
     nl->sphere.clear();
+    nl->sphere_bytes = 0;
     sphere_images(nl);
     if (!sphere_serves(nl->gcopy, nl)) return;
     for (int dtype : {QG_F32, QG_F64}) {
@@ -2145,10 +2180,10 @@ static bool sphere_apply_t(qg_ham* h, int nbands, const T* psi, int64_t ld, T* h
     int ty = sphere_pick_ty(nq, g.n[1], h->plan.rows_ty);
     if (ty == 0) return false;
     const SphereGeo* sg = sphere_geometry(nl, dtype, ty, may_build);
-    if (!sg && h->plan.rows_ty > 0) {
-        // nothing may be built now: the tile height prepared with the geometry
+    if ((!sg || !sg->ok) && h->plan.rows_ty > 0) {
+        // nothing may be built now, or not these: the tile height prepared with the geometry
         ty = sphere_pick_ty(nq, g.n[1], 0);
-        sg = sphere_geometry(nl, dtype, ty, false);
+        sg = sphere_geometry(nl, dtype, ty, may_build);
     }
     if (!sg || !sg->ok) return false;
     const bool two = nl->sphere_form.ns == 2;

@@ -38,4 +38,34 @@ inline int sphere_chunk_bands(int nbands, size_t per_band, size_t ncoef, size_t 
     return (int)((nbands + chunks - 1) / std::max<int64_t>(1, chunks));
 }
 
+// Byte offsets of the entry lists of one tile height and type in their one allocation: values and words
+// of the apply's trips and of the projection's slots (nv radial vectors each).
+//
+// The kernels issue the loads of their first kSphereAhead entries of a plane or epoch without a look at
+// their number, through buffer resources that end at the last one.  Whether the offset of such a load
+// counts in the range check is the hardware's affair: the slack keeps what the loads can address inside
+// the allocation either way.
+constexpr int kSphereAhead = 4;
+
+struct SphereListLayout {
+    size_t vals, slot_vals, words, slot_words, bytes;
+};
+
+inline SphereListLayout sphere_list_layout(int nv, size_t trips, size_t slots) {
+    SphereListLayout l;
+    l.vals = 0;
+    l.slot_vals = (size_t)1024 * nv * trips;
+    l.words = l.slot_vals + (size_t)1024 * nv * slots * kProjPlanes;
+    l.slot_words = l.words + (size_t)256 * trips;
+    l.bytes = l.slot_words + (size_t)256 * slots + (size_t)1024 * nv * kSphereAhead;
+    return l;
+}
+
+// What of a tile height's lists may be built where `room` bytes are left: 2 trips and slots, 1 the trips
+// alone (another projection serves), 0 neither.
+inline int sphere_lists_that_fit(int nv, size_t trips, size_t slots, size_t room) {
+    if (sphere_list_layout(nv, trips, slots).bytes <= room) return 2;
+    return sphere_list_layout(nv, trips, 0).bytes <= room ? 1 : 0;
+}
+
 }  // namespace qg

@@ -1,6 +1,8 @@
 // Host driver of qg_sphere_plan.hpp: prints what the sphere passes' size rules give.
 //   chunks <nbands> <ntile> <max_col> <nc> <ncoef> <bands per workgroup> <nz> <capacity>
 //       -> chunk, then for every chunk "bands slabs planes doubles"
+//   lists <nv> <trips> <slots> <room>
+//       -> "vals slot_vals words slot_words bytes fit", all but the last in bytes
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -20,6 +22,14 @@ int main(int argc, char** argv) {
                 qg::sphere_project_slabs(nz, (int64_t)ntile * ((n + nb - 1) / nb), slab1 * n, room);
             std::printf("%d %d %d %zu\n", n, s.nslab, s.tz, slab1 * n * s.nslab + (size_t)n * ncoef);
         }
+        return 0;
+    }
+    if (argc == 6 && !std::strcmp(argv[1], "lists")) {
+        const int nv = std::atoi(argv[2]);
+        const size_t trips = std::strtoull(argv[3], nullptr, 10), slots = std::strtoull(argv[4], nullptr, 10);
+        const qg::SphereListLayout l = qg::sphere_list_layout(nv, trips, slots);
+        std::printf("%zu %zu %zu %zu %zu %d\n", l.vals, l.slot_vals, l.words, l.slot_words, l.bytes,
+                    qg::sphere_lists_that_fit(nv, trips, slots, std::strtoull(argv[5], nullptr, 10)));
         return 0;
     }
     return 2;

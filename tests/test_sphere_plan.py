@@ -4,7 +4,10 @@ Chunks of the allocation-free application: for every band count, each chunk (the
 fits the fixed scratch, the chunks cover the bands, and the slabs of a chunk cover the grid.  Cells:
 (tile columns, most images of one, channels, coefficients, bands per workgroup, planes) of 216 atoms on
 120^3 in FP32 and FP64, 512 atoms on 128^3, 1000 atoms on 120^3 in FP64, and one band that fills the
-scratch by itself."""
+scratch by itself.
+
+Entry lists: their parts do not overlap, every load that the kernels issue ahead lies inside the
+allocation (also where an offset past a list's last entry is not checked), and what is built fits."""
 import os
 import shutil
 import subprocess
@@ -50,3 +53,25 @@ def test_every_chunk_fits(plan, cell):
 def test_band_that_does_not_fit(plan):
     assert plan("chunks", 3, 1000, 1000, 8, 8, 4, 64, CAPACITY) == ["1"] + ["1 1 64 8000008"] * 3
     assert plan("chunks", 3, 1100, 1000, 8, 8, 4, 64, CAPACITY) == ["0"]
+
+
+@pytest.mark.parametrize("nv", [2, 4])
+@pytest.mark.parametrize("trips,slots", [(1, 0), (1, 1), (1, 2), (7, 3), (5000, 900), (1 << 20, 0)])
+def test_list_layout(plan, nv, trips, slots):
+    vals, slot_vals, words, slot_words, size, _ = map(int, plan("lists", nv, trips, slots, 0)[0].split())
+    ahead = 4                       # entries a wavefront loads before it looks at their number
+    assert vals == 0 and slot_vals >= vals + 1024 * nv * trips
+    assert words >= slot_vals + 1024 * nv * 8 * slots and slot_words >= words + 256 * trips
+    assert size >= slot_words + 256 * slots
+    # from the end of the last plane's entries; a slot without points is addressed from the lists' start
+    assert vals + 1024 * nv * (trips + ahead) <= size and words + 256 * (trips + ahead) <= size
+    assert slot_vals + 1024 * nv * 8 * slots + 1024 * nv <= size and slot_words + 256 * (slots + ahead) <= size
+
+
+def test_lists_within_their_room(plan):
+    def fit(room):
+        return int(plan("lists", 2, 1000, 400, room)[0].split()[5])
+
+    both, trips = (int(plan("lists", 2, 1000, n, 0)[0].split()[4]) for n in (400, 0))
+    assert trips < both
+    assert [fit(r) for r in (0, trips - 1, trips, both - 1, both, 2 ** 63)] == [0, 0, 1, 1, 2, 2]
