@@ -375,8 +375,8 @@ typedef struct qg_lobpcg_opts {
     void* watch_user;
     int orth;                /* QG_ORTH_* (orthonormal basis only) */
     int gram_chunks;         /* K chunks of the split-K library Gram products (each chunk summed
-                                in the block precision, the chunks in FP64); 0: this engine's
-                                matrix-core kernel in FP64 (64 chunks where it does not serve),
+                                in the block precision, the chunks in FP64); 0: in FP64 this engine's
+                                matrix-core kernel or 64 chunks, whichever is faster at the size,
                                 chunks of at most ~6,750 terms in FP32 (256 at 120^3: longer FP32
                                 partial sums stalled the FP32 phase at 512 bands) */
     double reortho;          /* orthonormal basis: a second orthonormalisation pass runs when the

@@ -1,6 +1,7 @@
 // FP64 products of tall blocks (K grid points x a few hundred bands) on the FP64 matrix cores: the Gram
 // blocks C = A^T B of the Rayleigh-Ritz step and the Ritz update Out = A C.  Columns (bands) are
 // contiguous over the grid.
+#include "qg_gram64_split.hpp"
 #include "qg_internal.hpp"
 
 #include <algorithm>
@@ -142,9 +143,9 @@ __device__ __forceinline__ void gram64_wave(const GramArgs& g, unsigned char* sm
 // while one is in use.  Bands past the last read the last one, points past the last become zeros.
 // Bound by the FP64 matrix rate and, below ~100 bands, by memory; the wavefronts of a step are uneven
 // (144 bands: 23 of 20.25 tiles on the fullest SIMD).  Against the library's strided-batched product in
-// 64 ranges, us, both without the sum over the ranges: 512,000 points x 8 x 8 52 : 248, 64 x 64 134 : 328,
-// 96 x 96 228 : 325, 144 x 144 470 : 753 (floors 250 of memory, 300 of 71 TFLOP/s); 13,824 x 16 x 16
-// 18 : 129; 768,000 x 192 x 192 1128 : 1965; 1,728,000 x 432 x 432 12,800 : 13,500.
+// 64 ranges, us: 512,000 points x 8 x 8 75 : 269, 64 x 64 163 : 336, 96 x 96 257 : 338, 144 x 144
+// 490 : 757 (300 at 71 TFLOP/s); 13,824 x 16 x 16 25 : 138; where the library's tiles are full it is the
+// faster one (gram64_faster).
 template <int TM, int TN>
 __global__ __launch_bounds__(kGramThreads, 2) void gram64_kernel(GramArgs g) {
     extern __shared__ __align__(16) unsigned char gsmem[];
@@ -183,33 +184,13 @@ __global__ __launch_bounds__(256) void gram64_reduce_kernel(const double* __rest
                                               part[3][threadIdx.x];
 }
 
-struct GramSplit {
-    int mb, nb, bm, bn;     // blocks, and the tiles of the largest
-    int64_t nch, per;
-};
-
-// The tiles in the fewest blocks of at most 10 x 12, as even as they go; one workgroup per CU in all (its
-// accumulators take the registers), or four where the blocks alone come near that; no range shorter than
-// 512 points
-static GramSplit gram64_split(int64_t K, int M, int N) {
-    GramSplit g;
-    const int mt = (M + 15) / 16, nt = (N + 15) / 16;
-    g.mb = (mt + 9) / 10;
-    g.nb = (nt + 11) / 12;
-    g.bm = (mt + g.mb - 1) / g.mb;
-    g.bn = (nt + g.nb - 1) / g.nb;
-    const int blocks = g.mb * g.nb;
-    const int64_t want = std::min<int64_t>((K + 511) / 512, blocks <= 32 ? 256 / blocks : (1024 + blocks - 1) / blocks);
-    g.per = ((K + want - 1) / want + 15) / 16 * 16;
-    g.nch = (K + g.per - 1) / g.per;
-    return g;
-}
-
 size_t gram64_workspace(int64_t K, int M, int N) { return (size_t)gram64_split(K, M, N).nch * M * N * sizeof(double); }
 
-bool gram64_serves(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N) {
+// Whether the operands suit the kernel (whole 16-byte vectors) and it is the faster one against the
+// library's product in `chunks` chunks
+bool gram64_serves(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N, int64_t chunks) {
     return K >= 2 && K % 2 == 0 && M > 0 && N > 0 && lda % 2 == 0 && ldb % 2 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
-           reinterpret_cast<uintptr_t>(B) % 16 == 0;
+           reinterpret_cast<uintptr_t>(B) % 16 == 0 && gram64_faster(K, M, N, chunks);
 }
 
 // C (M x N, column stride ldc) = A^T B over K points

@@ -110,7 +110,7 @@ void gram_bf16(const float* A, const float* B, int64_t K, int M, int N, int64_t 
                double* C, int ldc, float* partial, size_t partial_floats, hipStream_t s, bool split);
 size_t gram_bf16_workspace(int64_t K, int M, int N);
 size_t gram64_workspace(int64_t K, int M, int N);
-bool gram64_serves(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N);
+bool gram64_serves(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N, int64_t chunks);
 void gram64(const double* A, int64_t lda, const double* B, int64_t ldb, int64_t K, int M, int N, double* C, int ldc,
             double* ws, size_t ws_bytes, hipStream_t s);
 bool update64(const double* A, int64_t lda, const double* C, int ldc, int64_t K, int N, double alpha, double beta,
@@ -260,20 +260,20 @@ static size_t gram_workspace(int64_t K, int M, int N, int want = 0) {
 
 // C (M x N, FP64, column stride ldc) = A^T B over K rows; A: M columns of length K (column m
 // at A + m lda), B: N columns (ld ldb).  The Gram blocks of the Rayleigh-Ritz matrices
-// (MakeMatrix_d_blas, lobpcg_d_multi_mpi.h:192-250).  FP64: the matrix-core kernel of
-// qg_dense64.hip (faster at every size measured there), unless the caller chose the number of
-// chunks or a column is not 16-byte aligned.  Otherwise split-K over the rows as one strided-batched library GEMM in the block
+// (MakeMatrix_d_blas, lobpcg_d_multi_mpi.h:192-250).  FP64: the matrix-core kernel of qg_dense64.hip
+// where it is the faster one (gram64_faster), unless the caller chose the number of chunks or a column is
+// not 16-byte aligned.  Otherwise split-K over the rows as one strided-batched library GEMM in the block
 // precision (enough parallel work for small M, N), then the chunks summed in FP64.
 template <class T>
 static void gram_splitk(rocblas_handle hb, hipStream_t s, const T* A, int64_t lda, const T* B, int64_t ldb, int64_t K,
                         int M, int N, double* C, int ldc, T* ws, size_t ws_bytes, int want_chunks = 0) {
+    const int64_t nch = gram_chunks<T>(K, want_chunks);
     if constexpr (sizeof(T) == 8) {
-        if (want_chunks <= 0 && gram64_serves(A, lda, B, ldb, K, M, N)) {
+        if (want_chunks <= 0 && gram64_serves(A, lda, B, ldb, K, M, N, nch)) {
             gram64(A, lda, B, ldb, K, M, N, C, ldc, ws, ws_bytes, s);
             return;
         }
     }
-    const int64_t nch = gram_chunks<T>(K, want_chunks);
     const int64_t kc = K / nch;
     const int64_t rem = K - nch * kc;
     const int64_t nn = (int64_t)M * N;
