@@ -13,6 +13,7 @@
 #include <mutex>
 #include <vector>
 #include "qg_internal.hpp"
+#include "qg_plan_store.hpp"
 
 namespace qg {
 
@@ -25,9 +26,6 @@ namespace qg {
 
 // FFT plans of one (precision, batch) of the Hamiltonian's grid
 struct FftPair {
-    int prec = -1;
-    int batch = 0;
-    uint64_t used = 0;           // last use, for replacement
     size_t work = 0;
     rocfft_plan fwd = nullptr, inv = nullptr;
     void release() {
@@ -41,14 +39,12 @@ struct FftPair {
 // learned preconditioner between band counts; making a pair takes milliseconds), their scratch
 // and the symbol.
 struct PrecondPlan {
-    static constexpr int kPairs = 4;
-    FftPair pairs[kPairs];
-    uint64_t uses = 0;
+    PlanStore<FftPair, 4> pairs;
+    MadeOnce symbol;
     rocfft_execution_info info = nullptr;
     DevBuf<unsigned char> work, spec;
     DevBuf<double> tx, ty, tz;   // 1-D symbol parts
     ~PrecondPlan() {
-        for (FftPair& p : pairs) p.release();
         if (info) rocfft_execution_info_destroy(info);
     }
 };
@@ -102,47 +98,39 @@ void precond_apply(qg_ham* h, int kind, double shift, int dtype, int nbands, voi
     const int batch = (int)std::max<int64_t>(1, std::min<int64_t>(nbands, (256ll << 20) / (nspec * 2 * es)));
     if (!h->precond) h->precond = new PrecondPlan;
     PrecondPlan& store = *h->precond;
-    if (!store.info) {
-        QG_FFT(rocfft_execution_info_create(&store.info));
+    if (!store.info) QG_FFT(rocfft_execution_info_create(&store.info));
+    store.symbol([&] {
         auto a = kinetic_symbol_1d(nx, g.h[0], nxh);
         auto b = kinetic_symbol_1d(ny, g.h[1], ny);
         auto c = kinetic_symbol_1d(nz, g.h[2], nz);
         store.tx.upload(a.data(), a.size());
         store.ty.upload(b.data(), b.size());
         store.tz.upload(c.data(), c.size());
-    }
-    FftPair* pair = nullptr;
-    for (FftPair& p : store.pairs)
-        if (p.fwd && p.inv && p.prec == dtype && p.batch == batch) pair = &p;
-    if (!pair) {
-        pair = &store.pairs[0];
-        for (FftPair& p : store.pairs)
-            if (p.used < pair->used) pair = &p;
+    });
+    const FftPair& pair = store.pairs.get(
+        dtype, batch,
         // a replaced pair may still be running
-        if (pair->fwd) QG_HIP(hipStreamSynchronize(s));
-        pair->release();
-        const size_t len[3] = {(size_t)nx, (size_t)ny, (size_t)nz};
-        const rocfft_precision p = dtype == QG_F32 ? rocfft_precision_single : rocfft_precision_double;
-        QG_FFT(rocfft_plan_create(&pair->fwd, rocfft_placement_notinplace, rocfft_transform_type_real_forward, p, 3, len,
-                                  batch, nullptr));
-        QG_FFT(rocfft_plan_create(&pair->inv, rocfft_placement_notinplace, rocfft_transform_type_real_inverse, p, 3, len,
-                                  batch, nullptr));
-        size_t w1 = 0, w2 = 0;
-        QG_FFT(rocfft_plan_get_work_buffer_size(pair->fwd, &w1));
-        QG_FFT(rocfft_plan_get_work_buffer_size(pair->inv, &w2));
-        pair->prec = dtype;
-        pair->batch = batch;
-        pair->work = std::max<size_t>(1, std::max(w1, w2));
-    }
-    pair->used = ++store.uses;
-    store.work.alloc(pair->work);
+        [&] { QG_HIP(hipStreamSynchronize(s)); },
+        [&](FftPair& made) {
+            const size_t len[3] = {(size_t)nx, (size_t)ny, (size_t)nz};
+            const rocfft_precision p = dtype == QG_F32 ? rocfft_precision_single : rocfft_precision_double;
+            QG_FFT(rocfft_plan_create(&made.fwd, rocfft_placement_notinplace, rocfft_transform_type_real_forward, p, 3,
+                                      len, batch, nullptr));
+            QG_FFT(rocfft_plan_create(&made.inv, rocfft_placement_notinplace, rocfft_transform_type_real_inverse, p, 3,
+                                      len, batch, nullptr));
+            size_t w1 = 0, w2 = 0;
+            QG_FFT(rocfft_plan_get_work_buffer_size(made.fwd, &w1));
+            QG_FFT(rocfft_plan_get_work_buffer_size(made.inv, &w2));
+            made.work = std::max<size_t>(1, std::max(w1, w2));
+        });
+    store.work.alloc(pair.work);
     store.spec.alloc((size_t)nspec * batch * 2 * es);
     struct {
         rocfft_plan fwd, inv;
         rocfft_execution_info info;
         DevBuf<unsigned char>&work, &spec;
         DevBuf<double>&tx, &ty, &tz;
-    } pl{pair->fwd, pair->inv, store.info, store.work, store.spec, store.tx, store.ty, store.tz};
+    } pl{pair.fwd, pair.inv, store.info, store.work, store.spec, store.tx, store.ty, store.tz};
     QG_FFT(rocfft_execution_info_set_stream(pl.info, s));
     QG_FFT(rocfft_execution_info_set_work_buffer(pl.info, pl.work.p, pl.work.n));
     for (int b0 = 0; b0 < nbands; b0 += batch) {
