@@ -207,10 +207,10 @@ int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void*
         const qg_grid& g = nl->gcopy;
         const int64_t ng = g.ng();
         const size_t es = dtype == QG_F32 ? 4 : 8;
-        // FP64 states: one pass over psi.  FP32 states keep the chain below and its kernels: the FP64 forces
+        // FP64 states: one pass over psi.  FP32 states run the chain below and its kernels: the FP64 forces
         // of FP32 arithmetic follow its order of rounding (another order moves them by 6e-7)
-        if (dtype == QG_F64 && sphere_nonlocal_force(nl, dtype, 1, nullptr, nullptr, psi, ld, nullptr, nl->force_part, nullptr,
-                                                 false, s)) {
+        if (dtype == QG_F64 && sphere_nonlocal_force(nl, 1, nullptr, nullptr, (const double*)psi, ld, nullptr,
+                                                     nl->force_part, nullptr, false, s)) {
             // the occupied states: their projections (in runs of consecutive bands), then forces
             // and energies on the device
             std::vector<int> occupied;
@@ -243,8 +243,8 @@ int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void*
                 k0 = k1;
             }
             if (forces_host)
-                (void)sphere_nonlocal_force(nl, dtype, nocc, nl->force_idx.p, w, psi, ld, c, nl->force_part, res + nocc,
-                                            true, s);
+                (void)sphere_nonlocal_force(nl, nocc, nl->force_idx.p, w, (const double*)psi, ld, c, nl->force_part,
+                                            res + nocc, true, s);
             hipLaunchKernelGGL(band_energy_kernel, dim3(nocc), dim3(64), 0, s, c, nl->d_coef_energy.p, ncoef, w, -0.5, res);
             QG_HIP(hipGetLastError());
             host.resize(nout);

@@ -345,9 +345,8 @@ bool sphere_kpoint_apply(qg_ham* h, const double* k, int dtype, int nbands, cons
 size_t sphere_project_need(qg_nonlocal* nl, int dtype, int nbands, bool cplx, bool may_build, size_t most = SIZE_MAX);
 bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld, const double* k, double* part,
                     double* coef, bool may_build, hipStream_t s, size_t most = SIZE_MAX);
-bool sphere_nonlocal_force(qg_nonlocal* nl, int dtype, int nocc, const int* band_idx, const double* weight,
-                           const void* psi, int64_t ld, const double* coef, DevBuf<double>& part, double* force,
-                           bool run, hipStream_t s);
+bool sphere_nonlocal_force(qg_nonlocal* nl, int nocc, const int* band_idx, const double* weight, const double* psi,
+                           int64_t ld, const double* coef, DevBuf<double>& part, double* force, bool run, hipStream_t s);
 size_t lds_limit();
 double* scratch_address();
 void rows_apply_noalloc(qg_ham* h, int dtype, int nbands, const void* psi, int64_t ld, void* hpsi, int64_t ld_out,

@@ -557,13 +557,14 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_hpsi_kernel(SphereArgs a, 
     sphere_body<T, NB, NS, NP, RAG, HV>(a, sc, V, psi, out, xcd_order(blockIdx.x, gridDim.x), smem);
 }
 
-// The nonlocal force pass: psi is read once (the chain of gradient blocks and their projections
-// moved psi eight times: 64 atoms, 80^3, 137 occupied FP64 bands 1.45 ms after the projection of
+// The nonlocal force pass of FP64 bands: psi is read once (the chain of gradient blocks and their
+// projections moved psi eight times: 64 atoms, 80^3, 137 occupied bands 1.45 ms after the projection of
 // psi, 0.53 ms here).
-template <class T, int NB, int NS, int NP, bool RAG, int HV>
-__global__ __launch_bounds__(kMaxThreads) void sphere_force_kernel(SphereArgs a, Coef8<T> sc, const T* __restrict__ psi) {
+template <int NB, int NS, int NP, bool RAG, int HV>
+__global__ __launch_bounds__(kMaxThreads) void sphere_force_kernel(SphereArgs a, Coef8<double> sc,
+                                                                   const double* __restrict__ psi) {
     extern __shared__ __align__(16) unsigned char smem[];
-    sphere_body<T, NB, NS, NP, RAG, HV, true>(a, sc, nullptr, psi, nullptr, xcd_order(blockIdx.x, gridDim.x), smem);
+    sphere_body<double, NB, NS, NP, RAG, HV, true>(a, sc, nullptr, psi, nullptr, xcd_order(blockIdx.x, gridDim.x), smem);
 }
 
 // force[atom][3]: the atom's partials, over its (tile, column image) pairs and their workgroups in
@@ -2090,37 +2091,38 @@ bool sphere_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int
     return sphere_project_t<double>(nl, nbands, (const double*)psi, ld, k, part, coef, may_build, most, s);
 }
 
-template <class T, int NB, int NS, int NP>
-static void sphere_force_launch(const SphereArgs& a, const Coef8<T>& sc, const T* psi, size_t lds, hipStream_t s) {
+template <int NB, int NS, int NP>
+static void sphere_force_launch(const SphereArgs& a, const Coef8<double>& sc, const double* psi, size_t lds, hipStream_t s) {
     const int64_t nwg = (int64_t)a.ntile * a.nslab * ((a.nbands + NB - 1) / NB);
     QG_REQUIRE(nwg < (1LL << 31), "too many workgroups");
     const dim3 grid((unsigned)nwg), blk(a.tpb);
-    const bool rag = a.nx % (16 / (int)sizeof(T)) != 0;
+    const bool rag = a.nx % 2 != 0;
     const int hv = sphere_halo_vectors(a.nq, a.tpb);
     QG_REQUIRE(hv <= (NB == 1 ? 8 : 1), "row tile too low for its halo");
     if (hv <= 1) {
-        if (rag) hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, true, 1>), grid, blk, lds, s, a, sc, psi);
-        else hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, false, 1>), grid, blk, lds, s, a, sc, psi);
+        if (rag) hipLaunchKernelGGL((sphere_force_kernel<NB, NS, NP, true, 1>), grid, blk, lds, s, a, sc, psi);
+        else hipLaunchKernelGGL((sphere_force_kernel<NB, NS, NP, false, 1>), grid, blk, lds, s, a, sc, psi);
     } else if constexpr (NB == 1) {
-        if (rag) hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, true, 8>), grid, blk, lds, s, a, sc, psi);
-        else hipLaunchKernelGGL((sphere_force_kernel<T, NB, NS, NP, false, 8>), grid, blk, lds, s, a, sc, psi);
+        if (rag) hipLaunchKernelGGL((sphere_force_kernel<NB, NS, NP, true, 8>), grid, blk, lds, s, a, sc, psi);
+        else hipLaunchKernelGGL((sphere_force_kernel<NB, NS, NP, false, 8>), grid, blk, lds, s, a, sc, psi);
     }
     QG_HIP(hipGetLastError());
 }
 
-template <class T>
-static bool sphere_force_t(qg_nonlocal* nl, int nocc, const int* band_idx, const double* weight, const T* psi, int64_t ld,
-                           const double* coef, DevBuf<double>& part, double* force, bool run, hipStream_t s) {
+// force[atom][3] (device) = sum_b weight_b sum_j E_j c_baj dV sum_i beta_aj D psi_b over the FP64 bands
+// band_idx[0 .. nocc) of psi (device arrays), coef their projections in that order.  False (nothing
+// launched) where the entry lists do not serve the grid or projector set; run false only says so.
+bool sphere_nonlocal_force(qg_nonlocal* nl, int nocc, const int* band_idx, const double* weight, const double* psi,
+                           int64_t ld, const double* coef, DevBuf<double>& part, double* force, bool run, hipStream_t s) {
+    if (!sphere_serves(nl->gcopy, nl)) return false;
     const qg_grid& g = nl->gcopy;
-    constexpr int VN = 16 / sizeof(T);
-    const int dtype = sizeof(T) == 4 ? QG_F32 : QG_F64;
-    const int nq = (g.n[0] + VN - 1) / VN;
+    const int nq = (g.n[0] + 1) / 2;
     const int ty = sphere_pick_ty(nq, g.n[1], 0);
-    const SphereGeo* sg = ty > 0 ? sphere_geometry(nl, dtype, ty, true) : nullptr;
+    const SphereGeo* sg = ty > 0 ? sphere_geometry(nl, QG_F64, ty, true) : nullptr;
     if (!sg || !sg->ok || sphere_halo_vectors(nq, sg->tpb) > 8) return false;
     const int nw = sg->tpb / 64;
     auto lds_of = [&](int b) {
-        return sphere_lds<T>(g.n[0], ty, b, nl->sphere_form.ns, nl->sphere_form.np, sg->max_col, nw);
+        return sphere_lds<double>(g.n[0], ty, b, nl->sphere_form.ns, nl->sphere_form.np, sg->max_col, nw);
     };
     // two bands share an entry, its running sums and their LDS updates (64 atoms, 80^3, 137 FP64
     // bands: 0.83 ms a call against 1.0 with one); 2 + 2 channels of two bands would spill
@@ -2137,36 +2139,24 @@ static bool sphere_force_t(qg_nonlocal* nl, int nocc, const int* band_idx, const
     part.alloc((size_t)a.ntile * per_tile * std::max(1, a.max_col) * 3);
     a.part = part.p;
     // 8th-order first-difference weights, dV of the projection's dot product in them
-    Coef8<T> sc{};
+    Coef8<double> sc{};
     const double w[4] = {672.0, -168.0, 32.0, -3.0};
     for (int m = 0; m < 4; ++m) {
-        sc.cx[m] = (T)(g.dvol() * w[m] / (840.0 * g.h[0]));
-        sc.cy[m] = (T)(g.dvol() * w[m] / (840.0 * g.h[1]));
-        sc.cz[m] = (T)(g.dvol() * w[m] / (840.0 * g.h[2]));
+        sc.cx[m] = g.dvol() * w[m] / (840.0 * g.h[0]);
+        sc.cy[m] = g.dvol() * w[m] / (840.0 * g.h[1]);
+        sc.cz[m] = g.dvol() * w[m] / (840.0 * g.h[2]);
     }
     const size_t lds = lds_of(nb);
     if (nl->sphere_form.ns == 2) {
-        sphere_force_launch<T, 1, 2, 2>(a, sc, psi, lds, s);
+        sphere_force_launch<1, 2, 2>(a, sc, psi, lds, s);
     } else {
-        if (nb == 2) sphere_force_launch<T, 2, 1, 1>(a, sc, psi, lds, s);
-        else sphere_force_launch<T, 1, 1, 1>(a, sc, psi, lds, s);
+        if (nb == 2) sphere_force_launch<2, 1, 1>(a, sc, psi, lds, s);
+        else sphere_force_launch<1, 1, 1>(a, sc, psi, lds, s);
     }
     hipLaunchKernelGGL(sphere_force_reduce_kernel, dim3(nl->geo.natoms), dim3(256), 0, s, a.part, sg->atom_ref_off,
                        sg->atom_ref, per_tile, a.max_col, force);
     QG_HIP(hipGetLastError());
     return true;
-}
-
-// force[atom][3] (device) = sum_b weight_b sum_j E_j c_baj dV sum_i beta_aj D psi_b over the bands
-// band_idx[0 .. nocc) of psi (device arrays), coef their projections in that order.  False (nothing
-// launched) where the entry lists do not serve the grid or projector set; run false only says so.
-bool sphere_nonlocal_force(qg_nonlocal* nl, int dtype, int nocc, const int* band_idx, const double* weight,
-                           const void* psi, int64_t ld, const double* coef, DevBuf<double>& part, double* force,
-                           bool run, hipStream_t s) {
-    if (!sphere_serves(nl->gcopy, nl)) return false;
-    if (dtype == QG_F32)
-        return sphere_force_t<float>(nl, nocc, band_idx, weight, (const float*)psi, ld, coef, part, force, run, s);
-    return sphere_force_t<double>(nl, nocc, band_idx, weight, (const double*)psi, ld, coef, part, force, run, s);
 }
 
 template <class T>
