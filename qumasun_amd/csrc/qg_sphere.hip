@@ -493,7 +493,7 @@ __device__ __forceinline__ void sphere_body(const SphereArgs& a, const Coef8<T>&
             bands(std::false_type{});
             // a list's zero times an infinite or undefined gradient is not zero
             if constexpr (FORCE)
-                if (__ballot(!__builtin_isfinite(f[0] + f[1] + f[2])) != 0) bands(std::true_type{});
+                if (__builtin_expect(__ballot(!__builtin_isfinite(f[0] + f[1] + f[2])) != 0, 0)) bands(std::true_type{});
             if constexpr (FORCE) {
                 if (slot < 0) {
                     flush(li, f);
@@ -841,7 +841,7 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_project_kernel(SphereProjA
                     for (int i = 0; i < CN; ++i) all += c[i];
                     return __builtin_isfinite(all);
                 };
-                if (__ballot(!coefficients()) != 0) {
+                if (__builtin_expect(__ballot(!coefficients()) != 0, 0)) {
                     // a list's zero times an infinity or NaN at a point outside the image is not zero: the
                     // slot's epoch once more, point by point, without those
 #pragma unroll
