@@ -10,6 +10,7 @@
 #include <random>
 #include <thread>
 #include "qg_internal.hpp"
+#include "qg_radial.hpp"
 
 namespace qg {
 
@@ -39,45 +40,12 @@ static void sphere_box(const qg_grid& g, const double R[3], double rc, int b[3],
 // Smallest n with n*y > x (integer division toward zero, as GetOverlapPeriodic's helper).
 static int first_multiple_above(int x, int y) { return (x >= 0) ? (x / y) + 1 : ((x + 1) / y); }
 
-// RadialGrid2::GetValueByXi (RadialGrid2.h:81-136): linear in the outer intervals, cubic
-// Hermite next to them, quintic Hermite with 4th-order derivative estimates inside.
-static double radial_by_xi_host(double xi, const double* v, int n, double xi_min, double xi_delta) {
-    const double rel = xi - xi_min;
-    const double fl = std::floor(rel / xi_delta);
-    const int i = (int)fl;
-    if (i >= n - 1) return 0.0;
-    if (i == 0 || i == n - 2) {
-        const double t = rel / xi_delta - fl;
-        return v[i] * (1.0 - t) + v[i + 1] * t;
-    }
-    const double t = rel / xi_delta - (double)i;
-    if (1 < i && i < n - 3) {
-        const double fm2 = v[i - 2], fm1 = v[i - 1], f0 = v[i], f1 = v[i + 1], f2 = v[i + 2], f3 = v[i + 3];
-        const double g0 = 2.0 / 3.0 * (f1 - fm1) - 1.0 / 12.0 * (f2 - fm2);
-        const double g1 = 2.0 / 3.0 * (f2 - f0) - 1.0 / 12.0 * (f3 - fm1);
-        const double h0 = 4.0 / 3.0 * (f1 + fm1) - 1.0 / 12.0 * (f2 + fm2) - 5.0 / 2.0 * f0;
-        const double h1 = 4.0 / 3.0 * (f2 + f0) - 1.0 / 12.0 * (f3 + fm1) - 5.0 / 2.0 * f1;
-        const double e0 = f1 - (f0 + g0 + h0 / 2.0);
-        const double e1 = g1 - (g0 + h0);
-        const double e2 = h1 - h0;
-        const double a3 = 10.0 * e0 - 4.0 * e1 + 0.5 * e2;
-        const double a4 = -15.0 * e0 + 7.0 * e1 - e2;
-        const double a5 = f1 - f0 - g0 - h0 / 2.0 - a3 - a4;
-        return f0 + t * (g0 + t * (h0 / 2.0 + t * (a3 + t * (a4 + t * a5))));
-    }
-    const double v0 = v[i], v1 = v[i + 1];
-    const double s1 = (v[i + 2] - v0) / 2.0, s0 = (v1 - v[i - 1]) / 2.0;
-    const double a = s1 + s0 - 2.0 * (v1 - v0);
-    const double b = -s1 - 2.0 * s0 + 3.0 * (v1 - v0);
-    return a * t * t * t + b * t * t + s0 * t + v0;
-}
-
 // p(r) of a channel at squared distance rr inside its cutoff
 // (PseudoPotOperator_mpi_v2.h:154-166 for tables).
 static double radial_host(const qg_proj_spec& s, double rr) {
     if (s.radial_kind == QG_RADIAL_GAUSSIAN) return s.amplitude * std::exp(-rr / (2.0 * s.sigma * s.sigma));
     if (s.r_min * s.r_min > rr) return s.table[0];
-    return radial_by_xi_host(0.5 * std::log(rr), s.table, s.n_table, s.xi_min, s.xi_delta);
+    return radial_by_rel(0.5 * std::log(rr) - s.xi_min, s.table, s.n_table, s.xi_delta);
 }
 
 // beta_j = p(r) Y_lm on every sphere point, image by image, rows in (z, y) order; real

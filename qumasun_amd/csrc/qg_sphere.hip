@@ -31,6 +31,7 @@
 #include <tuple>
 #include <type_traits>
 #include "qg_internal.hpp"
+#include "qg_radial.hpp"
 
 namespace qg {
 
@@ -1398,40 +1399,12 @@ __global__ __launch_bounds__(kMaxThreads) void sphere_kpoint_kernel(SphereArgs a
 }
 
 // ------------------------------------------------------------------ entry lists ----
-// radial function of a channel at squared distance rr (inside its cutoff), FP64:
-// RadialGrid2::GetValueByXi (RadialGrid2.h:81-136) for tables
+// radial function of a channel at squared distance rr (inside its cutoff), FP64
 __device__ double radial_dev(const DevProj& d, const double* tables, double rr) {
     if (d.kind == QG_RADIAL_GAUSSIAN) return d.amp * exp(-rr * d.inv_2s2);
     const double* v = tables + d.table_off;
     if (d.r_min2 > rr) return v[0];
-    const double rel = 0.5 * log(rr) - d.xi_min;
-    const double fl = floor(rel / d.xi_delta);
-    const int i = (int)fl, n = d.n_table;
-    if (i >= n - 1) return 0.0;
-    if (i == 0 || i == n - 2) {
-        const double t = rel / d.xi_delta - fl;
-        return v[i] * (1.0 - t) + v[i + 1] * t;
-    }
-    const double t = rel / d.xi_delta - (double)i;
-    if (1 < i && i < n - 3) {
-        const double fm2 = v[i - 2], fm1 = v[i - 1], f0 = v[i], f1 = v[i + 1], f2 = v[i + 2], f3 = v[i + 3];
-        const double g0 = 2.0 / 3.0 * (f1 - fm1) - 1.0 / 12.0 * (f2 - fm2);
-        const double g1 = 2.0 / 3.0 * (f2 - f0) - 1.0 / 12.0 * (f3 - fm1);
-        const double h0 = 4.0 / 3.0 * (f1 + fm1) - 1.0 / 12.0 * (f2 + fm2) - 5.0 / 2.0 * f0;
-        const double h1 = 4.0 / 3.0 * (f2 + f0) - 1.0 / 12.0 * (f3 + fm1) - 5.0 / 2.0 * f1;
-        const double e0 = f1 - (f0 + g0 + h0 / 2.0);
-        const double e1 = g1 - (g0 + h0);
-        const double e2 = h1 - h0;
-        const double a3 = 10.0 * e0 - 4.0 * e1 + 0.5 * e2;
-        const double a4 = -15.0 * e0 + 7.0 * e1 - e2;
-        const double a5 = f1 - f0 - g0 - h0 / 2.0 - a3 - a4;
-        return f0 + t * (g0 + t * (h0 / 2.0 + t * (a3 + t * (a4 + t * a5))));
-    }
-    const double v0 = v[i], v1 = v[i + 1];
-    const double s1 = (v[i + 2] - v0) / 2.0, s0 = (v1 - v[i - 1]) / 2.0;
-    const double a = s1 + s0 - 2.0 * (v1 - v0);
-    const double b = -s1 - 2.0 * s0 + 3.0 * (v1 - v0);
-    return a * t * t * t + b * t * t + s0 * t + v0;
+    return radial_by_rel(0.5 * log(rr) - d.xi_min, v, d.n_table, d.xi_delta);
 }
 
 struct BuildArgs {
