@@ -1669,8 +1669,9 @@ static void sphere_images(qg_nonlocal* nl) {
         for (int d = 0; d < 3; ++d) {
             s.b[d] = std::min(s.b[d], im.b[d]);
             s.e[d] = std::max(s.e[d], im.e[d]);
-            // displacements beyond the entry word's 11-bit fields
-            if (s.e[d] - s.b[d] > 900) { nl->sphere_form = SphereForm{}; return; }
+            // the image's points, and those up to a group's start before them, as displacements from its
+            // centre (which may lie outside the grid): the entry word has signed 11-bit fields
+            if (s.n[d] - s.b[d] > 1000 || s.e[d] - s.n[d] > 1000) { nl->sphere_form = SphereForm{}; return; }
         }
     }
     nl->d_sphere_img.upload(nl->sphere_img.data(), nl->sphere_img.size());
