@@ -144,9 +144,9 @@ int qg_nonlocal_update(qg_nonlocal* nl, int natoms, const double* xyz_host, cons
 int qg_nonlocal_destroy(qg_nonlocal* nl);
 /* Number of (atom, projector, m) coefficients per band (sum of TotalProjectorLM). */
 int qg_nonlocal_num_coef(const qg_nonlocal* nl);
-/* How H psi forms the projector values: 1 = the FP32 projector pass evaluates them in the
- * kernel from the image centres (every projector Gaussian with l <= 1; QG_NL_ANALYTIC=0 in
- * the environment at creation turns it off), 0 = per-point tables everywhere. FP64 launches
+/* How the table kernels of H psi form the projector values: 1 = their FP32 projector pass evaluates
+ * them in the kernel from the image centres (every projector Gaussian with l <= 1; QG_NL_ANALYTIC=0
+ * in the environment at creation turns it off), 0 = per-point tables everywhere. Their FP64 launches
  * and the fused single-pass form read tables. Diagnostic; no counterpart in the reference,
  * which always tabulates (SetBlockYlm.h). */
 int qg_nonlocal_projector_form(const qg_nonlocal* nl);
@@ -168,7 +168,8 @@ int qg_nonlocal_energy_force(qg_nonlocal* nl, int dtype, int nbands, const void*
                              const double* occ_host, double* energy, double* forces_host, void* stream);
 
 /* coef[b*ncoef + j] = dV * sum_i beta_j(i) psi_b(i)  (FP64 device array, ncoef per band).
- * Replaces mInnerNonlocalPsi_v2 (PseudoPotOperator_mpi_v2.h:336-463) for a band block. */
+ * Replaces mInnerNonlocalPsi_v2 (PseudoPotOperator_mpi_v2.h:336-463) for a band block.  The handle
+ * keeps the partial sums' scratch between calls, so calls on one handle must not overlap. */
 int qg_nonlocal_project(qg_nonlocal* nl, int dtype, int nbands, const void* psi, int64_t ld,
                         double* coef_dev, void* stream);
 /* hpsi[b] (+)= sum_j E_j coef_bj beta_j — ProjectionPP (PseudoPotOperator_mpi_v2.h:465-570)

@@ -334,9 +334,11 @@ __global__ __launch_bounds__(kUpdThreads, 2) void update64_kernel(UpdateArgs g) 
 
 // Out = alpha A C + beta Out; A, Out: N bands of K points, not overlapping.  False (nothing launched)
 // where a band is not 16-byte aligned, and where the library's product is as fast: its tiles are 128 bands
-// wide, these 16, so this one serves where at most 0.6 of the library's tiles are bands.  Median us on
-// 512,000 points, this : library: 16 bands 31 : 31, 32 68 : 125, 64 168 : 207, 100 332 : 316,
-// 144 634 : 730, 192 929 : 951; 262,144 points x 432 2034 : 1960.
+// wide, these 16, so this one serves where at most 0.6 of the library's tiles are bands (17-76 and 129-153).
+// Mean us of a solve's updates (with and without beta) on 512,000 points, this : library: 32 bands 65 : 115,
+// 64 147 : 193, 76 197 : 227, 96 278 : 277, 112 323 : 323, 128 469 : 366, 144 556 : 689, 153 673 : 757,
+// 176 1429 : 841, 192 853 : 909; on 64,000 points 64 22 : 37, 76 31 : 44, 112 49 : 62, 128 60 : 48,
+// 144 69 : 95, 153 84 : 105.
 bool update64(const double* A, int64_t lda, const double* C, int ldc, int64_t K, int N, double alpha, double beta,
               double* out, int64_t ldo, hipStream_t s) {
     if (K < 2 || K % 2 || lda % 2 || ldo % 2 || reinterpret_cast<uintptr_t>(A) % 16 ||

@@ -150,7 +150,7 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 // Points of one workgroup of the column sums: a band is cut into ranges, so that a block of any number
 // of bands fills the chip, and the ranges' sums are added in their order.  One workgroup per band took
 // 854 (coldot of a block with itself) and 1074 us (residual) at 512,000 points x 144 FP64 bands, ranges
-// take 126 and 335 us (floors at 4.68 TB/s 126 and 378).
+// take 126 and 335 us (4.7 and 5.3 TB/s; large passes that only read reach 6.0, two reads to a write 5.7).
 constexpr int64_t kColRange = 8192;
 
 // part[k][range] = sum_i a[k*ld + i] * b[k*ld + i] (FP64 accumulation)

@@ -2099,7 +2099,7 @@ bool sphere_nonlocal_force(qg_nonlocal* nl, int nocc, const int* band_idx, const
         return sphere_lds<double>(g.n[0], ty, b, nl->sphere_form.ns, nl->sphere_form.np, sg->max_col, nw);
     };
     // two bands share an entry, its running sums and their LDS updates (64 atoms, 80^3, 137 FP64
-    // bands: 0.83 ms a call against 1.0 with one); 2 + 2 channels of two bands would spill
+    // bands: 0.84 ms a call against 1.0 with one); 2 + 2 channels of two bands would spill
     int nb = nl->sphere_form.ns == 2 || (int64_t)sg->ntile * ((nocc + 1) / 2) < 256 ? 1 : 2;
     if (nb > 1 && (sphere_halo_vectors(nq, sg->tpb) > 1 || lds_of(nb) > lds_limit())) nb = 1;
     if (lds_of(nb) > lds_limit()) return false;
