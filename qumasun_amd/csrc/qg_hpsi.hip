@@ -1733,7 +1733,12 @@ int qg_hamiltonian_set_plan(qg_ham* h, const qg_hpsi_plan* plan) {
         // qg_nonlocal_update
         if (p.kernels == QG_KERNELS_ROWS && h->nl && !h->nl->rows_wanted) {
             h->nl->rows_wanted = true;
-            rows_prepare(h->nl);
+            try {
+                rows_prepare(h->nl);
+            } catch (...) {
+                h->nl->rows_wanted = false;
+                throw;
+            }
         }
         h->plan = p;
     });
